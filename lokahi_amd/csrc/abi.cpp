@@ -212,8 +212,7 @@ int strata_linear_bf16(strata_ctx* ctx, const void* x, int x_dtype, int64_t M, i
   STRATA_REQUIRE(M <= INT32_MAX && K <= INT32_MAX && N <= INT32_MAX, "shape too large");
   STRATA_REQUIRE(aligned16(x) && aligned16(w), "x and w must be 16-byte aligned");
   if (M == 0) return STRATA_OK;
-  // Each pass covers up to 4 x rows; more rows are processed in passes.
-  return strata_bf16_gemv(ctx, x, (int)M, (int)K, w, (int)N, y, y_dtype, stream);
+  return strata_bf16_linear(ctx, x, K, (int)M, (int)K, w, (int)N, y, y_dtype, stream);
 }
 
 // -------------------------------------------------------------------- rope

@@ -71,11 +71,21 @@ struct strata_decoder {
 namespace {
 
 // logits fp32 [M, vocab] = x bf16 [M, hidden] . lm_head^T: the bf16 head on
-// the dense GEMV, a q4 head (MLX 4-bit checkpoints, possibly tied to the
+// the dense linear, a q4 head (MLX 4-bit checkpoints, possibly tied to the
 // quantized embedding) on the q4 GEMV (llama_mlx.py:886-910).
-int lm_head_launch(strata_decoder* d, const void* x, int M, float* logits, void* stream) {
+// Rows of x are ldx elements apart.
+int lm_head_launch(strata_decoder* d, const void* x, int64_t ldx, int M, float* logits,
+                   void* stream) {
   const strata_llama_config& c = d->cfg;
   if (d->head_q4.w) {
+    if (ldx != c.hidden_size && M > 1) {  // the q4 GEMV takes contiguous rows
+      for (int m = 0; m < M; ++m) {
+        const int rc = lm_head_launch(d, static_cast<const char*>(x) + m * ldx * 2, ldx, 1,
+                                      logits + (int64_t)m * c.vocab_size, stream);
+        if (rc) return rc;
+      }
+      return STRATA_OK;
+    }
     if (d->head_lay.buf && M <= kGvMaxRows) {
       void* ys[1] = {logits};
       return strata_gemv_layout_run(d->head_lay, x, M, ys, STRATA_F32, nullptr, stream);
@@ -84,8 +94,8 @@ int lm_head_launch(strata_decoder* d, const void* x, int M, float* logits, void*
     w.y = logits;
     return strata_q4_gemv(d->ctx, x, STRATA_BF16, M, c.hidden_size, &w, 1, STRATA_F32, stream);
   }
-  return strata_bf16_gemv(d->ctx, x, M, c.hidden_size, d->lm_head, c.vocab_size, logits,
-                          STRATA_F32, stream);
+  return strata_bf16_linear(d->ctx, x, ldx, M, c.hidden_size, d->lm_head, c.vocab_size, logits,
+                            STRATA_F32, stream);
 }
 
 int alloc(void** p, size_t bytes) {
@@ -170,7 +180,7 @@ int forward_layers(strata_decoder* d, int B, int L, int pos0, void* stream, int 
       else RC(strata_q4_gemv_epi(d->ctx, d->act, T, F, &dn, 1, er, stream));
     }
     RC(strata_rmsnorm_launch(d->h, nullptr, d->final_norm, T, H, c.rms_norm_eps, d->hn, stream));
-    return lm_head_launch(d, d->hn, B, d->logits, stream);
+    return lm_head_launch(d, d->hn, H, B, d->logits, stream);
   }
   for (int li = 0; li < c.num_layers; ++li) {
     const strata_llama_layer& Lw = d->layers[li];
@@ -209,14 +219,8 @@ int forward_layers(strata_decoder* d, int B, int L, int pos0, void* stream, int 
   }
   // final norm of h + delta, then lm_head on the last position of each row
   RC(strata_rmsnorm_launch(d->h, d->delta, d->final_norm, T, H, c.rms_norm_eps, d->hn, stream));
-  if (L == 1) {
-    RC(lm_head_launch(d, d->hn, B, d->logits, stream));
-  } else {
-    for (int b = 0; b < B; ++b)
-      RC(lm_head_launch(d, static_cast<char*>(d->hn) + ((int64_t)b * L + L - 1) * H * 2, 1,
-                        d->logits + (int64_t)b * c.vocab_size, stream));
-  }
-  return STRATA_OK;
+  return lm_head_launch(d, static_cast<char*>(d->hn) + (int64_t)(L - 1) * H * 2, (int64_t)L * H, B,
+                        d->logits, stream);
 }
 
 int check_forward(strata_decoder* d, int B, int L) {

@@ -61,6 +61,9 @@ int strata_q4_gemv(strata_ctx* ctx, const void* x, int x_dtype, int M, int K,
                    const strata_q4_weight* ws, int count, int y_dtype, void* stream);
 int strata_bf16_gemv(strata_ctx* ctx, const void* x, int M, int K, const uint16_t* w, int N,
                      void* y, int y_dtype, void* stream);
+// y[m] = x[m] @ w^T, x rows ldx elements apart.
+int strata_bf16_linear(strata_ctx* ctx, const void* x, int64_t ldx, int M, int K,
+                       const uint16_t* w, int N, void* y, int y_dtype, void* stream);
 int strata_q4_gemm_launch(const void* x, int M, int K, const uint32_t* w, const uint16_t* s,
                           const uint16_t* b, int N, void* y, int y_dtype, void* stream);
 // Prefill q4 linear (bf16 x, M > 8): the hand-written fused-dequant MFMA

@@ -226,3 +226,33 @@ def test_gemm_mid_rows_split_k(dev, M, K, ns):
         assert rel_err(to_np_f32(a16), q4.quantized_matmul(xf, w, s, b)) < TOL_BF16
         assert torch.equal(ops.linear(xd, *dp, out_dtype=torch.float32), a32)
         assert torch.equal(ops.linear(xd, *dp), a16)
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 24576, 64), (9, 8200, 192), (32, 4097, 1024), (33, 8192, 320),
+                                   (64, 2049, 4096), (161, 1000, 128), (700, 513, 256), (13, 6144, 72)])
+def test_bf16_dense_linear_rows(dev, M, N, K):
+    """Several rows of the dense linear: the MFMA kernel's row tiles (32-160
+    rows, partial last ones), W tiles cut by N, an odd N (scalar stores), K
+    below one accumulation chain and not a multiple of it, and K % 64 != 0
+    (the GEMV).  fp32 sums of exact bf16 products: K terms of relative error
+    2^-24 each stay under K * 2^-24 of the sum of magnitudes, here far below
+    1e-5 of the result; bf16 outputs are the rounded fp32 ones."""
+    from lokahi_amd import ops
+    gen = torch.Generator(device=dev).manual_seed(M + N)
+    W = (torch.randn((N, K), generator=gen, device=dev) * 0.02).bfloat16()
+    x = torch.randn((M, K), generator=gen, device=dev).bfloat16()
+    ref = x.double() @ W.double().T
+    y = ops.linear(x, W, None, None, out_dtype=torch.float32)
+    assert float((y - ref).norm() / ref.norm()) < 1e-5
+    assert float((y - ref).abs().max() / ref.square().mean().sqrt()) < 1e-4
+    assert torch.equal(ops.linear(x, W, None, None), y.bfloat16())
+    if K % 64:
+        return  # the GEMV multiplies the last x chunk by zero weights past K
+    # an infinite or NaN activation reaches its own row only, as in a plain sum
+    W.abs_()
+    x[0, 0], x[1, K - 1], x[2, K // 2] = float("inf"), float("-inf"), float("nan")
+    y = ops.linear(x, W, None, None, out_dtype=torch.float32)
+    ref = x.float() @ W.float().T
+    assert torch.equal(y[:3].isnan(), ref[:3].isnan())
+    assert torch.equal(torch.where(y[:2].isinf(), y[:2], 0.), torch.where(ref[:2].isinf(), ref[:2], 0.))
+    assert bool(y[3:].isfinite().all())
