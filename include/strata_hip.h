@@ -145,6 +145,21 @@ int strata_attn_gqa(strata_ctx* ctx, const void* q, int q_dtype, const void* k, 
                     int Lq, int Lk, int D, int causal, int q_blk, int k_blk, float eps,
                     void* out, void* stream);
 
+/* No counterpart in the reference.  strata_attn_gqa with a caller-owned
+ * device workspace (16-byte aligned, at least strata_attn_workspace bytes to
+ * be used in full; NULL or 0 bytes: as strata_attn_gqa): a call with several
+ * query rows whose tiles would leave the GPU idle splits its keys over more
+ * workgroups, keeps their fp32 partials there and merges them.  The workspace
+ * is in use until the call's work on `stream` is done; calls that may overlap
+ * need one each.  strata_attn_workspace sets *bytes to 0 when no split pays. */
+int strata_attn_workspace(strata_ctx* ctx, int q_dtype, int k_dtype, int v_dtype, int B, int Hq,
+                          int Hkv, int Lq, int Lk, int D, int causal, int64_t* bytes);
+int strata_attn_gqa_ws(strata_ctx* ctx, const void* q, int q_dtype, const void* k, int k_dtype,
+                       const void* v, int v_dtype, int64_t kv_batch_stride,
+                       int64_t kv_head_stride, const int32_t* qpos, int B, int Hq, int Hkv,
+                       int Lq, int Lk, int D, int causal, int q_blk, int k_blk, float eps,
+                       void* out, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* No counterpart in the reference.  strata_attn_gqa for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): same arguments, results and errors, but

@@ -78,6 +78,11 @@ _SIGS = {
                          C.c_int, C.c_int64, C.c_int64, C.c_void_p, C.c_int, C.c_int, C.c_int,
                          C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float,
                          C.c_void_p, C.c_void_p], C.c_int),
+    "strata_attn_gqa_ws": ([C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_void_p,
+                         C.c_int, C.c_int64, C.c_int64, C.c_void_p, C.c_int, C.c_int, C.c_int,
+                         C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float,
+                         C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p], C.c_int),
+    "strata_attn_workspace": ([C.c_void_p] + [C.c_int] * 10 + [C.POINTER(C.c_int64)], C.c_int),
     "strata_attn_gqa_noalloc": ([C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_int,
                                  C.c_void_p, C.c_int, C.c_int64, C.c_int64, C.c_void_p, C.c_int,
                                  C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int,

@@ -232,6 +232,27 @@ int strata_attn_gqa(strata_ctx* ctx, const void* q, int q_dtype, const void* k, 
                     const void* v, int v_dtype, int64_t kv_batch_stride, int64_t kv_head_stride,
                     const int32_t* qpos, int B, int Hq, int Hkv, int Lq, int Lk, int D, int causal,
                     int q_blk, int k_blk, float eps, void* out, void* stream) {
+  return strata_attn_gqa_ws(ctx, q, q_dtype, k, k_dtype, v, v_dtype, kv_batch_stride,
+                            kv_head_stride, qpos, B, Hq, Hkv, Lq, Lk, D, causal, q_blk, k_blk, eps,
+                            out, nullptr, 0, stream);
+}
+
+int strata_attn_workspace(strata_ctx* ctx, int q_dtype, int k_dtype, int v_dtype, int B, int Hq,
+                          int Hkv, int Lq, int Lk, int D, int causal, int64_t* bytes) {
+  STRATA_REQUIRE(ctx != nullptr && bytes != nullptr, "ctx/bytes is NULL");
+  STRATA_REQUIRE(B > 0 && Lq >= 0 && Lk >= 0 && D > 0, "invalid shape");
+  STRATA_REQUIRE(Hkv > 0 && Hq > 0 && Hq % Hkv == 0,
+                 "query heads must be divisible by key/value heads");
+  *bytes = (int64_t)strata_attn_prefill_ws(ctx, q_dtype, k_dtype, v_dtype, B, Hq, Hkv, Lq, Lk, D,
+                                           causal);
+  return STRATA_OK;
+}
+
+int strata_attn_gqa_ws(strata_ctx* ctx, const void* q, int q_dtype, const void* k, int k_dtype,
+                       const void* v, int v_dtype, int64_t kv_batch_stride, int64_t kv_head_stride,
+                       const int32_t* qpos, int B, int Hq, int Hkv, int Lq, int Lk, int D,
+                       int causal, int q_blk, int k_blk, float eps, void* out, void* workspace,
+                       int64_t workspace_bytes, void* stream) {
   STRATA_REQUIRE(ctx != nullptr, "ctx is NULL");
   // Order and wording follow mlx_ops.py:48-67.
   STRATA_REQUIRE(q_blk > 0 && k_blk > 0, "attention block sizes must be positive");
@@ -248,9 +269,15 @@ int strata_attn_gqa(strata_ctx* ctx, const void* q, int q_dtype, const void* k, 
     return strata_zero_fill_launch(out, (int64_t)B * Hq * Lq * D * dtype_size(q_dtype), stream);
   }
   STRATA_REQUIRE(k && v, "null tensor pointer");
+  AttnExtra ex{};
+  if (workspace && workspace_bytes > 0) {
+    STRATA_REQUIRE(aligned16(workspace), "the attention workspace must be 16-byte aligned");
+    ex.ws = workspace;
+    ex.ws_bytes = (size_t)workspace_bytes;
+  }
   return strata_attention_dispatch(ctx, q, q_dtype, k, k_dtype, v, v_dtype, kv_batch_stride,
                                    kv_head_stride, qpos, B, Hq, Hkv, Lq, Lk, D, causal, eps, out,
-                                   AttnExtra{}, stream);
+                                   ex, stream);
 }
 
 int strata_attn_gqa_noalloc(strata_ctx* ctx, const void* q, int q_dtype, const void* k,

@@ -26,6 +26,7 @@
 //   * attn_prefill_f32 : the same for fp32 inputs on 16x16x4 fp32 MFMA.
 //   * attn_generic : any other shape (e.g. tiny head dims), one wave per query.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <cstdlib>
 
@@ -455,39 +456,80 @@ void launch_decode_merge(const float* part, int nsplit, int D, int rows, float e
 }
 
 // ----------------------------------------------------------- prefill on MFMA
-// Workgroup wg of the prefill grid -> (query tile, b, kv head, query head).
-// remap: workgroups are dealt to the 8 XCDs round-robin (wg % 8); a group
-// gi of the G query heads of one (query tile, b, kv head) goes to XCD
-// gi % 8 in G consecutive slots of that XCD, groups ordered longest causal
-// query tile first (measured 1.5x on the bf16 two-block kernel at 8k
-// causal).  Otherwise the order is query tile fastest, then head, then
-// batch.  Returns false for the padding of the last round.
+// Query rows of one (b, KV head) are packed: packed row r is query r / G of
+// query head hkv * G + r % G, so the rows of a tile share the KV head (a short
+// query fills tiles with its whole group) and have close positions (a causal
+// tile masks few keys).
+//
+// Workgroup wg of the prefill grid -> (tile of packed rows, b, KV head).
+// Workgroups are dealt to the 8 XCDs round-robin (wg % 8); kTileGroup
+// consecutive tiles of one (b, KV head) go to consecutive slots of one XCD
+// (their K/V tiles share its L2), groups ordered longest causal tiles first
+// (measured 1.5x on the bf16 two-block kernel at 8k causal).  Returns false
+// for the padding of the grid.
 constexpr int kXcds = 8;
-__host__ __device__ inline int prefill_grid(int nqt, int B, int Hkv, int G) {
-  const int groups = nqt * B * Hkv;
-  return (groups + kXcds - 1) / kXcds * kXcds * G;
+constexpr int kTileGroup = 4;
+__host__ __device__ inline int prefill_grid(int nqt, int B, int Hkv) {
+  const int groups = (nqt + kTileGroup - 1) / kTileGroup * B * Hkv;
+  return (groups + kXcds - 1) / kXcds * kXcds * kTileGroup;
 }
-__device__ inline bool prefill_item(bool remap, int wg, int nqt, int B, int Hkv, int G, int* qt,
-                                    int* b, int* hkv, int* hq) {
-  if (!remap) {
-    if (wg >= nqt * B * Hkv * G) return false;
-    *qt = wg % nqt;
-    *hq = (wg / nqt) % (Hkv * G);
-    *b = wg / (nqt * Hkv * G);
-    *hkv = *hq / G;
-    return true;
-  }
+__device__ inline bool prefill_item(int wg, int nqt, int B, int Hkv, int* qt, int* b, int* hkv) {
   const int xcd = wg % kXcds, slot = wg / kXcds;
-  const int g = slot % G, gi = (slot / G) * kXcds + xcd;
-  if (gi >= nqt * B * Hkv) return false;
-  const int per_tile = B * Hkv;
-  *qt = nqt - 1 - gi / per_tile;
-  const int rest = gi % per_tile;
+  const int gi = (slot / kTileGroup) * kXcds + xcd;
+  const int ng = (nqt + kTileGroup - 1) / kTileGroup, per = B * Hkv;
+  if (gi >= ng * per) return false;
+  *qt = (ng - 1 - gi / per) * kTileGroup + kTileGroup - 1 - slot % kTileGroup;
+  const int rest = gi % per;
   *b = rest / Hkv;
   *hkv = rest % Hkv;
-  *hq = *hkv * G + g;
-  return true;
+  return *qt < nqt;
 }
+
+// Key split of a prefill launch (gridDim.y = nsplit): split s of a tile takes
+// keys s * chunk .. +chunk and leaves, per output row, the unnormalised o in
+// o[row][s][D] and (m, l) in ms[row][s] for attn_prefill_merge (l = 0: no
+// visible key, o not written).  A tile that ends inside split 0 writes the
+// output itself and leaves l = -1 there.
+struct PrefillSplit {
+  int nsplit, chunk;
+  float* o;
+  float2* ms;
+};
+
+// Key limits of a wave's rows pr0 .. pr0 + R - 1 and of the workgroup's rows
+// (up to pr_end): kfull, keys every row of the wave sees (0 with a row past
+// the last: tiles then mask); need, keys any of its rows sees; kmax, keys any
+// row of the workgroup sees.  qp: this lane's position, -1 past the last row.
+// Without given positions they follow from the row numbers; given ones are
+// reduced over the R lanes that hold the wave's rows and over the workgroup
+// (s_kmax, two barriers).
+template <int R>
+__device__ __forceinline__ void key_limits(const int32_t* qpos, int causal, int qp, bool row_ok,
+                                           int pr0, int pr_end, int G, int Lq, int Lk, int* s_kmax,
+                                           int* kfull, int* need, int* kmax) {
+  const int rows = Lq * G;
+  if (!causal || !qpos) {
+    const int last = min(pr0 + R, rows) - 1, wg_last = min(pr_end, rows) - 1;
+    *kfull = pr0 + R <= rows ? (causal ? Lk - Lq + pr0 / G + 1 : Lk) : 0;
+    *need = last >= pr0 ? (causal ? Lk - Lq + last / G + 1 : Lk) : 0;
+    *kmax = causal ? Lk - Lq + wg_last / G + 1 : Lk;
+    return;
+  }
+  int f = row_ok ? qp + 1 : 0, n = qp + 1;
+#pragma unroll
+  for (int off = 1; off < R; off <<= 1) {
+    f = min(f, __shfl_xor(f, off, 64));
+    n = max(n, __shfl_xor(n, off, 64));
+  }
+  if (threadIdx.x == 0) *s_kmax = 0;
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) atomicMax(s_kmax, n);
+  __syncthreads();
+  *kfull = f;
+  *need = n;
+  *kmax = min(Lk, *s_kmax);
+}
+
 __device__ __forceinline__ f32x4_t mfma_f32(float a, float b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
@@ -498,18 +540,18 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
-// fp32 prefill.  1-D grid, block 256; workgroup -> (query tile qt, b, hq)
-// in plain order (prefill_item without the remap); wave w owns the 16 query
-// rows qt*64 + 16w + 0..15.  S^T = K Q^T and O^T += V P^T on 16x16x4 fp32
-// MFMAs; one LDS stage of K and V tiles (64 keys, row-major, padded rows).
+// fp32 prefill.  Block 256; wave w owns the 16 packed query rows qt*64 + 16w
+// + 0..15.  S^T = K Q^T and O^T += V P^T on 16x16x4 fp32 MFMAs; one LDS stage
+// of K and V tiles (64 keys, row-major, padded rows).
 // MFMA 16x16x4 layouts (wave64): A (16 x 4): lane l holds row l%16, k l/16;
 // B (4 x 16): lane l holds column l%16, k l/16; C (16 x 16): lane l holds
 // column l%16, rows 4(l/16) + 0..3.
-template <int D>
+template <int D, bool SPLIT>
 __global__ __launch_bounds__(256) void attn_prefill_f32(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     int64_t kv_bs, int64_t kv_hs, const int32_t* __restrict__ qpos, int B, int Hq, int Hkv,
-    int Lq, int Lk, int causal, float scale, float eps, int out_tm, float* __restrict__ out) {
+    int Lq, int Lk, int causal, float scale, float eps, int out_tm, float* __restrict__ out,
+    PrefillSplit sp) {
   constexpr int KT = 64;                 // keys per tile
   constexpr int PAD = 4;                 // LDS row padding (elements)
   constexpr int RS = D + PAD;            // LDS row stride
@@ -518,46 +560,17 @@ __global__ __launch_bounds__(256) void attn_prefill_f32(
   __shared__ int s_kmax;
 
   const int G = Hq / Hkv;
-  int qt, b, hkv, hq;
-  if (!prefill_item(false, blockIdx.x, (Lq + 63) / 64, B, Hkv, G, &qt, &b, &hkv, &hq))
-    return;  // grid padding
+  int qt, b, hkv;
+  if (!prefill_item(blockIdx.x, (Lq * G + 63) / 64, B, Hkv, &qt, &b, &hkv)) return;  // grid padding
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, grp = lane >> 4;
-  const int row = qt * 64 + 16 * wave + col;  // this lane's query row
+  const int pr = qt * 64 + 16 * wave + col;  // this lane's packed row
+  const int row = pr / G, hq = hkv * G + (pr - row * G);
   const bool row_ok = row < Lq;
   const int qp = row_ok ? (causal ? (qpos ? qpos[(int64_t)b * Lq + row] : Lk - Lq + row) : Lk - 1)
                         : -1;
-  // keys every row of the wave sees (no mask below) and keys any row needs
-  int kfull = row_ok ? (causal ? qp + 1 : Lk) : 0;
-  int wave_need = qp + 1;
-#pragma unroll
-  for (int off = 1; off < 16; off <<= 1) {
-    kfull = min(kfull, __shfl_xor(kfull, off, 64));
-    wave_need = max(wave_need, __shfl_xor(wave_need, off, 64));
-  }
-  if (threadIdx.x == 0) s_kmax = 0;
-  __syncthreads();
-  if (lane == 0) atomicMax(&s_kmax, wave_need);
-  __syncthreads();
-  const int kmax = causal ? min(Lk, s_kmax) : Lk;
-
   const float* kbase = k + (int64_t)b * kv_bs + (int64_t)hkv * kv_hs;
   const float* vbase = v + (int64_t)b * kv_bs + (int64_t)hkv * kv_hs;
-  // Q fragments as the B operand of S^T: column = query row, k = head dim 4s + grp.
-  constexpr int QF = D / 4;
-  float qf[QF];
-  {
-    const float* qrow = q + (((int64_t)b * Hq + hq) * Lq + (row_ok ? row : 0)) * D;
-#pragma unroll
-    for (int s = 0; s < QF; ++s) qf[s] = row_ok ? qrow[4 * s + grp] : 0.f;
-  }
-  constexpr int DT = D / 16;  // output d tiles
-  f32x4_t acc[DT];
-#pragma unroll
-  for (int i = 0; i < DT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
-  const float sl2 = scale * kLog2e;
-
   // Tiles: 16-byte chunks, chunk c of the tile -> (key t, element d0); keys
   // past Lk read key Lk - 1 (finite; their scores are masked, their
   // weights 0).  Tile t+1's loads are issued before tile t's math.
@@ -574,6 +587,36 @@ __global__ __launch_bounds__(256) void attn_prefill_f32(
       vreg[u] = *reinterpret_cast<const uint4*>(vbase + (int64_t)key * D + d0);
     }
   };
+  // the first tile's loads go out before given positions are reduced
+  const int split = SPLIT ? blockIdx.y : 0;
+  const int kb_begin = SPLIT ? split * sp.chunk : 0;
+  const bool empty = SPLIT && !qpos && causal && kb_begin > Lk - Lq + (min(qt * 64 + 64, Lq * G) - 1) / G;
+  if (!empty) fetch(kb_begin);
+  int kfull, wave_need, kmax;
+  key_limits<16>(qpos, causal, qp, row_ok, qt * 64 + 16 * wave, qt * 64 + 64, G, Lq, Lk, &s_kmax,
+                 &kfull, &wave_need, &kmax);
+  const int kb_end = SPLIT ? min(kmax, kb_begin + sp.chunk) : kmax;
+  const int64_t rid = ((int64_t)b * Hq + hq) * Lq + row;  // output row
+  if (SPLIT && kb_begin >= kmax && split > 0) {
+    if (row_ok && grp == 0) sp.ms[rid * sp.nsplit + split] = make_float2(-INFINITY, 0.f);
+    return;
+  }
+
+  // Q fragments as the B operand of S^T: column = query row, k = head dim 4s + grp.
+  constexpr int QF = D / 4;
+  float qf[QF];
+  {
+    const float* qrow = q + (row_ok ? rid : 0) * D;
+#pragma unroll
+    for (int s = 0; s < QF; ++s) qf[s] = row_ok ? qrow[4 * s + grp] : 0.f;
+  }
+  constexpr int DT = D / 16;  // output d tiles
+  f32x4_t acc[DT];
+#pragma unroll
+  for (int i = 0; i < DT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+  const float sl2 = scale * kLog2e;
+
   auto stage = [&]() {
 #pragma unroll
     for (int u = 0; u < NCH; ++u) {
@@ -583,13 +626,10 @@ __global__ __launch_bounds__(256) void attn_prefill_f32(
       *reinterpret_cast<uint4*>(&vs[t * RS + d0]) = vreg[u];
     }
   };
-  if (kmax > 0) {
-    fetch(0);
-    stage();
-  }
+  if (kb_end > kb_begin) stage();
   __syncthreads();
-  for (int kb0 = 0; kb0 < kmax; kb0 += KT) {
-    const bool more = kb0 + KT < kmax;
+  for (int kb0 = kb_begin; kb0 < kb_end; kb0 += KT) {
+    const bool more = kb0 + KT < kb_end;
     if (more) fetch(kb0 + KT);
     if (__builtin_amdgcn_readfirstlane((int)(kb0 < wave_need))) {
       // st[j][i] = score(this lane's row, key kb0 + 16j + 4 grp + i)
@@ -659,11 +699,21 @@ __global__ __launch_bounds__(256) void attn_prefill_f32(
   float l_tot = l_run;
   l_tot = xor_sum<16>(l_tot);
   l_tot = xor_sum<32>(l_tot);
+  if (SPLIT && (split > 0 || kmax > sp.chunk)) {
+    if (!row_ok) return;
+    if (grp == 0) sp.ms[rid * sp.nsplit + split] = make_float2(m_run, l_tot);
+    float* orow = sp.o + (rid * sp.nsplit + split) * D;
+    if (l_tot != 0.f)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+        *reinterpret_cast<f32x4_t*>(orow + dt * 16 + 4 * grp) = acc[dt];
+    return;
+  }
   if (row_ok) {
+    if (SPLIT && grp == 0) sp.ms[rid * sp.nsplit] = make_float2(0.f, -1.f);
     const float inv = 1.f / fmaxf(l_tot, eps);
     // out_tm: token-major [B, Lq, Hq, D] (the o_proj input); else [B, Hq, Lq, D]
-    float* orow = out + (out_tm ? (((int64_t)b * Lq + row) * Hq + hq) * D
-                                : (((int64_t)b * Hq + hq) * Lq + row) * D);
+    float* orow = out + (out_tm ? ((int64_t)b * Lq + row) * Hq + hq : rid) * D;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -678,8 +728,8 @@ __device__ __forceinline__ f32x16_t mfma32_bf16(const bf16x8_t& a, const bf16x8_
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// bf16 prefill on 32x32x16 MFMA tiles.  Workgroup = NW waves = 32 NW query
-// rows of one (b, query head) (grid order as prefill_item); wave w owns rows
+// bf16 prefill on 32x32x16 MFMA tiles.  Workgroup = NW waves = 32 NW packed
+// query rows of one (b, KV head) (grid order as prefill_item); wave w owns rows
 // qt*32NW + 32w + 0..31.  S^T = K Q^T and O^T += V^T P^T run as 32x32x16
 // MFMAs whose 32-cycle issue leaves room for other waves' softmax on the
 // SIMD; the P^T operand is the S^T accumulator itself (no shuffles).
@@ -694,12 +744,13 @@ __device__ __forceinline__ f32x16_t mfma32_bf16(const bf16x8_t& a, const bf16x8_
 // 32): lane l holds column l%32, rows 8(i/4) + 4(l/32) + i%4 for i < 16.
 typedef short v4i16_t __attribute__((ext_vector_type(4)));
 constexpr float kRescaleSlack = 8.f;
-template <int D, int NW, int NST, int KT>
+template <int D, int NW, int NST, int KT, bool SPLIT>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(KT == 32 ? 3 : 2)))
 void attn_prefill_mfma32(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
     int64_t kv_bs, int64_t kv_hs, const int32_t* __restrict__ qpos, int B, int Hq, int Hkv,
-    int Lq, int Lk, int causal, float scale, float eps, int out_tm, bf16_t* __restrict__ out) {
+    int Lq, int Lk, int causal, float scale, float eps, int out_tm, bf16_t* __restrict__ out,
+    PrefillSplit sp) {
   constexpr int KB = KT / 32;         // 32-key score blocks per tile
   constexpr int ROW = D * 2;          // bytes per K / V row
   constexpr int NCHK = D / 8;         // 16-byte chunks per row
@@ -713,32 +764,17 @@ void attn_prefill_mfma32(
   __shared__ int s_kmax;
 
   const int G = Hq / Hkv;
-  int qt, b, hkv, hq;
-  if (!prefill_item(true, blockIdx.x, (Lq + QR - 1) / QR, B, Hkv, G, &qt, &b, &hkv, &hq))
+  int qt, b, hkv;
+  if (!prefill_item(blockIdx.x, (Lq * G + QR - 1) / QR, B, Hkv, &qt, &b, &hkv))
     return;  // grid padding
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c32 = lane & 31, h = lane >> 5;
-  const int row = qt * QR + 32 * wave + c32;  // this lane's query row
+  const int pr = qt * QR + 32 * wave + c32;  // this lane's packed row
+  const int row = pr / G, hq = hkv * G + (pr - row * G);
   const bool row_ok = row < Lq;
   const int qp = row_ok ? (causal ? (qpos ? qpos[(int64_t)b * Lq + row] : Lk - Lq + row) : Lk - 1)
                         : -1;
-  // Keys every row of the wave sees (tiles below need no mask) and keys any
-  // row of it needs (tiles from there on are skipped); lanes l and l + 32
-  // hold the same row.
-  int kfull = row_ok ? (causal ? qp + 1 : Lk) : 0;
-  int wave_need = qp + 1;
-#pragma unroll
-  for (int off = 1; off < 32; off <<= 1) {
-    kfull = min(kfull, __shfl_xor(kfull, off, 64));
-    wave_need = max(wave_need, __shfl_xor(wave_need, off, 64));
-  }
-  if (threadIdx.x == 0) s_kmax = 0;
-  __syncthreads();
-  if (lane == 0) atomicMax(&s_kmax, wave_need);
-  __syncthreads();
-  const int kmax = causal ? min(Lk, s_kmax) : Lk;
-
   // Buffer descriptors of this head's K and V rows: keys at or past Lk
   // read as zero.
   const v4i32_t rk = rsrc(k + (int64_t)b * kv_bs + (int64_t)hkv * kv_hs, (uint32_t)Lk * ROW);
@@ -771,13 +807,19 @@ void attn_prefill_mfma32(
     }
   };
 
+  // The first tile's loads and the queries' go out before given positions are
+  // reduced (keys at or past Lk read as zero).
+  const int split = SPLIT ? blockIdx.y : 0;
+  const int kbeg = SPLIT ? split * sp.chunk : 0;
+  const bool empty = SPLIT && !qpos && causal && kbeg > Lk - Lq + (min(qt * QR + QR, Lq * G) - 1) / G;
+  if (!empty) issue(kbeg, 0);
+  const int64_t rid = ((int64_t)b * Hq + hq) * Lq + row;  // output row
   // Q^T fragments (the B operand of S^T): column = this lane's row, k = the
   // head dims 16 s + 8 h .. +8.
   constexpr int QS = D / 16;
   bf16x8_t qf[QS];
   {
-    const uint16_t* qrow = reinterpret_cast<const uint16_t*>(q) +
-                           (((int64_t)b * Hq + hq) * Lq + (row_ok ? row : 0)) * D;
+    const uint16_t* qrow = reinterpret_cast<const uint16_t*>(q) + (row_ok ? rid : 0) * D;
 #pragma unroll
     for (int s = 0; s < QS; ++s) {
       uint4 u = make_uint4(0, 0, 0, 0);
@@ -785,6 +827,18 @@ void attn_prefill_mfma32(
       qf[s] = __builtin_bit_cast(bf16x8_t, u);
     }
   }
+  // Tiles below kfull need no mask; tiles from wave_need on are skipped by the
+  // wave; lanes l and l + 32 hold the same row.
+  int kfull, wave_need, kmax;
+  key_limits<32>(qpos, causal, qp, row_ok, qt * QR + 32 * wave, qt * QR + QR, G, Lq, Lk, &s_kmax,
+                 &kfull, &wave_need, &kmax);
+  const int kend = SPLIT ? min(kmax, kbeg + sp.chunk) : kmax;
+  if (SPLIT && kbeg >= kmax && split > 0) {
+    if (row_ok && h == 0) sp.ms[rid * sp.nsplit + split] = make_float2(-INFINITY, 0.f);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS outlives the wave
+    return;
+  }
+
   constexpr int DB = D / 32;  // 32-row head-dim blocks of O^T
   f32x16_t acc[DB];
 #pragma unroll
@@ -825,17 +879,17 @@ void attn_prefill_mfma32(
     else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(6 * NI) : "memory");
   };
   static_assert(AHEAD <= 3, "wait_tiles covers up to three tiles in flight");
-  const int nt = (kmax + KT - 1) / KT;
+  const int nt = (kend - kbeg + KT - 1) / KT;
   // prologue: tiles 0 .. AHEAD - 1 in flight, tile 0 complete
-  for (int t = 0; t < AHEAD && t < nt; ++t) issue(t * KT, t);
+  for (int t = 1; t < AHEAD && t < nt; ++t) issue(kbeg + t * KT, t);
   wait_tiles(min(nt, AHEAD) - 1);
   __syncthreads();
   // one tile on stage ST (a compile-time constant, so every LDS address is a
   // lane offset plus an immediate)
   auto tile = [&](int t, auto STC) {
     constexpr int ST = decltype(STC)::value;
-    const int kb0 = t * KT;
-    if (t + AHEAD < nt) issue((t + AHEAD) * KT, (ST + AHEAD) % NST);  // the stage tile t - 1 used
+    const int kb0 = kbeg + t * KT;
+    if (t + AHEAD < nt) issue(kb0 + AHEAD * KT, (ST + AHEAD) % NST);  // the stage tile t - 1 used
     const uint8_t* ks = lds + ST * STAGE;
     // Waves whose rows see no key of the tile skip its math (one scalar
     // branch); rows of a live wave that see none are masked to p = 0.
@@ -947,12 +1001,25 @@ void attn_prefill_mfma32(
   }
 
   const float l_tot = xor_sum<32>(l_run);
+  if (SPLIT && (split > 0 || kmax > sp.chunk)) {
+    if (!row_ok) return;
+    if (h == 0) sp.ms[rid * sp.nsplit + split] = make_float2(m_run, l_tot);
+    float* orow = sp.o + (rid * sp.nsplit + split) * D;
+    if (l_tot != 0.f)
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; i += 4)
+          *reinterpret_cast<float4*>(orow + 32 * db + 2 * i + 4 * h) =
+              make_float4(acc[db][i], acc[db][i + 1], acc[db][i + 2], acc[db][i + 3]);
+    return;
+  }
   if (row_ok) {
+    if (SPLIT && h == 0) sp.ms[rid * sp.nsplit] = make_float2(0.f, -1.f);
     const float inv = 1.f / fmaxf(l_tot, eps);
     // out_tm: token-major [B, Lq, Hq, D] (the o_proj input); else [B, Hq, Lq, D]
     uint16_t* orow = reinterpret_cast<uint16_t*>(out) +
-                     (out_tm ? (((int64_t)b * Lq + row) * Hq + hq) * D
-                             : (((int64_t)b * Hq + hq) * Lq + row) * D);
+                     (out_tm ? ((int64_t)b * Lq + row) * Hq + hq : rid) * D;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -962,6 +1029,54 @@ void attn_prefill_mfma32(
         *reinterpret_cast<uint2*>(orow + 32 * db + 8 * g4 + 4 * h) = o2;
       }
   }
+}
+
+// The splits of a prefill launch merged: one wave per output row, 4 rows per
+// workgroup; lane l holds split l's (m, l) and its weight (at most 64 splits)
+// and the head-dim entries C*l .. C*l+C-1.
+template <typename TQ, int D>
+__global__ __launch_bounds__(256) void attn_prefill_merge(PrefillSplit sp, int64_t rows, int Hq,
+                                                          int Lq, float eps, int out_tm,
+                                                          TQ* __restrict__ out) {
+  constexpr int C = D / 64;
+  const int lane = threadIdx.x & 63;
+  const int64_t rid = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (rid >= rows) return;
+  const int S = sp.nsplit;
+  float2 my = sp.ms[rid * S + min(lane, S - 1)];
+  if (lane >= S) my.y = 0.f;
+  // (l != 0 and not l > 0: a NaN sum stays one)
+  if (__int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(my.y))) < 0.f)
+    return;  // written by its only split
+  const float mb = wave_max(my.y != 0.f ? my.x : -INFINITY);
+  const float mref = mb == -INFINITY ? 0.f : mb;
+  const float w = my.y != 0.f ? __builtin_amdgcn_exp2f(my.x - mref) : 0.f;
+  const float ss = wave_sum(my.y * w);
+  float acc[C] = {};
+  const float* o = sp.o + rid * S * D + C * lane;
+  // splits with no visible key are not written: their o is not used
+  constexpr int U = 16;  // splits whose loads are in flight together
+  uint64_t live = __ballot(my.y != 0.f);
+  while (live) {
+    float v[U][C], wv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int s = live ? __builtin_ctzll(live) : 0;
+      wv[u] = live ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s)) : 0.f;
+#pragma unroll
+      for (int c = 0; c < C; ++c) v[u][c] = live ? o[(int64_t)s * D + c] : 0.f;
+      live &= live - 1;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int c = 0; c < C; ++c) acc[c] = fmaf(v[u][c], wv[u], acc[c]);
+  }
+  const float inv = 1.f / fmaxf(ss, eps);
+  const int64_t bh = rid / Lq, row = rid - bh * Lq, b = bh / Hq;
+  TQ* orow = out + (out_tm ? (b * Lq + row) * Hq + (bh - b * Hq) : rid) * D + C * lane;
+#pragma unroll
+  for (int c = 0; c < C; ++c) Elem<TQ>::store(orow, c, acc[c] * inv);
 }
 
 // ---------------------------------------------------- batched decode on MFMA
@@ -1398,6 +1513,98 @@ int launch_decode(strata_ctx* ctx, const void* q, const void* k, const void* v, 
   return STRATA_OK;
 }
 
+// How a prefill launch covers (rows, keys): waves per workgroup, keys per LDS
+// tile and the key split.
+struct PrefillPlan {
+  int nw, kt, nsplit, chunk;
+};
+constexpr int kMaxPrefillSplits = 64;
+constexpr size_t kMaxPrefillWs = (size_t)512 << 20;  // longer splits where more would be needed
+size_t prefill_split_bytes(int64_t rows, int nsplit, int D) {
+  return nsplit > 1 ? (size_t)rows * nsplit * (D * 4 + 8) : 0;
+}
+PrefillPlan prefill_plan(int num_cus, bool f32, int B, int Hq, int Hkv, int Lq, int Lk, int D,
+                         int causal, size_t ws_bytes) {
+  const int64_t rows = (int64_t)Lq * (Hq / Hkv), all_rows = (int64_t)B * Hq * Lq;
+  PrefillPlan p;
+  p.nw = f32 ? 4 : (rows <= 32 ? 1 : rows <= 64 ? 2 : 4);
+  p.kt = f32 ? 64 : 32;
+  const int qr = (f32 ? 16 : 32) * p.nw;
+  const int64_t tiles = (rows + qr - 1) / qr * B * Hkv;
+  const int64_t longest = (Lk + p.kt - 1) / p.kt;  // steps of the longest tile
+  const double mean = std::max(1.0, causal ? (Lk - Lq / 2.0) / p.kt : (double)longest);
+  // Chunks that give every CU its share of workgroups: 3 of 4 waves (what fits
+  // and what the 8k causal launch runs best with), one of a single wave (8
+  // queries over 8k keys: 22 us against 30 with two).
+  const int per_cu = p.nw == 1 ? 1 : 3;
+  const int64_t least = f32 ? 1 : p.nw == 1 ? 4 : 8;
+  int64_t chunk = std::max(least, (int64_t)std::ceil(tiles * mean / (per_cu * (double)num_cus)));
+  chunk = std::max(chunk, (longest + kMaxPrefillSplits - 1) / kMaxPrefillSplits);
+  // Of that chunk and longer ones, the one whose cut of the longest tile's
+  // chain (us per step, measured) exceeds the cost of the partials by most: a
+  // merge launch, and their bytes written and read at 2.5 TB/s (100 queries
+  // after 4000 keys: 127 -> 30 us in 17 splits; a 1500-token prompt, 24 heads:
+  // 51 -> 46 in 3; 2048 tokens, 32 heads: 56 unsplit against 64 in 3).
+  const double step = f32 ? 5.5 : p.nw == 4 ? 0.9 : 1.1;
+  double best = 0;
+  p.nsplit = 1;
+  p.chunk = (int)(longest * p.kt);
+  for (; chunk < longest; chunk += chunk / 4 + 1) {
+    const int64_t ns = (longest + chunk - 1) / chunk;
+    if (prefill_split_bytes(all_rows, (int)ns, D) > ws_bytes) continue;
+    const double net = (longest - chunk) * step - 4 - all_rows * (mean / chunk) * (D * 4 + 8) * 2 / 2.5e6;
+    if (net > best) {
+      best = net;
+      p.nsplit = (int)ns;
+      p.chunk = (int)(chunk * p.kt);
+    }
+  }
+  // 64-key tiles (two workgroups per CU) halve the steps of launches that
+  // leave room: 2048 tokens, 32 heads 63 -> 56 us, 4096 tokens 155 -> 138;
+  // 4 x 2048 tokens 148 -> 154.
+  if (p.nsplit == 1 && p.nw == 4 && !f32 && tiles <= 4 * (int64_t)num_cus) p.kt = 64;
+  return p;
+}
+
+template <typename TQ, int D>
+void launch_prefill(strata_ctx* ctx, const void* q, const void* k, const void* v, int64_t kv_bs,
+                    int64_t kv_hs, const int32_t* qpos, int B, int Hq, int Hkv, int Lq, int Lk,
+                    int causal, float scale, float eps, void* out, const AttnExtra& ex,
+                    hipStream_t stream) {
+  constexpr bool f32 = sizeof(TQ) == 4;
+  const int64_t rows = (int64_t)B * Hq * Lq;
+  const PrefillPlan pl = prefill_plan(ctx->num_cus, f32, B, Hq, Hkv, Lq, Lk, D, causal, ex.ws_bytes);
+  PrefillSplit sp{pl.nsplit, pl.chunk, nullptr, nullptr};
+  if (pl.nsplit > 1) {
+    sp.o = static_cast<float*>(ex.ws);
+    sp.ms = reinterpret_cast<float2*>(sp.o + rows * pl.nsplit * D);
+  }
+  const int qr = (f32 ? 16 : 32) * pl.nw;
+  const int nqt = (int)(((int64_t)Lq * (Hq / Hkv) + qr - 1) / qr);
+  const dim3 grid(prefill_grid(nqt, B, Hkv), pl.nsplit);
+#define STRATA_PF(KERNEL)                                                                        \
+  hipLaunchKernelGGL(KERNEL, grid, dim3(64 * pl.nw), 0, stream, (const TQ*)q, (const TQ*)k,      \
+                     (const TQ*)v, kv_bs, kv_hs, qpos, B, Hq, Hkv, Lq, Lk, causal, scale, eps,   \
+                     ex.out_tm, (TQ*)out, sp)
+  if constexpr (f32) {
+    if (pl.nsplit > 1) STRATA_PF((attn_prefill_f32<D, true>));
+    else STRATA_PF((attn_prefill_f32<D, false>));
+  } else {
+#define STRATA_PFN(NW)                                                    \
+  if (pl.nsplit > 1) STRATA_PF((attn_prefill_mfma32<D, NW, 2, 32, true>)); \
+  else STRATA_PF((attn_prefill_mfma32<D, NW, 2, 32, false>))
+    if (pl.kt == 64) STRATA_PF((attn_prefill_mfma32<D, 4, 2, 64, false>));
+    else if (pl.nw == 1) { STRATA_PFN(1); }
+    else if (pl.nw == 2) { STRATA_PFN(2); }
+    else { STRATA_PFN(4); }
+#undef STRATA_PFN
+  }
+#undef STRATA_PF
+  if (pl.nsplit > 1)
+    hipLaunchKernelGGL((attn_prefill_merge<TQ, D>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0,
+                       stream, sp, rows, Hq, Lq, eps, ex.out_tm, (TQ*)out);
+}
+
 template <typename TQ, typename TK, typename TV>
 int launch_generic(const void* q, const void* k, const void* v, int64_t kv_bs, int64_t kv_hs,
                    const int32_t* qpos, int B, int Hq, int Hkv, int Lq, int Lk, int D, int causal,
@@ -1425,36 +1632,12 @@ int dispatch_types(strata_ctx* ctx, const void* q, const void* k, const void* v,
   }
   if constexpr (sizeof(TQ) == sizeof(TK) && sizeof(TK) == sizeof(TV)) {
     if (Lq > 1 && (D == 64 || D == 128)) {
-      if constexpr (sizeof(TQ) == 2) {
-        // 4 waves (128 query rows) per workgroup, two LDS stages of 32-key
-        // tiles (32 KB): three workgroups per CU (160 VGPRs), whose waves
-        // share each SIMD without sharing a barrier (8k causal: 586-602 us;
-        // 64-key tiles, two workgroups per CU: 606-628 us; 8 waves in one
-        // workgroup per CU: 683-696 us; a third stage: no gain)
-        constexpr int NWV = 4, NSTV = 2, KTV = 32;
-        const dim3 grid(prefill_grid((Lq + 32 * NWV - 1) / (32 * NWV), B, Hkv, Hq / Hkv));
-        if (D == 64)
-          hipLaunchKernelGGL((attn_prefill_mfma32<64, NWV, NSTV, KTV>), grid, dim3(64 * NWV), 0,
-                             stream, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, kv_bs,
-                             kv_hs, qpos, B, Hq, Hkv, Lq, Lk, causal, scale, eps, ex.out_tm,
-                             (bf16_t*)out);
-        else
-          hipLaunchKernelGGL((attn_prefill_mfma32<128, NWV, NSTV, KTV>), grid, dim3(64 * NWV), 0,
-                             stream, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, kv_bs,
-                             kv_hs, qpos, B, Hq, Hkv, Lq, Lk, causal, scale, eps, ex.out_tm,
-                             (bf16_t*)out);
-      } else {
-        // fp32: 16x16x4 MFMA tiles, 64 query rows per workgroup
-        const dim3 grid(prefill_grid((Lq + 63) / 64, B, Hkv, Hq / Hkv));
-        if (D == 64)
-          hipLaunchKernelGGL((attn_prefill_f32<64>), grid, dim3(256), 0, stream,
-                             (const float*)q, (const float*)k, (const float*)v, kv_bs, kv_hs, qpos,
-                             B, Hq, Hkv, Lq, Lk, causal, scale, eps, ex.out_tm, (float*)out);
-        else
-          hipLaunchKernelGGL((attn_prefill_f32<128>), grid, dim3(256), 0, stream,
-                             (const float*)q, (const float*)k, (const float*)v, kv_bs, kv_hs, qpos,
-                             B, Hq, Hkv, Lq, Lk, causal, scale, eps, ex.out_tm, (float*)out);
-      }
+      if (D == 64)
+        launch_prefill<TQ, 64>(ctx, q, k, v, kv_bs, kv_hs, qpos, B, Hq, Hkv, Lq, Lk, causal, scale,
+                               eps, out, ex, stream);
+      else
+        launch_prefill<TQ, 128>(ctx, q, k, v, kv_bs, kv_hs, qpos, B, Hq, Hkv, Lq, Lk, causal, scale,
+                                eps, out, ex, stream);
       STRATA_HIP_CHECK(hipGetLastError());
       return STRATA_OK;
     }
@@ -1486,6 +1669,16 @@ int strata_attn_decode_splits(strata_ctx* ctx, int B, int Hkv, int Lcap) {
     }
   }
   return nsplit;
+}
+
+// Bytes of workspace (AttnExtra::ws) with which the call splits its keys as it
+// does best; 0 when it needs none (decode, short keys, other head sizes).
+size_t strata_attn_prefill_ws(strata_ctx* ctx, int qd, int kd, int vd, int B, int Hq, int Hkv, int Lq,
+                              int Lk, int D, int causal) {
+  if (Lq <= 1 || (D != 64 && D != 128) || qd != kd || kd != vd) return 0;
+  const PrefillPlan p = prefill_plan(ctx->num_cus, qd == STRATA_F32, B, Hq, Hkv, Lq, Lk, D, causal,
+                                     kMaxPrefillWs);
+  return prefill_split_bytes((int64_t)B * Hq * Lq, p.nsplit, D);
 }
 
 int strata_attention_dispatch(strata_ctx* ctx, const void* q, int qd, const void* k, int kd,

@@ -57,6 +57,8 @@ struct strata_decoder {
   // for every call with the same batch and temperature.
   std::map<int, hipGraphExec_t> graphs;
   int graph_batch;
+  void* attn_ws = nullptr;  // key-split partials of prefill attention
+  size_t attn_ws_bytes = 0;
   float graph_temp;
   // Prefill GEMM layout of each layer's launches (q/k/v, o, gate/up, down),
   // re-laid out once at creation (null: re-laid out per call).
@@ -199,6 +201,8 @@ int forward_layers(strata_decoder* d, int B, int L, int pos0, void* stream, int 
                                    stream, d->rope_table));
     AttnExtra ex;
     ex.out_tm = 1;  // prefill writes [B, L, Hq, D], the o_proj input layout
+    ex.ws = d->attn_ws;
+    ex.ws_bytes = d->attn_ws_bytes;
     RC(strata_attention_dispatch(d->ctx, d->qr, STRATA_BF16, kc, STRATA_BF16, vc, STRATA_BF16,
                                  kv_bs, kv_hs, nullptr, B, Hq, Hkv, L, pos0 + L, D, 1, 1e-12f,
                                  d->attn, ex, stream));
@@ -395,6 +399,19 @@ int strata_decoder_create(strata_ctx* ctx, const strata_llama_config* cfg,
   if (!rc)
     rc = alloc(reinterpret_cast<void**>(&d->part),
                (size_t)kv->B * c.num_heads * part_stride(d->part_splits, c.head_dim) * 4);
+  // Key-split partials of prefill attention, sized for the prompt lengths up to
+  // max_tokens over a full cache; without them the attention runs unsplit.
+  for (int64_t l = max_tokens / kv->B; !rc && l > 1; l = l * 3 / 4)
+    d->attn_ws_bytes = std::max(d->attn_ws_bytes,
+                                strata_attn_prefill_ws(ctx, STRATA_BF16, STRATA_BF16, STRATA_BF16, kv->B,
+                                                       c.num_heads, c.num_kv_heads, (int)l, kv->Lmax,
+                                                       c.head_dim, 1));
+  d->attn_ws_bytes = std::min(d->attn_ws_bytes, (size_t)256 << 20);
+  if (d->attn_ws_bytes && hipMalloc(&d->attn_ws, d->attn_ws_bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    d->attn_ws = nullptr;
+    d->attn_ws_bytes = 0;
+  }
   if (!rc) rc = pack_prefill_weights(d);
   if (!rc) rc = build_decode_layouts(d);
   if (!rc) rc = strata_rope_table_launch(d->rope_table, kv->Lmax, c.head_dim, c.rope_theta, nullptr);
@@ -419,7 +436,7 @@ int strata_decoder_destroy(strata_decoder* d) {
   strata_gemv_layout_free(&d->head_lay);
   void* ptrs[] = {d->h, d->xn, d->q, d->k, d->v, d->qr, d->attn, d->o, d->gate, d->up, d->act,
                   d->delta, d->hn, d->logits, d->ids, d->tokens, d->counters, d->part, d->amax,
-                  d->rope_table, d->rope_cur};
+                  d->rope_table, d->rope_cur, d->attn_ws};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (d->stream) (void)hipStreamDestroy(d->stream);

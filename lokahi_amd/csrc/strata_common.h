@@ -211,6 +211,8 @@ struct AttnExtra {
   const int* dlen = nullptr;  // device key count (decode; overrides Lk, which is then capacity)
   float* part = nullptr;      // caller-owned split-K partials, B * Hq * part_stride(splits, D)
   int part_splits = 0;        // splits the partials buffer holds
+  void* ws = nullptr;         // prefill: caller-owned key-split partials (16-byte aligned)
+  size_t ws_bytes = 0;        // their size; 0: the keys are not split
   int out_tm = 0;             // prefill: write token-major [B, Lq, Hq, D]
 };
 

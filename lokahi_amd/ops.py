@@ -286,12 +286,29 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
             raise ValueError("k/v views do not match the given kv_strides")
     if out is None:
         out = torch.empty((B, Hq, Lq, D), dtype=q.dtype, device=q.device)
-    check(_lib().strata_attn_gqa(_ctx(dev), q.data_ptr(), _code(q), k.data_ptr(), _code(k),
-                                 v.data_ptr(), _code(v), bs, hs, _ptr(qpos), B, Hq, Hkv, Lq, Lk,
-                                 D, 1 if causal else 0, int(min(q_block_size, 2**31 - 1)),
-                                 int(min(k_block_size, 2**31 - 1)), float(eps), out.data_ptr(),
-                                 _stream(dev)))
+    ws = _attention_workspace(dev, q, k, v, causal) if Lq > 1 else None
+    check(_lib().strata_attn_gqa_ws(_ctx(dev), q.data_ptr(), _code(q), k.data_ptr(), _code(k),
+                                    v.data_ptr(), _code(v), bs, hs, _ptr(qpos), B, Hq, Hkv, Lq, Lk,
+                                    D, 1 if causal else 0, int(min(q_block_size, 2**31 - 1)),
+                                    int(min(k_block_size, 2**31 - 1)), float(eps), out.data_ptr(),
+                                    _ptr(ws), 0 if ws is None else ws.numel(), _stream(dev)))
     return out
+
+
+def _attention_workspace(dev: int, q, k, v, causal: bool) -> Optional[torch.Tensor]:
+    """Key-split partials of one call, from PyTorch's allocator (ordered on the
+    current stream, usable under graph capture); None when no split pays or
+    the memory is not there (the call then runs unsplit)."""
+    need = C.c_int64()
+    B, Hq, Lq, D = q.shape
+    check(_lib().strata_attn_workspace(_ctx(dev), _code(q), _code(k), _code(v), B, Hq, k.shape[1],
+                                       Lq, k.shape[2], D, 1 if causal else 0, C.byref(need)))
+    if not need.value:
+        return None
+    try:
+        return torch.empty(need.value, dtype=torch.uint8, device=q.device)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def attention_no_mask(q, k, v, position_ids=None, q_block_size: int = 32768,

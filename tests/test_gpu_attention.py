@@ -275,3 +275,55 @@ def test_decode_split_k_back_to_back_and_graph_replays(dev):
         assert rel_err(got, ref) < TOL_BF16 and np.abs(got - ref).max() < 2e-2
         e = to_np_f32(ops.attention(eq, ek, ev))
         assert rel_err(e, eref) < TOL_BF16
+
+
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,D,Lq,Lk,causal,given", [
+    ("bf16", 1, 8, 2, 128, 2, 1000, True, False),    # 8 packed rows: one wave per tile
+    ("bf16", 2, 6, 2, 64, 17, 1500, True, True),     # group 3, two waves, ragged rows and keys
+    ("bf16", 1, 8, 2, 128, 100, 4100, True, False),  # four waves, an uneven last split
+    ("bf16", 1, 6, 2, 128, 333, 1333, False, False), # not causal
+    ("bf16", 1, 6, 2, 128, 1400, 1400, True, False), # a prompt: tiles that end in the first split
+    ("f32", 1, 8, 2, 64, 512, 512, True, False), ("f32", 2, 6, 2, 128, 37, 437, True, True),
+    ("f32", 1, 4, 4, 64, 70, 300, False, False)])
+def test_prefill_key_splits(dev, dtype, B, Hq, Hkv, D, Lq, Lk, causal, given):
+    """Prefill whose keys are split over workgroups (with the workspace ops
+    passes) against float64, and against the call without a workspace.  Given
+    positions include rows that see no key (0, as keys masked for every row
+    give), rows that end in the first split and repeats.  The weights of a
+    split are exact powers of two apart from one fp32 rounding each, so the
+    split result stays within the unsplit one's own distance from float64
+    (bf16: weights and outputs rounded at 2^-9; fp32: 2^-24 per sum term)."""
+    import ctypes as C
+    from lokahi_amd import _abi, ops
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    gen = torch.Generator(device=dev).manual_seed(Lq + Lk)
+    q = torch.randn((B, Hq, Lq, D), generator=gen, device=dev).to(dt)
+    k = torch.randn((B, Hkv, Lk, D), generator=gen, device=dev).to(dt)
+    v = torch.randn((B, Hkv, Lk, D), generator=gen, device=dev).to(dt)
+    need = C.c_int64()
+    _abi.check(_abi.load().strata_attn_workspace(ops._ctx(0), ops._code(q), ops._code(k), ops._code(v),
+                                                 B, Hq, Hkv, Lq, Lk, D, int(causal), C.byref(need)))
+    assert need.value > 0  # the call is split
+    pos = torch.arange(Lk - Lq, Lk, device=dev, dtype=torch.int32).expand(B, Lq)
+    if given:
+        pos = torch.randint(0, Lk, (B, Lq), generator=gen, device=dev, dtype=torch.int32)
+        pos[0, 3], pos[0, 5], pos[-1, 7] = -1, 0, pos[-1, 6]
+    row = pos[:, None, :, None] if causal else torch.full((B, 1, Lq, 1), Lk, device=dev)
+    mask = torch.arange(Lk, device=dev) <= row
+    sc = torch.matmul(q.double(), k.double().repeat_interleave(Hq // Hkv, 1).transpose(2, 3).contiguous())
+    w = torch.exp(sc / D**0.5 - sc.amax(-1, keepdim=True) / D**0.5) * mask
+    ref = torch.matmul(w, v.double().repeat_interleave(Hq // Hkv, 1)) / w.sum(-1, keepdim=True).clamp_min(1e-12)
+    got = ops.attention(q, k, v, query_positions=pos if given else None, causal=causal)
+    one = torch.empty_like(q)
+    p32 = pos.contiguous()
+    _abi.check(_abi.load().strata_attn_gqa(
+        ops._ctx(0), q.data_ptr(), ops._code(q), k.data_ptr(), ops._code(k), v.data_ptr(), ops._code(v),
+        Hkv * Lk * D, Lk * D, p32.data_ptr() if given else None, B, Hq, Hkv, Lq, Lk, D, int(causal),
+        32768, 1024, C.c_float(1e-12), one.data_ptr(), ops._stream(0)))
+    err, err1 = (float((o.double() - ref).norm() / ref.norm()) for o in (got, one))
+    assert err1 < (5e-3 if dtype == "bf16" else 2e-6) and err < 1.2 * err1 + 1e-7, (err, err1)
+    # a NaN key reaches the rows that see it, and no other
+    k[0, 0, Lk // 3] = float("nan")
+    got = ops.attention(q, k, v, query_positions=pos if given else None, causal=causal)
+    sees = (mask[0, 0, :, Lk // 3] if causal else torch.ones(Lq, dtype=torch.bool, device=dev))
+    assert bool(got[0, :Hq // Hkv, sees].isnan().all()) and bool(got[0, Hq // Hkv:].isfinite().all())
