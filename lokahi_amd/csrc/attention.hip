@@ -730,11 +730,12 @@ __device__ __forceinline__ f32x16_t mfma32_bf16(const bf16x8_t& a, const bf16x8_
 
 // bf16 prefill on 32x32x16 MFMA tiles.  Workgroup = NW waves = 32 NW packed
 // query rows of one (b, KV head) (grid order as prefill_item); wave w owns rows
-// qt*32NW + 32w + 0..31.  S^T = K Q^T and O^T += V^T P^T run as 32x32x16
+// qt*32NW + 32w + 0..31 (KS > 1: KS such groups of waves, each with its own
+// ring, take the key tiles in turn and meet in LDS at the end).  S^T = K Q^T and O^T += V^T P^T run as 32x32x16
 // MFMAs whose 32-cycle issue leaves room for other waves' softmax on the
 // SIMD; the P^T operand is the S^T accumulator itself (no shuffles).
 // K and V tiles (KT keys) are streamed by direct global -> LDS loads into a
-// ring of NST stages, row-major with XOR-swizzled 16-byte chunks: the loads
+// ring of two stages, row-major with XOR-swizzled 16-byte chunks: the loads
 // of tile t + NST - 1 are issued at the top of tile t, and no register holds
 // them.  V^T operands come from row-major V through the LDS transpose read
 // (ds_read_b64_tr_b16: in each 16-lane group, lane l' receives element
@@ -744,8 +745,9 @@ __device__ __forceinline__ f32x16_t mfma32_bf16(const bf16x8_t& a, const bf16x8_
 // 32): lane l holds column l%32, rows 8(i/4) + 4(l/32) + i%4 for i < 16.
 typedef short v4i16_t __attribute__((ext_vector_type(4)));
 constexpr float kRescaleSlack = 8.f;
-template <int D, int NW, int NST, int KT, bool SPLIT>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(KT == 32 ? 3 : 2)))
+template <int D, int NW, int KS, int KT, bool SPLIT>
+__global__ __launch_bounds__(NW * KS * 64)
+__attribute__((amdgpu_waves_per_eu(KT == 32 && KS == 1 ? 3 : 2)))
 void attn_prefill_mfma32(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
     int64_t kv_bs, int64_t kv_hs, const int32_t* __restrict__ qpos, int B, int Hq, int Hkv,
@@ -756,20 +758,25 @@ void attn_prefill_mfma32(
   constexpr int NCHK = D / 8;         // 16-byte chunks per row
   constexpr int TILE = KT * ROW;      // bytes of one K or V tile
   constexpr int STAGE = 2 * TILE;     // K tile, then V tile
+  constexpr int NST = 2;              // stages of a ring
+  constexpr int RING = NST * STAGE;
   constexpr int AHEAD = NST - 1;      // tiles in flight ahead of the one computed
   constexpr int QR = 32 * NW;         // query rows per workgroup
   constexpr int NI = KT * NCHK / (64 * NW);  // 16-byte loads per thread per tile and operand
   static_assert(NI >= 1 && KT * NCHK % (64 * NW) == 0, "tile loads must divide over the workgroup");
-  __shared__ __attribute__((aligned(16))) uint8_t lds[NST * STAGE];
+  __shared__ __attribute__((aligned(16))) uint8_t lds_all[KS * RING];
   __shared__ int s_kmax;
+  __shared__ float2 s_ml[KS > 1 ? (KS - 1) * NW * 64 : 1];
 
   const int G = Hq / Hkv;
   int qt, b, hkv;
   if (!prefill_item(blockIdx.x, (Lq * G + QR - 1) / QR, B, Hkv, &qt, &b, &hkv))
     return;  // grid padding
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wave_all % NW, ks_id = wave_all / NW;
   const int c32 = lane & 31, h = lane >> 5;
+  uint8_t* lds = lds_all + ks_id * RING;
   const int pr = qt * QR + 32 * wave + c32;  // this lane's packed row
   const int row = pr / G, hq = hkv * G + (pr - row * G);
   const bool row_ok = row < Lq;
@@ -812,7 +819,7 @@ void attn_prefill_mfma32(
   const int split = SPLIT ? blockIdx.y : 0;
   const int kbeg = SPLIT ? split * sp.chunk : 0;
   const bool empty = SPLIT && !qpos && causal && kbeg > Lk - Lq + (min(qt * QR + QR, Lq * G) - 1) / G;
-  if (!empty) issue(kbeg, 0);
+  if (!empty) issue(kbeg + ks_id * KT, 0);
   const int64_t rid = ((int64_t)b * Hq + hq) * Lq + row;  // output row
   // Q^T fragments (the B operand of S^T): column = this lane's row, k = the
   // head dims 16 s + 8 h .. +8.
@@ -869,7 +876,6 @@ void attn_prefill_mfma32(
     const int col = 32 * db + v_col;
     v_off[db] = TILE + v_key * ROW + 16 * ((col / 8) ^ fv(v_key)) + 2 * (col % 8);
   }
-  static_assert(NST == 2 || NST == 3, "the tile loop cycles two or three stages");
 
   // Wait until at most n tiles' loads (2 NI each) of this thread are in flight.
   auto wait_tiles = [&](int n) {
@@ -879,21 +885,22 @@ void attn_prefill_mfma32(
     else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(6 * NI) : "memory");
   };
   static_assert(AHEAD <= 3, "wait_tiles covers up to three tiles in flight");
-  const int nt = (kend - kbeg + KT - 1) / KT;
+  // this wave's tiles: ks_id, ks_id + KS, ... of the nt_all
+  const int nt_all = (kend - kbeg + KT - 1) / KT;
+  const int nt = (nt_all - ks_id + KS - 1) / KS, steps = (nt_all + KS - 1) / KS;
   // prologue: tiles 0 .. AHEAD - 1 in flight, tile 0 complete
-  for (int t = 1; t < AHEAD && t < nt; ++t) issue(kbeg + t * KT, t);
-  wait_tiles(min(nt, AHEAD) - 1);
+  wait_tiles(0);
   __syncthreads();
   // one tile on stage ST (a compile-time constant, so every LDS address is a
   // lane offset plus an immediate)
   auto tile = [&](int t, auto STC) {
     constexpr int ST = decltype(STC)::value;
-    const int kb0 = kbeg + t * KT;
-    if (t + AHEAD < nt) issue(kb0 + AHEAD * KT, (ST + AHEAD) % NST);  // the stage tile t - 1 used
+    const int kb0 = kbeg + (t * KS + ks_id) * KT;
+    if (t + AHEAD < nt) issue(kb0 + AHEAD * KS * KT, (ST + AHEAD) % NST);  // the stage tile t - 1 used
     const uint8_t* ks = lds + ST * STAGE;
     // Waves whose rows see no key of the tile skip its math (one scalar
     // branch); rows of a live wave that see none are masked to p = 0.
-    if (__builtin_amdgcn_readfirstlane((int)(kb0 < wave_need))) {
+    if (__builtin_amdgcn_readfirstlane((int)(kb0 < wave_need && t < nt))) {
       __builtin_amdgcn_s_setprio(1);
       // st[kb][i] = score(this lane's row, key kb0 + 32 kb + 8(i/4) + 4h + i%4)
       f32x16_t sc[KB];
@@ -990,13 +997,52 @@ void attn_prefill_mfma32(
     wait_tiles(min(nt - 1, t + AHEAD) - (t + 1));
     __syncthreads();
   };
-  for (int t = 0; t < nt; t += NST) {
+  for (int t = 0; t < steps; t += NST) {
     tile(t, std::integral_constant<int, 0>{});
-    if (t + 1 >= nt) break;
+    if (t + 1 >= steps) break;
     tile(t + 1, std::integral_constant<int, 1>{});
-    if constexpr (NST == 3) {
-      if (t + 2 >= nt) break;
-      tile(t + 2, std::integral_constant<int, 2 % NST>{});
+  }
+
+  if constexpr (KS > 1) {
+    // The KS partial results of a row meet in LDS (the rings are done: every
+    // wave has passed the last tile's barrier): wave ks_id > 0 leaves o, then
+    // (m, l); wave 0 adds them up in order.
+    constexpr int PER = DB * 4 * 64 * 16;  // bytes of one wave's o
+    static_assert((KS - 1) * NW * PER <= KS * RING, "the rings hold the partial results");
+    if (ks_id > 0) {
+      const int slot = (ks_id - 1) * NW + wave;
+      float4* o = reinterpret_cast<float4*>(lds_all + slot * PER) + lane;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; i += 4)
+          o[(db * 4 + i / 4) * 64] =
+              make_float4(acc[db][i], acc[db][i + 1], acc[db][i + 2], acc[db][i + 3]);
+      s_ml[slot * 64 + lane] = make_float2(m_run, l_run);
+    }
+    __syncthreads();
+    if (ks_id > 0) return;
+#pragma unroll
+    for (int j = 0; j < KS - 1; ++j) {
+      const int slot = j * NW + wave;
+      const float2 ml = s_ml[slot * 64 + lane];
+      const float mn = fmaxf(m_run, ml.x);
+      const bool none = mn == -INFINITY;  // neither saw a key: both are zero
+      const float a0 = none ? 1.f : __builtin_amdgcn_exp2f(m_run - mn);
+      const float a1 = none ? 1.f : __builtin_amdgcn_exp2f(ml.x - mn);
+      const float4* o = reinterpret_cast<const float4*>(lds_all + slot * PER) + lane;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; i += 4) {
+          const float4 v4 = o[(db * 4 + i / 4) * 64];
+          acc[db][i] = fmaf(acc[db][i], a0, v4.x * a1);
+          acc[db][i + 1] = fmaf(acc[db][i + 1], a0, v4.y * a1);
+          acc[db][i + 2] = fmaf(acc[db][i + 2], a0, v4.z * a1);
+          acc[db][i + 3] = fmaf(acc[db][i + 3], a0, v4.w * a1);
+        }
+      l_run = fmaf(l_run, a0, ml.y * a1);
+      m_run = mn;
     }
   }
 
@@ -1516,7 +1562,7 @@ int launch_decode(strata_ctx* ctx, const void* q, const void* k, const void* v, 
 // How a prefill launch covers (rows, keys): waves per workgroup, keys per LDS
 // tile and the key split.
 struct PrefillPlan {
-  int nw, kt, nsplit, chunk;
+  int nw, ks, kt, nsplit, chunk;
 };
 constexpr int kMaxPrefillSplits = 64;
 constexpr size_t kMaxPrefillWs = (size_t)512 << 20;  // longer splits where more would be needed
@@ -1529,6 +1575,7 @@ PrefillPlan prefill_plan(int num_cus, bool f32, int B, int Hq, int Hkv, int Lq, 
   PrefillPlan p;
   p.nw = f32 ? 4 : (rows <= 32 ? 1 : rows <= 64 ? 2 : 4);
   p.kt = f32 ? 64 : 32;
+  p.ks = 1;
   const int qr = (f32 ? 16 : 32) * p.nw;
   const int64_t tiles = (rows + qr - 1) / qr * B * Hkv;
   const int64_t longest = (Lk + p.kt - 1) / p.kt;  // steps of the longest tile
@@ -1540,29 +1587,35 @@ PrefillPlan prefill_plan(int num_cus, bool f32, int B, int Hq, int Hkv, int Lq, 
   const int64_t least = f32 ? 1 : p.nw == 1 ? 4 : 8;
   int64_t chunk = std::max(least, (int64_t)std::ceil(tiles * mean / (per_cu * (double)num_cus)));
   chunk = std::max(chunk, (longest + kMaxPrefillSplits - 1) / kMaxPrefillSplits);
+  // Without a split, two wave groups of a workgroup share each tile's keys
+  // where that leaves CUs unused (1500 tokens, 24 heads: 51 -> 38 us; 2048
+  // tokens, 32 heads: 57 -> 51; 4 x 500 tokens stay: 24 against 26).
+  if (!f32 && p.nw == 4 && longest >= 6 &&
+      (tiles <= num_cus || (tiles <= 2 * (int64_t)num_cus && longest >= 32)))
+    p.ks = 2;
   // Of that chunk and longer ones, the one whose cut of the longest tile's
   // chain (us per step, measured) exceeds the cost of the partials by most: a
   // merge launch, and their bytes written and read at 2.5 TB/s (100 queries
-  // after 4000 keys: 127 -> 30 us in 17 splits; a 1500-token prompt, 24 heads:
-  // 51 -> 46 in 3; 2048 tokens, 32 heads: 56 unsplit against 64 in 3).
+  // after 4000 keys: 127 -> 32 us; 500 after 8000: 257 -> 94).
   const double step = f32 ? 5.5 : p.nw == 4 ? 0.9 : 1.1;
+  const double unsplit = longest * step / (p.ks == 2 ? 1.6 : 1.0);
   double best = 0;
   p.nsplit = 1;
   p.chunk = (int)(longest * p.kt);
   for (; chunk < longest; chunk += chunk / 4 + 1) {
     const int64_t ns = (longest + chunk - 1) / chunk;
     if (prefill_split_bytes(all_rows, (int)ns, D) > ws_bytes) continue;
-    const double net = (longest - chunk) * step - 4 - all_rows * (mean / chunk) * (D * 4 + 8) * 2 / 2.5e6;
+    const double net = unsplit - chunk * step - 4 - all_rows * (mean / chunk) * (D * 4 + 8) * 2 / 2.5e6;
     if (net > best) {
       best = net;
       p.nsplit = (int)ns;
       p.chunk = (int)(chunk * p.kt);
     }
   }
+  if (p.nsplit > 1) p.ks = 1;
   // 64-key tiles (two workgroups per CU) halve the steps of launches that
-  // leave room: 2048 tokens, 32 heads 63 -> 56 us, 4096 tokens 155 -> 138;
-  // 4 x 2048 tokens 148 -> 154.
-  if (p.nsplit == 1 && p.nw == 4 && !f32 && tiles <= 4 * (int64_t)num_cus) p.kt = 64;
+  // leave room: 4096 tokens, 32 heads 155 -> 138 us; 4 x 2048 tokens 148 -> 154.
+  if (p.nsplit == 1 && p.ks == 1 && p.nw == 4 && !f32 && tiles <= 4 * (int64_t)num_cus) p.kt = 64;
   return p;
 }
 
@@ -1583,7 +1636,7 @@ void launch_prefill(strata_ctx* ctx, const void* q, const void* k, const void* v
   const int nqt = (int)(((int64_t)Lq * (Hq / Hkv) + qr - 1) / qr);
   const dim3 grid(prefill_grid(nqt, B, Hkv), pl.nsplit);
 #define STRATA_PF(KERNEL)                                                                        \
-  hipLaunchKernelGGL(KERNEL, grid, dim3(64 * pl.nw), 0, stream, (const TQ*)q, (const TQ*)k,      \
+  hipLaunchKernelGGL(KERNEL, grid, dim3(64 * pl.nw * pl.ks), 0, stream, (const TQ*)q, (const TQ*)k,      \
                      (const TQ*)v, kv_bs, kv_hs, qpos, B, Hq, Hkv, Lq, Lk, causal, scale, eps,   \
                      ex.out_tm, (TQ*)out, sp)
   if constexpr (f32) {
@@ -1591,9 +1644,10 @@ void launch_prefill(strata_ctx* ctx, const void* q, const void* k, const void* v
     else STRATA_PF((attn_prefill_f32<D, false>));
   } else {
 #define STRATA_PFN(NW)                                                    \
-  if (pl.nsplit > 1) STRATA_PF((attn_prefill_mfma32<D, NW, 2, 32, true>)); \
-  else STRATA_PF((attn_prefill_mfma32<D, NW, 2, 32, false>))
-    if (pl.kt == 64) STRATA_PF((attn_prefill_mfma32<D, 4, 2, 64, false>));
+  if (pl.nsplit > 1) STRATA_PF((attn_prefill_mfma32<D, NW, 1, 32, true>)); \
+  else STRATA_PF((attn_prefill_mfma32<D, NW, 1, 32, false>))
+    if (pl.kt == 64) STRATA_PF((attn_prefill_mfma32<D, 4, 1, 64, false>));
+    else if (pl.ks == 2) STRATA_PF((attn_prefill_mfma32<D, 4, 2, 32, false>));
     else if (pl.nw == 1) { STRATA_PFN(1); }
     else if (pl.nw == 2) { STRATA_PFN(2); }
     else { STRATA_PFN(4); }

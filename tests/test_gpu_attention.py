@@ -327,3 +327,35 @@ def test_prefill_key_splits(dev, dtype, B, Hq, Hkv, D, Lq, Lk, causal, given):
     got = ops.attention(q, k, v, query_positions=pos if given else None, causal=causal)
     sees = (mask[0, 0, :, Lk // 3] if causal else torch.ones(Lq, dtype=torch.bool, device=dev))
     assert bool(got[0, :Hq // Hkv, sees].isnan().all()) and bool(got[0, Hq // Hkv:].isfinite().all())
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,Lq,Lk", [(24, 8, 128, 200, 200), (6, 2, 64, 193, 211),
+                                            (32, 8, 128, 700, 707), (8, 8, 128, 130, 1000),
+                                            (32, 8, 128, 1100, 1100), (32, 8, 128, 3000, 3000)])
+def test_prefill_without_split(dev, Hq, Hkv, D, Lq, Lk):
+    """Unsplit bf16 prefill (no workspace): key tiles shared by two wave groups
+    of a workgroup (an odd and an even number of tiles, a last tile for one
+    group only), 64-key tiles, and the plain kernel, against float64 rows and
+    each row's independence of the others in its tile."""
+    import ctypes as C
+    from lokahi_amd import _abi, ops
+    gen = torch.Generator(device=dev).manual_seed(Lq + D)
+    q, k, v = (torch.randn((1, h, l, D), generator=gen, device=dev).bfloat16()
+               for h, l in ((Hq, Lq), (Hkv, Lk), (Hkv, Lk)))
+
+    def call(q):
+        out = torch.empty_like(q)
+        _abi.check(_abi.load().strata_attn_gqa(
+            ops._ctx(0), q.data_ptr(), ops._code(q), k.data_ptr(), ops._code(k), v.data_ptr(),
+            ops._code(v), Hkv * Lk * D, Lk * D, None, 1, Hq, Hkv, q.shape[2], Lk, D, 1, 32768, 1024,
+            C.c_float(1e-12), out.data_ptr(), ops._stream(0)))
+        return out
+
+    got = call(q)
+    rows = torch.tensor(sorted({0, 1, 31, 32, Lq // 2, Lq - 2, Lq - 1}), device=dev)
+    sc = torch.matmul(q[:, :, rows].double(),
+                      k.double().repeat_interleave(Hq // Hkv, 1).transpose(2, 3).contiguous()) / D**0.5
+    sc.masked_fill_(torch.arange(Lk, device=dev) > (rows + Lk - Lq)[:, None], float("-inf"))
+    ref = torch.matmul(torch.softmax(sc, -1), v.double().repeat_interleave(Hq // Hkv, 1))
+    assert float((got[:, :, rows].double() - ref).norm() / ref.norm()) < 5e-3
+    assert bool(got.isfinite().all())
