@@ -85,20 +85,20 @@ __device__ __forceinline__ void group_tile(int t, int mt, int nt, int* tm, int* 
 // words.  Three stages: the loads of step g + 2 are issued at the top of
 // step g.
 constexpr int kWBytes = 4 * 64 * 32;             // 8 KB
-constexpr int kSBBytes = 4 * 64 * 4;             // 1 KB
+constexpr int kSBBytes = 4 * 64 * 4;             // 1 KB (MLX: s words, then as many b words)
 constexpr int kStages = 3;
 
 // N % 256 == 0, K % 64 == 0, and every operand under 4 GiB (the launcher
 // checks); any M.
 // Per-M-tile constants: TM = 256 (one workgroup per CU) or 128 (two per
 // CU, for problems with few 256-row tiles).
-template <int TM>
+template <int TM, bool MLX>
 struct Tile {
   static constexpr int MB = TM / 32;                    // 32-row MFMA blocks per wave
   static constexpr int XCH = TM * 8 / NTHR;             // X chunks (16 B) per thread per step
   static constexpr int kXBytes = TM * TK * 2;
-  static constexpr int kStage = kXBytes + kWBytes + kSBBytes;
-  static constexpr int kDmaPerStep = XCH + 2 + 1;       // per lane: X chunks, W halves, (s, b)
+  static constexpr int kStage = kXBytes + kWBytes + (MLX ? 2 : 1) * kSBBytes;
+  static constexpr int kDmaPerStep = XCH + 2 + (MLX ? 2 : 1);  // per lane: X chunks, W halves, s and b
   static constexpr size_t kLds = (size_t)kStages * kStage;
 };
 
@@ -109,6 +109,13 @@ struct GemmOut {
   void* y[kMaxGemmProblems];
   int n0[kMaxGemmProblems + 1];
   int count;
+};
+
+// MLX layout: the linears' own tensors, read as they are.
+struct GemmSrc {
+  const uint32_t* w[kMaxGemmProblems];
+  const uint16_t* s[kMaxGemmProblems];
+  const uint16_t* b[kMaxGemmProblems];
 };
 
 // The part of the problem space one launch covers: M tiles 0 .. mt - 1 (the
@@ -125,13 +132,18 @@ struct GemmSplit {
 // SPLIT: the launch's K slices write fp32 partial sums (sp.part) instead
 // of the outputs; a separate instance, so the other one carries no partial
 // pointer arithmetic (it spilled to scratch when it did).
-template <int TM, typename YT, bool SPLIT>
+// MLX: codes, scales and biases come from the linears' own tensors (src)
+// instead of the re-laid-out copy: 32 bytes of a row per K step (the other
+// three steps of a 128-byte line come from L2), and s and b as the 4-byte pair
+// of groups that holds this step's (K % 128 == 0).
+template <int TM, typename YT, bool SPLIT, bool MLX>
 __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(TM == 256 ? 1 : 2, TM == 256 ? 1 : 2)))
 void q4_gemm_mfma_kernel(const uint16_t* __restrict__ x, int M, int K,
                          const uint32_t* __restrict__ wt, const uint32_t* __restrict__ sbt,
-                         int N, GemmOut out, GemmSplit sp) {
-  constexpr int MB = Tile<TM>::MB, XCH = Tile<TM>::XCH, kXBytes = Tile<TM>::kXBytes;
-  constexpr int kStage = Tile<TM>::kStage, kDmaPerStep = Tile<TM>::kDmaPerStep;
+                         int N, GemmOut out, GemmSplit sp, GemmSrc src) {
+  using T = Tile<TM, MLX>;
+  constexpr int MB = T::MB, XCH = T::XCH, kXBytes = T::kXBytes;
+  constexpr int kStage = T::kStage, kDmaPerStep = T::kDmaPerStep;
   constexpr int QPS = 8 / MB;  // dequant quarters per sub-step
   // Sub-step that reads step g + 1's code words and scales (after this
   // lane's loads of step g + 1 are waited for, which needs every load of
@@ -158,9 +170,19 @@ void q4_gemm_mfma_kernel(const uint16_t* __restrict__ x, int M, int K,
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(
       (__attribute__((address_space(3))) uint8_t*)lds);
 
+  // The tile's problem (wave-uniform): the last one starting at or before n0.
+  int p = 0;
+#pragma unroll
+  for (int t = 1; t < kMaxGemmProblems; ++t)
+    if (t < out.count && n0 >= out.n0[t]) p = t;
+  const int nl = n0 - out.n0[p];  // the tile's first row in its linear
+
   const v4i32_t rx = rsrc(x, (uint32_t)((size_t)M * kb));
-  const v4i32_t rw = rsrc(wt, (uint32_t)((size_t)G * wgb));
-  const v4i32_t rs = rsrc(sbt, (uint32_t)((size_t)G * sgb));
+  const v4i32_t rw = MLX ? rsrc(src.w[p] + (int64_t)nl * (K / 8), (uint32_t)TN * (K / 2))
+                         : rsrc(wt, (uint32_t)((size_t)G * wgb));
+  const v4i32_t rs = MLX ? rsrc(src.s[p] + (int64_t)nl * G, (uint32_t)TN * G * 2)
+                         : rsrc(sbt, (uint32_t)((size_t)G * sgb));
+  const v4i32_t rb = MLX ? rsrc(src.b[p] + (int64_t)nl * G, (uint32_t)TN * G * 2) : rs;
 
   // X DMA instruction i of wave w fills 16-byte slots S = (8w + i) * 64 + lane
   // of the stage: row r = S / 8, slot p = lane % 8 holds chunk
@@ -168,9 +190,12 @@ void q4_gemm_mfma_kernel(const uint16_t* __restrict__ x, int M, int K,
   const uint32_t xl0 = (lane >> 3) * kb + (((lane & 7) ^ (lane >> 4)) << 4);
   const uint32_t xl1 = (lane >> 3) * kb + (((lane & 7) ^ (4 + (lane >> 4))) << 4);
   // W DMA j of this wave: 16-byte chunk q = 64 j + lane = row q/2, half q%2
-  // of the group-major codes (rows of one group are 32 bytes apart).
-  const uint32_t wl = lane * 16;
-  const uint32_t sl = lane * 4;
+  // of the group-major codes (rows of one group are 32 bytes apart); in the
+  // MLX layout rows are K / 2 bytes apart and a row's halves are swapped here
+  // when bit 2 of the row is set.
+  const uint32_t wl = MLX ? (lane >> 1) * (uint32_t)(K / 2) + (((lane & 1) ^ ((lane >> 3) & 1)) << 4)
+                          : lane * 16;
+  const uint32_t sl = MLX ? lane * (uint32_t)G * 2 : lane * 4;
   // DMA piece p (0 .. kDmaPerStep - 1) of step g into stage stg: X chunks
   // 0-7, the two weight halves, the scales, the biases.
   auto issue1 = [&](int g, int stg, int p) {
@@ -181,7 +206,12 @@ void q4_gemm_mfma_kernel(const uint16_t* __restrict__ x, int M, int K,
     } else if (p < XCH + 2) {
       const int j = p - XCH;
       dma16(base + kXBytes + wave * 2048 + j * 1024, wl, rw,
-            g * wgb + (uint32_t)(n0 + wave * WN + j * 32) * 32);
+            MLX ? (uint32_t)(wave * WN + j * 32) * (K / 2) + g * 32
+                : g * wgb + (uint32_t)(n0 + wave * WN + j * 32) * 32);
+    } else if (MLX) {
+      const int j = p - XCH - 2;
+      dma4(base + kXBytes + kWBytes + j * kSBBytes + wave * 256, sl, j ? rb : rs,
+           (uint32_t)(wave * WN) * G * 2 + (g & ~1) * 2);
     } else {
       dma4(base + kXBytes + kWBytes + wave * 256, sl, rs, g * sgb + (uint32_t)(n0 + wave * WN) * 4);
     }
@@ -201,17 +231,19 @@ void q4_gemm_mfma_kernel(const uint16_t* __restrict__ x, int M, int K,
   // C (32 x 32): lane l holds column l % 32, rows 8 (i / 4) + 4 (l / 32) +
   // i % 4 for i < 16.
   const int c32 = lane & 31, kh = lane >> 5;
-  // A fragment (mb, kblk): row mb*32 + c32, 16-byte chunk 2 kblk + kh of the
+  // k order: k block kblk of a step takes k 8 kblk .. +8 (kh = 0) and 32 +
+  // 8 kblk .. +8 (kh = 1), so a lane's code words are one 16-byte half of its
+  // row's group.
+  // A fragment (mb, kblk): row mb*32 + c32, 16-byte chunk 4 kh + kblk of the
   // swizzled row ((r >> 1) & 7 == (c32 >> 1) & 7 for every mb).
   auto aoff = [&](int mb, int kblk) {
-    return ((mb * 32 + c32) * TK + (((2 * kblk + kh) ^ ((c32 >> 1) & 7)) << 3)) * 2;
+    return ((mb * 32 + c32) * TK + (((4 * kh + kblk) ^ ((c32 >> 1) & 7)) << 3)) * 2;
   };
 
-  // B fragment (nb, kblk) = 8 codes of row nb*32 + c32, word 2 kblk + kh of
-  // the group, found as word kblk of the row's 16-byte half kh (the re-layout
-  // stores each row as its even words, then its odd words, the two halves
-  // swapped on rows with bit 2 set so that the 8 lanes of one LDS read cycle
-  // cover all banks).  bf[nb][kblk]: frag (nb, k) of step g is rewritten for
+  // B fragment (nb, kblk) = 8 codes of row nb*32 + c32, word 4 kh + kblk of
+  // the group: word kblk of the row's 16-byte half kh (the two halves are
+  // swapped in LDS on rows with bit 2 set so that the 8 lanes of one LDS read
+  // cycle cover all banks).  bf[nb][kblk]: frag (nb, k) of step g is rewritten for
   // step g + 1 in the k block after its last use (k block 3 of step g + 1
   // during k block 0 of step g + 1).
   uint4 bf[NB][KB];
@@ -220,11 +252,26 @@ void q4_gemm_mfma_kernel(const uint16_t* __restrict__ x, int M, int K,
   // ahead of their first use.
   uint4 dw[NB], dwn[NB];
   float dsf[NB], dbf[NB];
-  uint32_t dsbn[NB];
-  auto read_sb = [&](int stg, uint32_t (&o)[NB]) {
+  uint32_t dsbn[NB], dbn[NB];  // (MLX: the s pair, and the b pair in dbn)
+  auto read_sb = [&](int stg) {
     const uint8_t* ss = lds + stg * kStage + kXBytes + kWBytes + wave * 256;
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) o[nb] = *reinterpret_cast<const uint32_t*>(ss + (nb * 32 + c32) * 4);
+    for (int nb = 0; nb < NB; ++nb) {
+      dsbn[nb] = *reinterpret_cast<const uint32_t*>(ss + (nb * 32 + c32) * 4);
+      if (MLX) dbn[nb] = *reinterpret_cast<const uint32_t*>(ss + kSBBytes + (nb * 32 + c32) * 4);
+    }
+  };
+  auto set_sb = [&](int g) {  // of group g, from what read_sb read
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      if (MLX) {
+        dsf[nb] = __uint_as_float((g & 1) ? dsbn[nb] & 0xffff0000u : dsbn[nb] << 16);
+        dbf[nb] = __uint_as_float((g & 1) ? dbn[nb] & 0xffff0000u : dbn[nb] << 16);
+      } else {
+        dsf[nb] = __uint_as_float(dsbn[nb] << 16);
+        dbf[nb] = __uint_as_float(dsbn[nb] & 0xffff0000u);
+      }
+    }
   };
   auto read_w = [&](int stg, uint4 (&o)[NB]) {
     const uint8_t* ws = lds + stg * kStage + kXBytes + wave * 2048;
@@ -270,13 +317,9 @@ void q4_gemm_mfma_kernel(const uint16_t* __restrict__ x, int M, int K,
   issue(min(g0 + 1, g1 - 1), 1);
   vm_wait_step();
   __syncthreads();
-  read_sb(0, dsbn);
+  read_sb(0);
   read_w(0, dw);
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-    dsf[nb] = __uint_as_float(dsbn[nb] << 16);
-    dbf[nb] = __uint_as_float(dsbn[nb] & 0xffff0000u);
-  }
+  set_sb(g0);
   dequant_all(0);
 
   // One K step = 32 sub-steps (k block kblk = st / 8, row block mb = st % 8),
@@ -317,16 +360,13 @@ void q4_gemm_mfma_kernel(const uint16_t* __restrict__ x, int M, int K,
       if (st == kReadSt - 1) vm_wait_step();
 #endif
       if (st == kReadSt) {  // step g + 1's words, four sub-steps before their first use
-        read_sb(stg1, dsbn);
+        read_sb(stg1);
         read_w(stg1, dwn);
       }
       if (st == 3 * MB) {  // step g's last dequant was one sub-step earlier
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          dw[nb] = dwn[nb];
-          dsf[nb] = __uint_as_float(dsbn[nb] << 16);
-          dbf[nb] = __uint_as_float(dsbn[nb] & 0xffff0000u);
-        }
+        for (int nb = 0; nb < NB; ++nb) dw[nb] = dwn[nb];
+        set_sb(g + 1);
       }
 #ifndef GEMM_EXP_NO_DEQ
 #pragma unroll
@@ -356,13 +396,8 @@ void q4_gemm_mfma_kernel(const uint16_t* __restrict__ x, int M, int K,
         for (int i = 0; i < 16; ++i)
           pb[(int64_t)(mb * 32 + 8 * (i / 4) + i % 4) * ld + nb * 32] = acc[mb][nb][i];
   } else {
-  // The tile's problem (wave-uniform): the last one starting at or before n0.
-  int p = 0;
-#pragma unroll
-  for (int t = 1; t < kMaxGemmProblems; ++t)
-    if (t < out.count && n0 >= out.n0[t]) p = t;
   const int np = out.n0[p + 1] - out.n0[p];
-  YT* yb = static_cast<YT*>(out.y[p]) + (int64_t)(m0 + 4 * kh) * np + (n0 - out.n0[p]) +
+  YT* yb = static_cast<YT*>(out.y[p]) + (int64_t)(m0 + 4 * kh) * np + nl +
            wave * WN + c32;
   if (m0 + TM <= M) {  // a full tile (wave-uniform): stores without a row check
 #pragma unroll
@@ -425,9 +460,8 @@ __global__ __launch_bounds__(256) void q4_gemm_splitk_reduce(const float* __rest
 
 // Re-layout of one q4 weight for the kernel above (a pass over the weight,
 // ~1% of the GEMM at 8192 rows): codes group-major, wt[g][n][8 words], so a
-// K step's rows are contiguous, each row's words in the order 0 2 4 6 | 1 3
-// 5 7 (halves swapped when bit 2 of n is set); scale and bias of (n, g)
-// packed in one word, sbt[g][n] = s | b << 16.
+// K step's rows are contiguous, each row's two 16-byte halves swapped when bit
+// 2 of n is set; scale and bias of (n, g) packed in one word, sbt[g][n] = s | b << 16.
 // Rows 0 .. Np - 1 of one weight go to rows n_off .. of a layout Ntot rows
 // wide (the linears of one launch, concatenated).  A workgroup moves a tile
 // of 32 rows x 8 groups: thread t takes row t / 8 and group t % 8, so the
@@ -443,10 +477,9 @@ __global__ __launch_bounds__(256) void q4_gemm_relayout_kernel(
   const int64_t i = (int64_t)nl * G + g;  // (row, group) of the source
   const int n = n_off + nl;
   const uint4 lo = w[i * 2], hi = w[i * 2 + 1];
-  const uint4 ev = make_uint4(lo.x, lo.z, hi.x, hi.z), od = make_uint4(lo.y, lo.w, hi.y, hi.w);
   const int sw = (n >> 2) & 1;
-  wt[((int64_t)g * Ntot + n) * 2 + sw] = ev;
-  wt[((int64_t)g * Ntot + n) * 2 + (sw ^ 1)] = od;
+  wt[((int64_t)g * Ntot + n) * 2 + sw] = lo;
+  wt[((int64_t)g * Ntot + n) * 2 + (sw ^ 1)] = hi;
   sbt[(int64_t)g * Ntot + n] = (uint32_t)s[i] | ((uint32_t)b[i] << 16);
 }
 
@@ -565,23 +598,39 @@ size_t plan_part_bytes(const SplitPlan& pl, int M, const strata_q4_weight* ws) {
   return need;
 }
 
-template <int TM, typename YT, bool SPLIT>
-void gemm_go(const void* x, int M, int K, const uint32_t* wt, const uint32_t* sbt, int N,
-             const GemmOut& out, const GemmSplit& sp, hipStream_t st) {
+template <int TM, typename YT, bool SPLIT, bool MLX>
+void gemm_go_l(const void* x, int M, int K, const uint32_t* wt, const uint32_t* sbt, int N,
+               const GemmOut& out, const GemmSplit& sp, const GemmSrc& src, hipStream_t st) {
+  using T = Tile<TM, MLX>;
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute((const void*)q4_gemm_mfma_kernel<TM, YT, SPLIT>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, Tile<TM>::kLds);
+    (void)hipFuncSetAttribute((const void*)q4_gemm_mfma_kernel<TM, YT, SPLIT, MLX>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, T::kLds);
     attr = true;
   }
-  hipLaunchKernelGGL((q4_gemm_mfma_kernel<TM, YT, SPLIT>), dim3(sp.mt * sp.nts * sp.S), dim3(NTHR),
-                     Tile<TM>::kLds, st, (const uint16_t*)x, M, K, wt, sbt, N, out, sp);
+  hipLaunchKernelGGL((q4_gemm_mfma_kernel<TM, YT, SPLIT, MLX>), dim3(sp.mt * sp.nts * sp.S),
+                     dim3(NTHR), T::kLds, st, (const uint16_t*)x, M, K, wt, sbt, N, out, sp, src);
+}
+template <int TM, typename YT, bool SPLIT>
+void gemm_go(const void* x, int M, int K, const uint32_t* wt, const uint32_t* sbt, int N,
+             const GemmOut& out, const GemmSplit& sp, const GemmSrc& src, hipStream_t st) {
+  if (wt) gemm_go_l<TM, YT, SPLIT, false>(x, M, K, wt, sbt, N, out, sp, src, st);
+  else gemm_go_l<TM, YT, SPLIT, true>(x, M, K, wt, sbt, N, out, sp, src, st);
 }
 }  // namespace
 
 size_t strata_q4_gemm_mfma_part_bytes(int M, int K, const strata_q4_weight* ws, int count) {
   if (count < 1 || count > kMaxGemmProblems) return 0;
   return plan_part_bytes(split_plan(M, K, ws, count, num_cus(), true), M, ws);
+}
+
+bool strata_q4_gemm_mlx_fits(int K, const strata_q4_weight* ws, int count) {
+  if (K % 128 != 0 || (uint64_t)K / 2 * TN >= (1ull << 32)) return false;
+  for (int p = 0; p < count; ++p)
+    if (!aligned16(ws[p].w) ||
+        ((reinterpret_cast<uintptr_t>(ws[p].scales) | reinterpret_cast<uintptr_t>(ws[p].biases)) & 3))
+      return false;
+  return true;
 }
 
 int strata_q4_gemm_mfma_launch(const void* x, int M, int K, const strata_q4_weight* ws, int count,
@@ -602,10 +651,19 @@ int strata_q4_gemm_mfma_run(const void* x, int M, int K, const void* packed,
   STRATA_REQUIRE(M > 0, "q4 GEMM (256-column kernel): M must be positive");
   STRATA_REQUIRE((uint64_t)M * K * 2 < (1ull << 32) && (uint64_t)N * K / 2 < (1ull << 32),
                  "q4 GEMM (256-column kernel): operands must be under 4 GiB");
-  STRATA_REQUIRE(packed && (reinterpret_cast<uintptr_t>(packed) & 15) == 0,
-                 "q4 GEMM: unaligned packed buffer");
+  STRATA_REQUIRE((reinterpret_cast<uintptr_t>(packed) & 15) == 0, "q4 GEMM: unaligned packed buffer");
+  GemmSrc src{};
+  if (!packed) {
+    STRATA_REQUIRE(strata_q4_gemm_mlx_fits(K, ws, count),
+                   "q4 GEMM: the MLX layout needs K %% 128 == 0 and aligned tensors");
+    for (int p = 0; p < count; ++p) {
+      src.w[p] = ws[p].w;
+      src.s[p] = ws[p].scales;
+      src.b[p] = ws[p].biases;
+    }
+  }
   const uint32_t* wt = static_cast<const uint32_t*>(packed);
-  const uint32_t* sbt = wt + (size_t)N * K / 8;
+  const uint32_t* sbt = wt ? wt + (size_t)N * K / 8 : nullptr;
   hipStream_t st = as_stream(stream);
   const bool bf = y_dtype == STRATA_BF16;
   const int cus = num_cus();
@@ -616,13 +674,13 @@ int strata_q4_gemm_mfma_run(const void* x, int M, int K, const void* packed,
     const int TM = big ? 256 : 128;
     const GemmSplit sp{(M + TM - 1) / TM, ntile0, nts, S, S > 1 ? part : nullptr};
     if (S > 1)  // 128-row tiles; the partial sums are fp32 whatever y's dtype
-      gemm_go<128, float, true>(x, M, K, wt, sbt, N, out, sp, st);
+      gemm_go<128, float, true>(x, M, K, wt, sbt, N, out, sp, src, st);
     else if (big) {
-      if (bf) gemm_go<256, bf16_t, false>(x, M, K, wt, sbt, N, out, sp, st);
-      else gemm_go<256, float, false>(x, M, K, wt, sbt, N, out, sp, st);
+      if (bf) gemm_go<256, bf16_t, false>(x, M, K, wt, sbt, N, out, sp, src, st);
+      else gemm_go<256, float, false>(x, M, K, wt, sbt, N, out, sp, src, st);
     } else {
-      if (bf) gemm_go<128, bf16_t, false>(x, M, K, wt, sbt, N, out, sp, st);
-      else gemm_go<128, float, false>(x, M, K, wt, sbt, N, out, sp, st);
+      if (bf) gemm_go<128, bf16_t, false>(x, M, K, wt, sbt, N, out, sp, src, st);
+      else gemm_go<128, float, false>(x, M, K, wt, sbt, N, out, sp, src, st);
     }
   };
   SplitPlan pl = split_plan(M, K, ws, count, cus, part != nullptr);

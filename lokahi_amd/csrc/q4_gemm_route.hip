@@ -2,8 +2,8 @@
 // the q4 -> bf16 expansion behind strata_dequantize_q4.
 //
 // Same maths as mx.quantized_matmul(transpose=True) (src/ollm/llama_mlx.py:53-74)
-// on the prefill path: the fused-dequant MFMA GEMM for 40 rows and more
-// (q4_gemm_mfma.hip), the skinny MFMA kernel below (q4_gemm_skinny.hip),
+// on the prefill path: the fused-dequant MFMA GEMM for many rows
+// (q4_gemm_mfma.hip), the skinny MFMA kernel for few (q4_gemm_skinny.hip),
 // the 128 x 128 tile kernel for shapes neither takes (q4_gemm.hip).
 #include <hip/hip_runtime.h>
 
@@ -62,29 +62,28 @@ int strata_q4_dequant_launch(const uint32_t* w, const uint16_t* s, const uint16_
 
 int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const strata_q4_weight* ws,
                          int count, int y_dtype, void* stream, const GemmPacked* packed) {
-  const size_t ye = y_dtype == STRATA_BF16 ? 2 : 4;
   // Each linear goes its own way, so that it gives the same bits in a
   // fused call as alone:
-  //   * from kMfmaMidRows rows, N a multiple of 256: the 256-column MFMA
-  //     kernel over all rows (a partial last row tile; K split over several
-  //     workgroups for linears with few tiles), the linears of one call in
-  //     as few launches as their splits allow;
-  //   * below that, shapes the skinny kernel takes (K % 512 == 0, N % 16 ==
-  //     0): the skinny kernel, rows in slices of 64, one launch per slice;
+  //   * from kMfmaMidRows rows (65 for fewer than kMidWideN columns), N a
+  //     multiple of 256: the 256-column MFMA kernel over all rows (a partial
+  //     last row tile; K split over several workgroups for linears with few
+  //     tiles), the linears of one call in as few launches as their splits
+  //     allow;
+  //   * up to 64 rows otherwise, shapes the skinny kernel takes (K % 512 == 0,
+  //     N % 16 == 0): the skinny kernel, one launch;
   //   * anything else: the 128 x 128 kernel, one launch per linear.
-  const int mid_min = kMfmaMidRows;
   const bool x_ok = aligned16(x) && K % 64 == 0 && (uint64_t)M * K * 2 < (1ull << 32);
-  strata_q4_weight fast[kMaxGemmProblems];
-  int nfast = 0;
+  strata_q4_weight fast[kMaxGemmProblems], few[kMaxGemmProblems];
+  int nfast = 0, nfew = 0;
   int64_t Nfast = 0;
   for (int i = 0; i < count; ++i) {
-    bool f = false;
-    if (M >= mid_min)
-      f = x_ok && ws[i].N % 256 == 0 && aligned16(ws[i].w) &&
-          (uint64_t)(Nfast + ws[i].N) * K / 2 < (1ull << 32);
-    else
-      f = aligned16(x) && strata_q4_skinny_fits(1, K, &ws[i], 1);
-    if (f && nfast < kMaxGemmProblems) {
+    const bool mid = M >= kMfmaMidRows && x_ok && ws[i].N % 256 == 0 && aligned16(ws[i].w) &&
+                     (uint64_t)(Nfast + ws[i].N) * K / 2 < (1ull << 32) && nfast < kMaxGemmProblems;
+    const bool skinny = M <= kSkinnyMaxRows && aligned16(x) && strata_q4_skinny_fits(M, K, &ws[i], 1) &&
+                        nfew < kMaxGemmProblems;
+    if (skinny && !(mid && ws[i].N >= kMidWideN)) {
+      few[nfew++] = ws[i];
+    } else if (mid) {
       fast[nfast++] = ws[i];
       Nfast += ws[i].N;
     } else {
@@ -93,21 +92,11 @@ int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const str
       if (rc) return rc;
     }
   }
-  if (nfast == 0) return STRATA_OK;
-  if (M < mid_min) {
-    for (int r0 = 0; r0 < M; r0 += kSkinnyMaxRows) {
-      const int mr = std::min(kSkinnyMaxRows, M - r0);
-      strata_q4_weight sl[kMaxGemmProblems];
-      for (int i = 0; i < nfast; ++i) {
-        sl[i] = fast[i];
-        sl[i].y = static_cast<char*>(fast[i].y) + (size_t)r0 * fast[i].N * ye;
-      }
-      const int rc = strata_q4_gemm_skinny(static_cast<const uint16_t*>(x) + (size_t)r0 * K, mr,
-                                           K, sl, nfast, y_dtype, stream);
-      if (rc) return rc;
-    }
-    return STRATA_OK;
+  if (nfew > 0) {
+    const int rc = strata_q4_gemm_skinny(x, M, K, few, nfew, y_dtype, stream);
+    if (rc) return rc;
   }
+  if (nfast == 0) return STRATA_OK;
   // The decoder's load-time re-layout is used when it was built for exactly
   // these linears (all of them on this path, the same total N and K);
   // otherwise this call re-lays the weights out into the scratch arena,
@@ -117,13 +106,17 @@ int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const str
                           ? packed->buf
                           : nullptr;
   const size_t pb = strata_q4_gemm_mfma_part_bytes(M, K, fast, nfast);
-  const size_t pk = pk_in ? 0 : (strata_q4_gemm_mfma_scratch(Nfast, K) + 255) / 256 * 256;
+  // Up to kMlxMaxRows rows the kernel reads the linears' own tensors instead
+  // (the same bits): the re-layout takes as long as the GEMM gains (8B gate/up:
+  // 128 rows 77 -> 53 us, 512 rows 139 -> 138, 1000 rows 243 against 267).
+  const bool mlx = !pk_in && M <= kMlxMaxRows && strata_q4_gemm_mlx_fits(K, fast, nfast);
+  const size_t pk = pk_in || mlx ? 0 : (strata_q4_gemm_mfma_scratch(Nfast, K) + 255) / 256 * 256;
   void* scr = nullptr;
   if (pk + pb > 0) {
     const int rc = strata_ctx_scratch(ctx, pk + pb, &scr, stream);
     if (rc) return rc;
   }
-  if (!pk_in) {
+  if (!pk_in && !mlx) {
     const int rc = strata_q4_gemm_pack(fast, nfast, K, scr, stream);
     if (rc) return rc;
     pk_in = scr;

@@ -1,4 +1,4 @@
-// q4 linear for a few rows (9 <= M < 40 on the default path, up to 64): Y[M, N] =
+// q4 linear for a few rows (9 <= M <= 32, narrow linears up to 64): Y[M, N] =
 // X[M, K] @ dequant(W)[N, K]^T on bf16 16x16x32 MFMAs, every weight read once.
 //
 // Same maths as mx.quantized_matmul(transpose=True) (src/ollm/llama_mlx.py:
@@ -12,24 +12,24 @@
 // workgroups streaming their weight rows in parallel.
 //   * Workgroup = 4 waves on the same NC x 16 columns; wave w reduces the K
 //     quarter w, and the four partial sums meet in LDS at the end.
-//   * Per 128-k chunk a lane loads, for each of its NC columns (row
-//     n0 + 16 c + lane % 16), the 16-byte code run of k 32 (lane / 16) .. +32
-//     with that group's scale and bias, and for each of its MB x row blocks
-//     (row 16 mb + lane % 16) the 32 x values of the same k.  Word j of the
-//     run is the B operand of MFMA k-step j: lane (c, g) supplies k slots
-//     8 g .. 8 g + 7 of each 32-k step from k 32 g + 8 j .. +8, and its A
-//     operand (x) uses the same k, so the dot products are unchanged.
-//   * The next NB - 1 chunks' loads are issued before the current chunk's
-//     math (NB register sets).
+//   * Per 128-k chunk lane (c, g) needs, of each of its NC columns (row n0 +
+//     16 cc + c), the 16-byte code run of k 32 g .. +32 with that group's scale
+//     and bias, and of each of its MB x row blocks (row 16 mb + c) the 32 x
+//     values of the same k.  Word j of the run is the B operand of MFMA k-step
+//     j: the lane supplies k slots 8 g .. +7 of each 32-k step from k 32 g + 8 j
+//     .. +8, and its A operand (x) uses the same k, so the dot products are
+//     unchanged.
+//   * All of it reaches LDS by direct global -> LDS loads into a ring private
+//     to the wave (NST stages, no barrier), four x rows of 256 bytes or 16
+//     weight rows of 64 bytes per instruction.  Loaded straight into
+//     registers, an x instruction touched 32 cache lines (64-byte strides) and
+//     those were most of the time (24 rows: 3B down, 3072 x 8192, 20.7 -> 11.9
+//     us; 8B down 34.3 -> 20.2, q/k/v 21.1 -> 12.7, gate/up 49.8 -> 36.3).
+//     16-byte slots are XOR-swizzled so that the operand reads of 16 lanes meet
+//     16 distinct slots of the 64 banks.
 //   * Outputs: lane (c, g) of the 16x16 accumulator holds column c and rows
 //     4 g .. 4 g + 3.
-#include <type_traits>
-
 #include "strata_internal.h"
-
-#ifndef SKINNY_NB
-#define SKINNY_NB 3
-#endif
 
 namespace {
 
@@ -69,10 +69,20 @@ __device__ __forceinline__ uint4 dequant8(uint32_t w, float s, float b) {
   return o;
 }
 
-template <int MB, int NC, int NB, typename YT>
+template <int MB, int NC>
+struct SkinnyStage {
+  static constexpr int kX = MB * 16 * 256, kW = NC * 16 * 64, kSB = NC * 2 * 256;
+  static constexpr int kBytes = kX + kW + kSB;
+  static constexpr int kLoads = MB * 4 + NC * 3;  // per lane and chunk
+};
+
+template <int MB, int NC, int NST, typename YT>
 __global__ __launch_bounds__(256) void q4_gemm_skinny_kernel(const uint16_t* __restrict__ x, int M,
                                                              int K, SkinnyBatch bt) {
-  __shared__ f32x4_t red[3][MB * NC][64];
+  using S = SkinnyStage<MB, NC>;
+  constexpr int RING = NST * S::kBytes;
+  static_assert(MB * NC * 64 * 16 <= RING, "a wave's ring holds its partial sums");
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds_all[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, kq = lane >> 4;
@@ -83,45 +93,33 @@ __global__ __launch_bounds__(256) void q4_gemm_skinny_kernel(const uint16_t* __r
     if (t < bt.count && col0 >= bt.p[t].col0) p = t;
   const SkinnyProblem& P = bt.p[p];
   const int n0 = col0 - P.col0;
-  const int nv = K >> 5, ng = K >> 6;
   const int kw = K >> 2, kbeg = wave * kw, nch = kw >> 7;
-
-  const uint4* wr[NC];
-  const uint16_t* sr[NC];
-  const uint16_t* br[NC];
+  const uint32_t xb = (uint32_t)K * 2, wb = (uint32_t)K / 2, sb = (uint32_t)K / 32;  // bytes per row
+  // x rows at or past M read as zero
+  const v4i32_t rx = rsrc(x, (uint32_t)M * xb);
+  const v4i32_t rw = rsrc(reinterpret_cast<const uint8_t*>(P.w) + (int64_t)n0 * wb, 16 * NC * wb);
+  const v4i32_t rs = rsrc(reinterpret_cast<const uint8_t*>(P.s) + (int64_t)n0 * sb, 16 * NC * sb);
+  const v4i32_t rb = rsrc(reinterpret_cast<const uint8_t*>(P.b) + (int64_t)n0 * sb, 16 * NC * sb);
+  uint8_t* lds = lds_all + wave * RING;
+  const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(
+      (__attribute__((address_space(3))) uint8_t*)lds);
+  // x load i fills rows 4 i .. +3: slot q of row r holds 16-byte chunk q ^ (r % 16)
+  uint32_t xv[4];
 #pragma unroll
-  for (int cc = 0; cc < NC; ++cc) {
-    const int row = n0 + 16 * cc + c;
-    wr[cc] = P.w + (int64_t)row * nv;
-    sr[cc] = P.s + (int64_t)row * ng;
-    br[cc] = P.b + (int64_t)row * ng;
-  }
-  const uint16_t* xr[MB];
-  bool live[MB];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    const int m = 16 * mb + c;
-    live[mb] = m < M;
-    xr[mb] = x + (int64_t)min(m, M - 1) * K;
-  }
-
-  uint4 wv[NB][NC], xv[NB][MB][4];
-  uint32_t sv[NB][NC], bv[NB][NC];
-  // The register set is a compile-time constant (std::integral_constant), so
-  // the sets stay in registers whatever the inliner decides.
-  auto issue = [&](auto BC, int ch) {
-    constexpr int buf = decltype(BC)::value;
-    const int kb = kbeg + (ch << 7) + 32 * kq;  // this lane's first k of the chunk
+  for (int i = 0; i < 4; ++i) xv[i] = kq * xb + ((c ^ (4 * i + kq)) << 4);
+  // a weight load fills 16 rows: slot q of row r holds piece q ^ (r / 4 % 4)
+  const uint32_t wv = (lane >> 2) * wb + (((lane & 3) ^ ((lane >> 4) & 3)) << 4);
+  const uint32_t sv = c * sb;  // the pair of groups of the chunk
+  auto issue = [&](int ch, int st) {
+    const uint32_t k = kbeg + (ch << 7), base = lds0 + st * S::kBytes;
 #pragma unroll
     for (int cc = 0; cc < NC; ++cc) {
-      wv[buf][cc] = load_nt(wr[cc] + (kb >> 5));
-      sv[buf][cc] = sr[cc][kb >> 6];
-      bv[buf][cc] = br[cc][kb >> 6];
+      dma16(base + S::kX + cc * 1024, wv, rw, 16 * cc * wb + k / 2);
+      dma4(base + S::kX + S::kW + cc * 512, sv, rs, 16 * cc * sb + k / 32);
+      dma4(base + S::kX + S::kW + cc * 512 + 256, sv, rb, 16 * cc * sb + k / 32);
     }
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) xv[buf][mb][j] = reinterpret_cast<const uint4*>(xr[mb] + kb)[j];
+    for (int i = 0; i < MB * 4; ++i) dma16(base + i * 1024, xv[i & 3], rx, 4 * i * xb + k * 2);
   };
 
   f32x4_t acc[MB][NC];
@@ -130,51 +128,50 @@ __global__ __launch_bounds__(256) void q4_gemm_skinny_kernel(const uint16_t* __r
 #pragma unroll
     for (int cc = 0; cc < NC; ++cc) acc[mb][cc] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  auto compute = [&](auto BC) {
-    constexpr int buf = decltype(BC)::value;
+  for (int s = 0; s < NST - 1; ++s) issue(min(s, nch - 1), s);
+  int st = 0;
+  for (int ch = 0; ch < nch; ++ch) {
+    // The stage read last is refilled (past the end with the last chunk again,
+    // which nothing reads): its LDS reads are done first.
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    issue(min(ch + NST - 1, nch - 1), st == 0 ? NST - 1 : st - 1);
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NST - 1) * S::kLoads) : "memory");
+    const uint8_t* sg = lds + st * S::kBytes;
+    uint4 xr[MB][4], wr[NC];
+    uint32_t sr[NC], br[NC];
 #pragma unroll
     for (int cc = 0; cc < NC; ++cc) {
-      const float s = __uint_as_float(sv[buf][cc] << 16), b = __uint_as_float(bv[buf][cc] << 16);
-      const uint32_t ww[4] = {wv[buf][cc].x, wv[buf][cc].y, wv[buf][cc].z, wv[buf][cc].w};
+      wr[cc] = *reinterpret_cast<const uint4*>(sg + S::kX + cc * 1024 + c * 64 + ((kq ^ (c >> 2)) << 4));
+      sr[cc] = *reinterpret_cast<const uint32_t*>(sg + S::kX + S::kW + cc * 512 + lane * 4);
+      br[cc] = *reinterpret_cast<const uint32_t*>(sg + S::kX + S::kW + cc * 512 + 256 + lane * 4);
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        xr[mb][j] = *reinterpret_cast<const uint4*>(sg + (16 * mb + c) * 256 + (((4 * kq + j) ^ c) << 4));
+#pragma unroll
+    for (int cc = 0; cc < NC; ++cc) {
+      // the lane's group is the pair's first (kq < 2) or second
+      const float s = __uint_as_float(kq < 2 ? sr[cc] << 16 : sr[cc] & 0xffff0000u);
+      const float b = __uint_as_float(kq < 2 ? br[cc] << 16 : br[cc] & 0xffff0000u);
+      const uint32_t ww[4] = {wr[cc].x, wr[cc].y, wr[cc].z, wr[cc].w};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint4 bw = dequant8(ww[j], s, b);
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-          const uint4 a = live[mb] ? xv[buf][mb][j] : make_uint4(0, 0, 0, 0);
-          acc[mb][cc] = mfma16x32(a, bw, acc[mb][cc]);
-        }
+        for (int mb = 0; mb < MB; ++mb) acc[mb][cc] = mfma16x32(xr[mb][j], bw, acc[mb][cc]);
       }
     }
-  };
-
-  // NB register sets: chunks ch + 1 .. ch + NB - 1 are in flight while
-  // chunk ch is computed (set indices are compile-time constants)
-  issue(std::integral_constant<int, 0>{}, 0);
-  if constexpr (NB > 2)
-    if (1 < nch) issue(std::integral_constant<int, 1>{}, 1);
-  if constexpr (NB > 3)
-    if (2 < nch) issue(std::integral_constant<int, 2>{}, 2);
-  auto step = [&](int ch, auto BC) {
-    constexpr int BUF = decltype(BC)::value;
-    if (ch + NB - 1 < nch) issue(std::integral_constant<int, (BUF + NB - 1) % NB>{}, ch + NB - 1);
-    compute(BC);
-  };
-  for (int ch = 0; ch < nch; ch += NB) {
-    step(ch, std::integral_constant<int, 0>{});
-    if (ch + 1 < nch) step(ch + 1, std::integral_constant<int, 1 % NB>{});
-    if constexpr (NB > 2)
-      if (ch + 2 < nch) step(ch + 2, std::integral_constant<int, 2 % NB>{});
-    if constexpr (NB > 3)
-      if (ch + 3 < nch) step(ch + 3, std::integral_constant<int, 3 % NB>{});
+    st = st == NST - 1 ? 0 : st + 1;
   }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // the ring is the wave's again
 
   // the four K quarters meet in LDS; wave 0 adds them in wave order and stores
   if (wave > 0) {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int cc = 0; cc < NC; ++cc) red[wave - 1][mb * NC + cc][lane] = acc[mb][cc];
+    for (int i = 0; i < MB * NC; ++i)
+      reinterpret_cast<f32x4_t*>(lds)[i * 64 + lane] = acc[i / NC][i % NC];
   }
   __syncthreads();
   if (wave != 0) return;
@@ -185,7 +182,8 @@ __global__ __launch_bounds__(256) void q4_gemm_skinny_kernel(const uint16_t* __r
     for (int cc = 0; cc < NC; ++cc) {
       f32x4_t v = acc[mb][cc];
 #pragma unroll
-      for (int w = 0; w < 3; ++w) v += red[w][mb * NC + cc][lane];
+      for (int w = 1; w < 4; ++w)
+        v += reinterpret_cast<const f32x4_t*>(lds_all + w * RING)[(mb * NC + cc) * 64 + lane];
       const int n = n0 + 16 * cc + c;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -195,17 +193,26 @@ __global__ __launch_bounds__(256) void q4_gemm_skinny_kernel(const uint16_t* __r
     }
 }
 
+template <int MB, int NC, int NST, typename YT>
+void launch_skinny_t(const uint16_t* x, int M, int K, const SkinnyBatch& bt, int cols,
+                     hipStream_t stream) {
+  constexpr int lds = 4 * NST * SkinnyStage<MB, NC>::kBytes;
+  static bool attr = false;
+  if (!attr) {
+    (void)hipFuncSetAttribute((const void*)q4_gemm_skinny_kernel<MB, NC, NST, YT>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    attr = true;
+  }
+  hipLaunchKernelGGL((q4_gemm_skinny_kernel<MB, NC, NST, YT>), dim3(cols / (16 * NC)), dim3(256), lds,
+                     stream, x, M, K, bt);
+}
+// Two stages: a third costs workgroups per CU (8B gate/up, 9 rows: 29 us
+// against 33, down 24 rows 20 against 23).
 template <int MB, int NC>
 void launch_skinny(const uint16_t* x, int M, int K, const SkinnyBatch& bt, int cols, int y_dtype,
                    hipStream_t stream) {
-  constexpr int NB = SKINNY_NB;
-  const dim3 grid(cols / (16 * NC));
-  if (y_dtype == STRATA_BF16)
-    hipLaunchKernelGGL((q4_gemm_skinny_kernel<MB, NC, NB, bf16_t>), grid, dim3(256), 0, stream, x,
-                       M, K, bt);
-  else
-    hipLaunchKernelGGL((q4_gemm_skinny_kernel<MB, NC, NB, float>), grid, dim3(256), 0, stream, x,
-                       M, K, bt);
+  if (y_dtype == STRATA_BF16) launch_skinny_t<MB, NC, 2, bf16_t>(x, M, K, bt, cols, stream);
+  else launch_skinny_t<MB, NC, 2, float>(x, M, K, bt, cols, stream);
 }
 
 }  // namespace
@@ -214,7 +221,9 @@ bool strata_q4_skinny_fits(int M, int K, const strata_q4_weight* ws, int count) 
   if (M < 1 || M > kSkinnyMaxRows || K % 512 != 0 || count < 1 || count > kMaxGemmProblems)
     return false;
   for (int i = 0; i < count; ++i)
-    if (ws[i].N % 16 != 0 || !aligned16(ws[i].w)) return false;
+    if (ws[i].N % 16 != 0 || !aligned16(ws[i].w) ||
+        ((reinterpret_cast<uintptr_t>(ws[i].scales) | reinterpret_cast<uintptr_t>(ws[i].biases)) & 3))
+      return false;
   return true;
 }
 

@@ -83,21 +83,28 @@ int strata_q4_gemm_mfma_launch(const void* x, int M, int K, const strata_q4_weig
                                int y_dtype, void* scratch, void* stream);
 // The same in two parts: the weights' re-layout into `packed`
 // (strata_q4_gemm_mfma_scratch(sum of N, K) bytes, 16-byte aligned; done
-// once at load time by the decoder), then GEMMs on it (the ws' w, scales and
-// biases are not read, only N and y).
+// once at load time by the decoder), then GEMMs on it (with `packed` the ws' w,
+// scales and biases are not read, only N and y).
 int strata_q4_gemm_pack(const strata_q4_weight* ws, int count, int K, void* packed, void* stream);
 // Any M.  With `part` (fp32 scratch of part_bytes), linears whose tiles
 // leave CUs idle split K over several workgroups and add the slices up in
 // order (strata_q4_gemm_mfma_part_bytes sizes it); without it, no split.
+// packed == nullptr: the ws' own tensors are read (strata_q4_gemm_mlx_fits).
+bool strata_q4_gemm_mlx_fits(int K, const strata_q4_weight* ws, int count);
 int strata_q4_gemm_mfma_run(const void* x, int M, int K, const void* packed,
                             const strata_q4_weight* ws, int count, int y_dtype, void* stream,
                             float* part = nullptr, size_t part_bytes = 0);
 size_t strata_q4_gemm_mfma_part_bytes(int M, int K, const strata_q4_weight* ws, int count);
-// From this many rows the linears sharing x go to the 256-column MFMA kernel
-// when every N is a multiple of 256 (STRATA_GEMM_MFMA_MIN_M overrides).
-// (Measured on the 8B shapes: the skinny kernel is faster up to ~32 rows,
-// this one from ~48.)
-constexpr int kMfmaMidRows = 40;
+// From this many rows a linear of at least kMidWideN columns (a multiple of
+// 256) goes to the 256-column MFMA kernel; narrower ones from one row past
+// the skinny kernel's 64.  Skinny against MFMA kernel: 8B gate/up at 32 rows 36
+// against 42 us, at 39 rows 60 against 42; 3B gate/up 17.6 against 25 and 30
+// against 25.5; at 64 rows q/k/v 20.4 against 22.3 (8B) and 17.1 against 20.3
+// (3B), down 30.9 against 30.7 and 17.5 against 24.7.
+constexpr int kMfmaMidRows = 33;
+constexpr int kMidWideN = 8192;
+// Rows up to which a call without a load-time re-layout reads the MLX tensors.
+constexpr int kMlxMaxRows = 512;
 // Prefill linears sharing x (M > 8 rows, bf16 x): one launch where the
 // shapes allow, else one per linear.
 // A load-time re-layout (strata_q4_gemm_pack) of `count` linears with N
@@ -111,7 +118,7 @@ struct GemmPacked {
 int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const strata_q4_weight* ws,
                          int count, int y_dtype, void* stream, const GemmPacked* packed = nullptr);
 // Linears sharing x for a few rows (M <= kSkinnyMaxRows, K % 512 == 0, every
-// N % 16 == 0, 16-byte aligned weights and x): one launch, each weight read once.
+// N % 16 == 0, 16-byte aligned weights and x, 4-byte aligned scales and biases): one launch, each weight read once.
 constexpr int kSkinnyMaxRows = 64;
 bool strata_q4_skinny_fits(int M, int K, const strata_q4_weight* ws, int count);
 int strata_q4_gemm_skinny(const void* x, int M, int K, const strata_q4_weight* ws, int count,

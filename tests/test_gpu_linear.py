@@ -256,3 +256,36 @@ def test_bf16_dense_linear_rows(dev, M, N, K):
     assert torch.equal(y[:3].isnan(), ref[:3].isnan())
     assert torch.equal(torch.where(y[:2].isinf(), y[:2], 0.), torch.where(ref[:2].isinf(), ref[:2], 0.))
     assert bool(y[3:].isfinite().all())
+
+
+@pytest.mark.parametrize("M,K,ns", [(9, 512, (16, 48)), (16, 3072, (16384, 64)), (17, 1024, (1040,)),
+                                    (32, 4096, (8192, 8192)), (33, 1536, (8192, 1024, 80)),
+                                    (49, 2048, (256, 8192)), (64, 512, (768, 16)),
+                                    (65, 1024, (256, 8192)), (129, 192, (512,)), (130, 128, (256,))])
+def test_gemm_rows_at_kernel_borders(dev, M, K, ns):
+    """Row counts where a linear's kernel changes (32 / 33 by width, 64 / 65),
+    16-row blocks of the skinny kernel, linears of one call on different
+    kernels, and K % 128 != 0 (the MFMA kernel's per-call re-layout).  fp32
+    sums of exact bf16 products against float64: K terms at 2^-24 each."""
+    from lokahi_amd import ops
+    rng = np.random.default_rng(M * 13 + K)
+    probs = [_problem(rng, n, K)[:3] for n in ns]
+    x = f32_to_bf16_bits(rng.normal(0, 1, (M, K)).astype(np.float32))
+    dprobs = [tuple(to_dev(a, dev) for a in p) for p in probs]
+    xd = to_dev(x, dev)
+    ys = ops.linear_multi(xd, dprobs, out_dtype=torch.float32)
+    for (w, s, b), y, dp in zip(probs, ys, dprobs):
+        wq = round_bf16(q4.dequantize(w, s, b, 64).astype(np.float32)).astype(np.float64)
+        ref = bf16_bits_to_f32(x).astype(np.float64) @ wq.T
+        assert rel_err(to_np_f32(y), ref) < 1e-5
+        assert torch.equal(ops.linear(xd, *dp, out_dtype=torch.float32), y)
+
+
+def test_gemm_layouts_agree(dev):
+    """The MFMA kernel on the linear's own tensors (up to 512 rows) and on its
+    re-laid-out copy (more rows) gives the same bits for the same rows."""
+    from lokahi_amd import ops
+    gen = torch.Generator(device=dev).manual_seed(4)
+    w = ops.quantize(torch.randn((14336, 512), generator=gen, device=dev) * 0.02)
+    x = torch.randn((513, 512), generator=gen, device=dev).bfloat16()
+    assert torch.equal(ops.linear(x, *w)[:512], ops.linear(x[:512], *w))
