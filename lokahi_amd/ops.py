@@ -15,6 +15,7 @@ Each function mirrors the reference operation it replaces:
 from __future__ import annotations
 
 import ctypes as C
+import struct
 from typing import Optional, Sequence, Tuple
 
 import torch
@@ -25,6 +26,14 @@ from ._abi import BF16, F32, check
 _DT = {torch.float32: F32, torch.bfloat16: BF16}
 
 
+# Every call below runs a few microseconds of kernels, so its host side counts:
+# raw stream handles, outputs allocated in their final shape and C structs
+# packed by struct.Struct (a ctypes array of Structures takes 3 us for two
+# weights) instead of the objects around them.
+_raw_stream = torch._C._cuda_getCurrentRawStream
+_Q4 = {n: struct.Struct("PPPqP" * n) for n in range(1, 9)}  # strata_q4_weight[n]
+
+
 def _code(t: torch.Tensor) -> int:
     try:
         return _DT[t.dtype]
@@ -33,13 +42,13 @@ def _code(t: torch.Tensor) -> int:
 
 
 def _dev(t: torch.Tensor) -> int:
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError("tensors must live on the HIP device (torch 'cuda' device)")
-    return t.device.index or 0
+    return t.get_device()
 
 
-def _stream(device: int) -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream(device: int) -> int:
+    return _raw_stream(device)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -47,11 +56,18 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _ctx(device: int):
-    return _abi.context(device).handle
+    c = _abi._contexts.get(device)
+    return (c if c is not None else _abi.context(device)).handle
 
 
 def _lib():
-    return _abi.load()
+    return _abi._lib or _abi.load()
+
+
+def _rows(x: torch.Tensor, K: int):
+    """(contiguous x, rows of K elements)."""
+    x = x.contiguous()
+    return x, x.numel() // K if K else x.reshape(-1, K).shape[0]
 
 
 # ----------------------------------------------------------------- linear
@@ -63,27 +79,26 @@ def linear(x: torch.Tensor, weight: torch.Tensor, scales: Optional[torch.Tensor]
     dev = _dev(x)
     if mode != "affine":
         raise ValueError(f"unsupported quantization mode {mode!r}")
-    lead = x.shape[:-1]
-    K = x.shape[-1]
-    x2 = x.reshape(-1, K).contiguous()
-    M = x2.shape[0]
-    out_dtype = out_dtype or x.dtype
+    shape = x.shape
+    K = shape[-1]
+    x2, M = _rows(x, K)
+    N = weight.shape[0]
     if scales is None:
-        N = weight.shape[0]
         if weight.dtype != torch.bfloat16 or weight.shape[1] != K:
             raise ValueError("dense weight must be bf16 [N, K]")
-        y = torch.empty((M, N), dtype=out_dtype, device=x.device)
-        check(_lib().strata_linear_bf16(_ctx(dev), x2.data_ptr(), _code(x2), M, K,
-                                        weight.contiguous().data_ptr(), N, y.data_ptr(),
-                                        _code(y), _stream(dev)))
-        return y.reshape(*lead, N)
-    N = weight.shape[0]
-    _check_q4(weight, scales, biases, N, K, group_size, bits)
-    y = torch.empty((M, N), dtype=out_dtype, device=x.device)
-    check(_lib().strata_linear_q4(_ctx(dev), x2.data_ptr(), _code(x2), M, K, weight.data_ptr(),
-                                  scales.data_ptr(), biases.data_ptr(), N, int(group_size),
-                                  int(bits), y.data_ptr(), _code(y), _stream(dev)))
-    return y.reshape(*lead, N)
+        w = weight.contiguous()  # held until the launch
+        y = x.new_empty((*shape[:-1], N), dtype=out_dtype)
+        rc = _lib().strata_linear_bf16(_ctx(dev), x2.data_ptr(), _code(x2), M, K, w.data_ptr(), N,
+                                       y.data_ptr(), _code(y), _raw_stream(dev))
+    else:
+        _check_q4(weight, scales, biases, N, K, group_size, bits)
+        y = x.new_empty((*shape[:-1], N), dtype=out_dtype)
+        rc = _lib().strata_linear_q4(_ctx(dev), x2.data_ptr(), _code(x2), M, K, weight.data_ptr(),
+                                     scales.data_ptr(), biases.data_ptr(), N, int(group_size),
+                                     int(bits), y.data_ptr(), _code(y), _raw_stream(dev))
+    if rc:
+        check(rc)
+    return y
 
 
 def _check_q4(w, s, b, N, K, group_size, bits):
@@ -91,11 +106,12 @@ def _check_q4(w, s, b, N, K, group_size, bits):
         raise ValueError(f"only 4-bit quantization is supported (got bits={bits})")
     if group_size is None or K % group_size:
         raise ValueError(f"K={K} must be divisible by group_size={group_size}")
-    if w.dtype not in (torch.uint32, torch.int32) or tuple(w.shape) != (N, K // 8):
+    if w.dtype not in (torch.uint32, torch.int32) or w.shape != (N, K // 8):
         raise ValueError(f"packed weight must be uint32 [N, K/8] = [{N}, {K // 8}], "
                          f"got {w.dtype} {tuple(w.shape)}")
+    groups = (N, K // group_size)
     for name, t in (("scales", s), ("biases", b)):
-        if t is None or t.dtype != torch.bfloat16 or tuple(t.shape) != (N, K // group_size):
+        if t is None or t.dtype != torch.bfloat16 or t.shape != groups:
             raise ValueError(f"{name} must be bf16 [N, K/group_size]")
     if not (w.is_contiguous() and s.is_contiguous() and b.is_contiguous()):
         raise ValueError("quantized weight tensors must be contiguous")
@@ -107,23 +123,25 @@ def linear_multi(x: torch.Tensor, weights: Sequence[Tuple[torch.Tensor, torch.Te
                  out_dtype: Optional[torch.dtype] = None):
     """Several q4 linears sharing ``x`` in one launch; returns the outputs."""
     dev = _dev(x)
-    K = x.shape[-1]
-    lead = x.shape[:-1]
-    x2 = x.reshape(-1, K).contiguous()
-    M = x2.shape[0]
-    out_dtype = out_dtype or x.dtype
-    arr = (_abi.Q4Weight * len(weights))()
-    ys = []
+    shape = x.shape
+    K = shape[-1]
+    lead = shape[:-1]
+    x2, M = _rows(x, K)
+    ys, args = [], []
     for i, (w, s, b) in enumerate(weights):
         N = w.shape[0]
         _check_q4(w, s, b, N, K, group_size, bits)
-        y = outs[i] if outs is not None else torch.empty((M, N), dtype=out_dtype, device=x.device)
+        y = outs[i] if outs is not None else x.new_empty((*lead, N), dtype=out_dtype)
         ys.append(y)
-        arr[i] = _abi.Q4Weight(w.data_ptr(), s.data_ptr(), b.data_ptr(), N, y.data_ptr())
-    check(_lib().strata_linear_q4_multi(_ctx(dev), x2.data_ptr(), _code(x2), M, K, arr,
-                                        len(weights), group_size, bits, _code(ys[0]),
-                                        _stream(dev)))
-    return [y.reshape(*lead, y.shape[-1]) for y in ys]
+        args += (w.data_ptr(), s.data_ptr(), b.data_ptr(), N, y.data_ptr())
+    pack = _Q4.get(len(ys))
+    if pack is None:  # none or more than 8: refused by the library
+        pack = struct.Struct("PPPqP" * len(ys))
+    rc = _lib().strata_linear_q4_multi(_ctx(dev), x2.data_ptr(), _code(x2), M, K, pack.pack(*args),
+                                       len(ys), group_size, bits, _code(ys[0]), _raw_stream(dev))
+    if rc:
+        check(rc)
+    return ys if outs is None else [y.reshape(*lead, y.shape[-1]) for y in ys]
 
 
 class Q4Layout:
@@ -151,6 +169,7 @@ class Q4Layout:
         h = C.c_void_p()
         check(_lib().strata_q4_layout_create(_ctx(self.device), arr, len(weights), K, C.byref(h)))
         self._h = h
+        self._ptrs = struct.Struct("P" * len(self.N))
 
     def __call__(self, x: torch.Tensor, *, outs: Optional[Sequence[torch.Tensor]] = None,
                  out_dtype: Optional[torch.dtype] = None):
@@ -159,15 +178,19 @@ class Q4Layout:
         if x.dtype != torch.bfloat16 or x.shape[-1] != self.K:
             raise ValueError(f"x must be bf16 [..., {self.K}]")
         lead = x.shape[:-1]
-        x2 = x.reshape(-1, self.K).contiguous()
-        M = x2.shape[0]
-        out_dtype = out_dtype or torch.bfloat16
-        ys = list(outs) if outs is not None else [
-            torch.empty((M, n), dtype=out_dtype, device=x.device) for n in self.N]
-        ptrs = (C.c_void_p * len(ys))(*[y.data_ptr() for y in ys])
-        check(_lib().strata_linear_q4_layout(_ctx(self.device), x2.data_ptr(), BF16, M, self._h,
-                                             ptrs, _code(ys[0]), _stream(self.device)))
-        return [y.reshape(*lead, y.shape[-1]) for y in ys]
+        x2, M = _rows(x, self.K)
+        if outs is not None:
+            ys = list(outs)
+        else:
+            out_dtype = out_dtype or torch.bfloat16
+            ys = [x.new_empty((*lead, n), dtype=out_dtype) for n in self.N]
+        ptrs = [y.data_ptr() for y in ys]
+        pack = self._ptrs if len(ptrs) == len(self.N) else struct.Struct("P" * len(ptrs))
+        rc = _lib().strata_linear_q4_layout(_ctx(self.device), x2.data_ptr(), BF16, M, self._h,
+                                            pack.pack(*ptrs), _code(ys[0]), _raw_stream(self.device))
+        if rc:
+            check(rc)
+        return ys if outs is None else [y.reshape(*lead, y.shape[-1]) for y in ys]
 
     def close(self):
         if getattr(self, "_h", None) is not None:
@@ -193,7 +216,7 @@ def quantize(weight: torch.Tensor, group_size: int = 64):
     sc = torch.empty((N, K // group_size), dtype=torch.bfloat16, device=w.device)
     bi = torch.empty_like(sc)
     check(_lib().strata_quantize_q4(_ctx(dev), w.data_ptr(), _code(w), N, K, group_size,
-                                    packed.data_ptr(), sc.data_ptr(), bi.data_ptr(), _stream(dev)))
+                                    packed.data_ptr(), sc.data_ptr(), bi.data_ptr(), _raw_stream(dev)))
     return packed, sc, bi
 
 
@@ -207,7 +230,7 @@ def dequantize(weight: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
     out = torch.empty((N, K), dtype=torch.bfloat16, device=weight.device)
     check(_lib().strata_dequantize_q4(_ctx(dev), weight.data_ptr(), scales.data_ptr(),
                                       biases.data_ptr(), N, K, group_size, bits, out.data_ptr(),
-                                      _stream(dev)))
+                                      _raw_stream(dev)))
     return out
 
 
@@ -228,13 +251,15 @@ def rope(q: Optional[torch.Tensor], k: Optional[torch.Tensor], position_ids: tor
     check(_lib().strata_rope(_ctx(dev), _ptr(q), _ptr(k), pos.data_ptr(), B,
                              q.shape[1] if q is not None else 0,
                              k.shape[1] if k is not None else 0, L, D, float(theta),
-                             _code(ref), _stream(dev)))
+                             _code(ref), _raw_stream(dev)))
 
 
 # --------------------------------------------------------------- attention
 def _normalize_query_positions(query_positions, batch: int, lq: int, device) -> torch.Tensor:
     """``_normalize_query_positions`` (mlx_ops.py:17-29)."""
     pos = torch.as_tensor(query_positions, dtype=torch.int32, device=device)
+    if batch == 1 and pos.ndim == 1 and pos.shape[0] == lq:
+        return pos.contiguous()
     if pos.ndim == 1:
         pos = pos[None, :]
     if tuple(pos.shape) == (1, lq) and batch > 1:
@@ -258,14 +283,15 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if q_block_size <= 0 or k_block_size <= 0:
         raise ValueError("attention block sizes must be positive")
     B, Hq, Lq, D = q.shape
-    _, Hkv, Lk, Dk = k.shape
+    Bk, Hkv, Lk, Dk = k.shape
+    Bv, Hv, Lv, Dv = v.shape
     if D != Dk:
         raise ValueError("q and k must share last-dim size")
-    if k.shape[0] != B or v.shape[0] != B:
+    if Bk != B or Bv != B:
         raise ValueError("q, k, and v must share batch size")
-    if v.shape[1] != Hkv or v.shape[2] != Lk:
+    if Hv != Hkv or Lv != Lk:
         raise ValueError("k and v must share head and sequence dimensions")
-    if v.shape[3] != D:
+    if Dv != D:
         raise ValueError("q, k, and v must share last-dim size")
     if Hkv <= 0 or Hq % Hkv != 0:
         raise ValueError("query heads must be divisible by key/value heads")
@@ -282,16 +308,20 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         bs, hs = Hkv * Lk * D, Lk * D
     else:
         bs, hs = kv_strides
-        if k.stride() != v.stride() or k.stride()[2:] != (D, 1) or (k.stride(0), k.stride(1)) != (bs, hs):
+        st = k.stride()
+        if st != v.stride() or st[2:] != (D, 1) or st[0] != bs or st[1] != hs:
             raise ValueError("k/v views do not match the given kv_strides")
     if out is None:
-        out = torch.empty((B, Hq, Lq, D), dtype=q.dtype, device=q.device)
+        out = q.new_empty((B, Hq, Lq, D))
     ws = _attention_workspace(dev, q, k, v, causal) if Lq > 1 else None
-    check(_lib().strata_attn_gqa_ws(_ctx(dev), q.data_ptr(), _code(q), k.data_ptr(), _code(k),
-                                    v.data_ptr(), _code(v), bs, hs, _ptr(qpos), B, Hq, Hkv, Lq, Lk,
-                                    D, 1 if causal else 0, int(min(q_block_size, 2**31 - 1)),
-                                    int(min(k_block_size, 2**31 - 1)), float(eps), out.data_ptr(),
-                                    _ptr(ws), 0 if ws is None else ws.numel(), _stream(dev)))
+    rc = _lib().strata_attn_gqa_ws(
+        _ctx(dev), q.data_ptr(), _code(q), k.data_ptr(), _code(k), v.data_ptr(), _code(v), bs, hs,
+        None if qpos is None else qpos.data_ptr(), B, Hq, Hkv, Lq, Lk, D, 1 if causal else 0,
+        q_block_size if q_block_size <= 2**31 - 1 else 2**31 - 1,
+        k_block_size if k_block_size <= 2**31 - 1 else 2**31 - 1, eps, out.data_ptr(),
+        None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _raw_stream(dev))
+    if rc:
+        check(rc)
     return out
 
 
@@ -329,7 +359,7 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float,
     if out is None:
         out = torch.empty_like(x)
     check(_lib().strata_rmsnorm(_ctx(dev), x.data_ptr(), _ptr(residual), weight.data_ptr(), rows,
-                                H, float(eps), out.data_ptr(), _stream(dev)))
+                                H, float(eps), out.data_ptr(), _raw_stream(dev)))
     return out
 
 
@@ -338,7 +368,7 @@ def silu_mul(g: torch.Tensor, u: torch.Tensor, out: Optional[torch.Tensor] = Non
     if out is None:
         out = torch.empty_like(g)
     check(_lib().strata_silu_mul(_ctx(dev), g.data_ptr(), u.data_ptr(), g.numel(), out.data_ptr(),
-                                 _stream(dev)))
+                                 _raw_stream(dev)))
     return out
 
 
@@ -347,7 +377,7 @@ def add(x: torch.Tensor, r: torch.Tensor, out: Optional[torch.Tensor] = None):
     if out is None:
         out = torch.empty_like(x)
     check(_lib().strata_add(_ctx(dev), x.data_ptr(), r.data_ptr(), x.numel(), out.data_ptr(),
-                            _stream(dev)))
+                            _raw_stream(dev)))
     return out
 
 
@@ -358,7 +388,7 @@ def embed(table: torch.Tensor, ids: torch.Tensor, out: Optional[torch.Tensor] = 
     if out is None:
         out = torch.empty((*ids.shape, H), dtype=table.dtype, device=table.device)
     check(_lib().strata_embed(_ctx(dev), table.data_ptr(), V, H, ids32.data_ptr(), ids32.numel(),
-                              out.data_ptr(), _stream(dev)))
+                              out.data_ptr(), _raw_stream(dev)))
     return out
 
 
@@ -371,5 +401,5 @@ def argmax(logits: torch.Tensor, out: Optional[torch.Tensor] = None):
     if out is None:
         out = torch.empty(lg.shape[0], dtype=torch.int32, device=logits.device)
     check(_lib().strata_argmax(_ctx(dev), lg.data_ptr(), lg.shape[0], V, out.data_ptr(),
-                               _stream(dev)))
+                               _raw_stream(dev)))
     return out
