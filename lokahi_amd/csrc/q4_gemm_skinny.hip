@@ -76,7 +76,14 @@ struct SkinnyStage {
   static constexpr int kLoads = MB * 4 + NC * 3;  // per lane and chunk
 };
 
-template <int MB, int NC, int NST, typename YT>
+// EXACT (at most 8 rows of the decode linears, MB = 1): the weights are not
+// rounded.  Codes enter the MFMA as the exact bf16 values 128 + q (a mask and
+// an OR per pair, x permuted to the pairs' order), every 32 k sum on their own,
+// and the group's scale and bias apply to the fp32 sums: y += s sum x (128 + q)
+// + (b - 128 s) sum x, the sums of x from MFMAs against ones.  (Sums over the
+// whole group of 64 are 15% further from the exact product than the GEMV's
+// 32-element slices, these are not.)
+template <int MB, int NC, int NST, bool EXACT, typename YT>
 __global__ __launch_bounds__(256) void q4_gemm_skinny_kernel(const uint16_t* __restrict__ x, int M,
                                                              int K, SkinnyBatch bt) {
   using S = SkinnyStage<MB, NC>;
@@ -137,6 +144,45 @@ __global__ __launch_bounds__(256) void q4_gemm_skinny_kernel(const uint16_t* __r
     issue(min(ch + NST - 1, nch - 1), st == 0 ? NST - 1 : st - 1);
     asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NST - 1) * S::kLoads) : "memory");
     const uint8_t* sg = lds + st * S::kBytes;
+    if constexpr (EXACT) {
+      static_assert(MB == 1, "one block of rows");
+      const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
+      uint4 xp[4];  // k 32 s + 8 kq .. +7 in the order 0 4 1 5 2 6 3 7
+      uint32_t wd[NC][4], sr[NC], br[NC];
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc) {
+        sr[cc] = *reinterpret_cast<const uint32_t*>(sg + S::kX + S::kW + cc * 512 + lane * 4);
+        br[cc] = *reinterpret_cast<const uint32_t*>(sg + S::kX + S::kW + cc * 512 + 256 + lane * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          wd[cc][j] = *reinterpret_cast<const uint32_t*>(sg + S::kX + cc * 1024 + c * 64 +
+                                                         ((j ^ (c >> 2)) << 4) + kq * 4);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint4 v = *reinterpret_cast<const uint4*>(sg + c * 256 + (((4 * j + kq) ^ c) << 4));
+        xp[j] = make_uint4(__builtin_amdgcn_perm(v.z, v.x, 0x05040100), __builtin_amdgcn_perm(v.z, v.x, 0x07060302),
+                           __builtin_amdgcn_perm(v.w, v.y, 0x05040100), __builtin_amdgcn_perm(v.w, v.y, 0x07060302));
+      }
+      const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4_t xs = mfma16x32(xp[j], ones, zero);
+#pragma unroll
+        for (int cc = 0; cc < NC; ++cc) {
+          const uint32_t w = wd[cc][j];
+          const f32x4_t d =
+              mfma16x32(xp[j], make_uint4((w & 0x000f000fu) | 0x43004300u, ((w >> 4) & 0x000f000fu) | 0x43004300u,
+                                          ((w >> 8) & 0x000f000fu) | 0x43004300u,
+                                          ((w >> 12) & 0x000f000fu) | 0x43004300u), zero);
+          const float s = __uint_as_float(j >= 2 ? sr[cc] & 0xffff0000u : sr[cc] << 16);
+          const float b = __uint_as_float(j >= 2 ? br[cc] & 0xffff0000u : br[cc] << 16);
+          const float cb = fmaf(-128.f, s, b);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[0][cc][r] = fmaf(cb, xs[r], fmaf(s, d[r], acc[0][cc][r]));
+        }
+      }
+    } else {
     uint4 xr[MB][4], wr[NC];
     uint32_t sr[NC], br[NC];
 #pragma unroll
@@ -162,6 +208,7 @@ __global__ __launch_bounds__(256) void q4_gemm_skinny_kernel(const uint16_t* __r
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) acc[mb][cc] = mfma16x32(xr[mb][j], bw, acc[mb][cc]);
       }
+    }
     }
     st = st == NST - 1 ? 0 : st + 1;
   }
@@ -193,17 +240,17 @@ __global__ __launch_bounds__(256) void q4_gemm_skinny_kernel(const uint16_t* __r
     }
 }
 
-template <int MB, int NC, int NST, typename YT>
+template <int MB, int NC, int NST, bool EXACT, typename YT>
 void launch_skinny_t(const uint16_t* x, int M, int K, const SkinnyBatch& bt, int cols,
                      hipStream_t stream) {
   constexpr int lds = 4 * NST * SkinnyStage<MB, NC>::kBytes;
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute((const void*)q4_gemm_skinny_kernel<MB, NC, NST, YT>,
+    (void)hipFuncSetAttribute((const void*)q4_gemm_skinny_kernel<MB, NC, NST, EXACT, YT>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     attr = true;
   }
-  hipLaunchKernelGGL((q4_gemm_skinny_kernel<MB, NC, NST, YT>), dim3(cols / (16 * NC)), dim3(256), lds,
+  hipLaunchKernelGGL((q4_gemm_skinny_kernel<MB, NC, NST, EXACT, YT>), dim3(cols / (16 * NC)), dim3(256), lds,
                      stream, x, M, K, bt);
 }
 // Two stages: a third costs workgroups per CU (8B gate/up, 9 rows: 29 us
@@ -211,8 +258,8 @@ void launch_skinny_t(const uint16_t* x, int M, int K, const SkinnyBatch& bt, int
 template <int MB, int NC>
 void launch_skinny(const uint16_t* x, int M, int K, const SkinnyBatch& bt, int cols, int y_dtype,
                    hipStream_t stream) {
-  if (y_dtype == STRATA_BF16) launch_skinny_t<MB, NC, 2, bf16_t>(x, M, K, bt, cols, stream);
-  else launch_skinny_t<MB, NC, 2, float>(x, M, K, bt, cols, stream);
+  if (y_dtype == STRATA_BF16) launch_skinny_t<MB, NC, 2, false, bf16_t>(x, M, K, bt, cols, stream);
+  else launch_skinny_t<MB, NC, 2, false, float>(x, M, K, bt, cols, stream);
 }
 
 }  // namespace
@@ -228,7 +275,7 @@ bool strata_q4_skinny_fits(int M, int K, const strata_q4_weight* ws, int count) 
 }
 
 int strata_q4_gemm_skinny(const void* x, int M, int K, const strata_q4_weight* ws, int count,
-                          int y_dtype, void* stream) {
+                          int y_dtype, void* stream, bool exact) {
   STRATA_REQUIRE(strata_q4_skinny_fits(M, K, ws, count),
                  "q4 skinny GEMM: needs 1 <= M <= %d, K %% 512 == 0, N %% 16 == 0", kSkinnyMaxRows);
   STRATA_REQUIRE(aligned16(x), "q4 skinny GEMM: x must be 16-byte aligned");
@@ -244,6 +291,19 @@ int strata_q4_gemm_skinny(const void* x, int M, int K, const strata_q4_weight* w
   }
   hipStream_t s = as_stream(stream);
   const uint16_t* xx = static_cast<const uint16_t*>(x);
+  if (exact) {
+    STRATA_REQUIRE(M <= 16, "q4 skinny GEMM: at most 16 rows without rounding");
+    const bool bf = y_dtype == STRATA_BF16;
+    if (n64 && cols >= 16384) {
+      if (bf) launch_skinny_t<1, 4, 2, true, bf16_t>(xx, M, K, bt, cols, s);
+      else launch_skinny_t<1, 4, 2, true, float>(xx, M, K, bt, cols, s);
+    } else {
+      if (bf) launch_skinny_t<1, 1, 2, true, bf16_t>(xx, M, K, bt, cols, s);
+      else launch_skinny_t<1, 1, 2, true, float>(xx, M, K, bt, cols, s);
+    }
+    STRATA_HIP_CHECK(hipGetLastError());
+    return STRATA_OK;
+  }
   // 64-column workgroups (4 column blocks share each x fragment) when that
   // still gives >= 256 workgroups, else 16-column workgroups; x row blocks of
   // 16 per wave up to 2 (64 columns) or 4 (16 columns) within the registers.

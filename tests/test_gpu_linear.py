@@ -289,3 +289,24 @@ def test_gemm_layouts_agree(dev):
     w = ops.quantize(torch.randn((14336, 512), generator=gen, device=dev) * 0.02)
     x = torch.randn((513, 512), generator=gen, device=dev).bfloat16()
     assert torch.equal(ops.linear(x, *w)[:512], ops.linear(x[:512], *w))
+
+
+@pytest.mark.parametrize("M,K,ns", [(3, 512, (16,)), (4, 1024, (1024, 48)), (5, 4096, (4096, 1024)),
+                                    (7, 3072, (16384, 64)), (8, 14336, (64,)), (4, 4096, (256,)),
+                                    (8, 448, (100,))])
+def test_few_rows_keep_fp32_weights(dev, M, K, ns):
+    """3-8 rows on the matrix cores (K % 512 == 0, N % 16 == 0) and the GEMV's
+    shapes beside them: the weights' fp32 values, not their bf16 rounding.
+    Codes enter as 128 + q, so sums of 32 terms carry 2^-24 of about 128 / 8
+    times the result's size: below 1e-5 of the largest output, which bf16
+    weights (2^-9 each) miss a hundredfold."""
+    from lokahi_amd import ops
+    rng = np.random.default_rng(M * 17 + K)
+    probs = [_problem(rng, n, K)[:3] for n in ns]
+    x = f32_to_bf16_bits(rng.normal(0, 1, (M, K)).astype(np.float32))
+    dprobs = [tuple(to_dev(a, dev) for a in p) for p in probs]
+    xd = to_dev(x, dev)
+    for (w, s, b), y, dp in zip(probs, ops.linear_multi(xd, dprobs, out_dtype=torch.float32), dprobs):
+        ref = bf16_bits_to_f32(x).astype(np.float64) @ q4.dequantize(w, s, b, 64).astype(np.float64).T
+        assert rel_err(to_np_f32(y), ref) < 1e-5
+        assert torch.equal(ops.linear(xd, *dp, out_dtype=torch.float32), y)
