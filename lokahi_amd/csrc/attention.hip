@@ -462,27 +462,24 @@ void launch_decode_merge(const float* part, int nsplit, int D, int rows, float e
 // tile masks few keys).
 //
 // Workgroup wg of the prefill grid -> (tile of packed rows, b, KV head).
-// Workgroups are dealt to the 8 XCDs round-robin (wg % 8); kTileGroup
-// consecutive tiles of one (b, KV head) go to consecutive slots of one XCD
-// (their K/V tiles share its L2), groups ordered longest causal tiles first
-// (measured 1.5x on the bf16 two-block kernel at 8k causal).  Returns false
+// Workgroups are dealt to the 8 XCDs round-robin (wg % 8), longest causal
+// tiles first (measured 1.5x on the bf16 two-block kernel at 8k causal), so
+// with 8 KV heads an XCD works on one head of one b at a time, whose K/V tiles
+// stay in its L2 (groups of four consecutive tiles: 0-2% slower, 8k causal 561
+// against 555 us; a serpentine order over 32 CUs: 0-5% slower).  Returns false
 // for the padding of the grid.
 constexpr int kXcds = 8;
-constexpr int kTileGroup = 4;
 __host__ __device__ inline int prefill_grid(int nqt, int B, int Hkv) {
-  const int groups = (nqt + kTileGroup - 1) / kTileGroup * B * Hkv;
-  return (groups + kXcds - 1) / kXcds * kXcds * kTileGroup;
+  return (nqt * B * Hkv + kXcds - 1) / kXcds * kXcds;
 }
 __device__ inline bool prefill_item(int wg, int nqt, int B, int Hkv, int* qt, int* b, int* hkv) {
-  const int xcd = wg % kXcds, slot = wg / kXcds;
-  const int gi = (slot / kTileGroup) * kXcds + xcd;
-  const int ng = (nqt + kTileGroup - 1) / kTileGroup, per = B * Hkv;
-  if (gi >= ng * per) return false;
-  *qt = (ng - 1 - gi / per) * kTileGroup + kTileGroup - 1 - slot % kTileGroup;
-  const int rest = gi % per;
+  const int per = B * Hkv;
+  if (wg >= nqt * per) return false;
+  *qt = nqt - 1 - wg / per;
+  const int rest = wg % per;
   *b = rest / Hkv;
   *hkv = rest % Hkv;
-  return *qt < nqt;
+  return true;
 }
 
 // Key split of a prefill launch (gridDim.y = nsplit): split s of a tile takes
@@ -492,6 +489,7 @@ __device__ inline bool prefill_item(int wg, int nqt, int B, int Hkv, int* qt, in
 // output itself and leaves l = -1 there.
 struct PrefillSplit {
   int nsplit, chunk;
+  int rows;  // packed query rows per tile (fp32 kernel: 16, 32 or 64)
   float* o;
   float2* ms;
 };
@@ -540,8 +538,9 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
-// fp32 prefill.  Block 256; wave w owns the 16 packed query rows qt*64 + 16w
-// + 0..15.  S^T = K Q^T and O^T += V P^T on 16x16x4 fp32 MFMAs; one LDS stage
+// fp32 prefill.  Block 256; wave w owns the 16 packed query rows
+// qt*sp.rows + 16w + 0..15; with 16 or 32 rows per tile the other waves only
+// load.  S^T = K Q^T and O^T += V P^T on 16x16x4 fp32 MFMAs; one LDS stage
 // of K and V tiles (64 keys, row-major, padded rows).
 // MFMA 16x16x4 layouts (wave64): A (16 x 4): lane l holds row l%16, k l/16;
 // B (4 x 16): lane l holds column l%16, k l/16; C (16 x 16): lane l holds
@@ -561,12 +560,13 @@ __global__ __launch_bounds__(256) void attn_prefill_f32(
 
   const int G = Hq / Hkv;
   int qt, b, hkv;
-  if (!prefill_item(blockIdx.x, (Lq * G + 63) / 64, B, Hkv, &qt, &b, &hkv)) return;  // grid padding
+  const int qr = sp.rows;
+  if (!prefill_item(blockIdx.x, (Lq * G + qr - 1) / qr, B, Hkv, &qt, &b, &hkv)) return;  // padding
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, grp = lane >> 4;
-  const int pr = qt * 64 + 16 * wave + col;  // this lane's packed row
+  const int pr = qt * qr + 16 * wave + col;  // this lane's packed row
   const int row = pr / G, hq = hkv * G + (pr - row * G);
-  const bool row_ok = row < Lq;
+  const bool row_ok = 16 * wave < qr && row < Lq;
   const int qp = row_ok ? (causal ? (qpos ? qpos[(int64_t)b * Lq + row] : Lk - Lq + row) : Lk - 1)
                         : -1;
   const float* kbase = k + (int64_t)b * kv_bs + (int64_t)hkv * kv_hs;
@@ -590,11 +590,11 @@ __global__ __launch_bounds__(256) void attn_prefill_f32(
   // the first tile's loads go out before given positions are reduced
   const int split = SPLIT ? blockIdx.y : 0;
   const int kb_begin = SPLIT ? split * sp.chunk : 0;
-  const bool empty = SPLIT && !qpos && causal && kb_begin > Lk - Lq + (min(qt * 64 + 64, Lq * G) - 1) / G;
+  const bool empty = SPLIT && !qpos && causal && kb_begin > Lk - Lq + (min(qt * qr + qr, Lq * G) - 1) / G;
   if (!empty) fetch(kb_begin);
   int kfull, wave_need, kmax;
-  key_limits<16>(qpos, causal, qp, row_ok, qt * 64 + 16 * wave, qt * 64 + 64, G, Lq, Lk, &s_kmax,
-                 &kfull, &wave_need, &kmax);
+  key_limits<16>(qpos, causal, qp, row_ok, 16 * wave < qr ? qt * qr + 16 * wave : Lq * G,
+                 qt * qr + qr, G, Lq, Lk, &s_kmax, &kfull, &wave_need, &kmax);
   const int kb_end = SPLIT ? min(kmax, kb_begin + sp.chunk) : kmax;
   const int64_t rid = ((int64_t)b * Hq + hq) * Lq + row;  // output row
   if (SPLIT && kb_begin >= kmax && split > 0) {
@@ -1562,7 +1562,7 @@ int launch_decode(strata_ctx* ctx, const void* q, const void* k, const void* v, 
 // How a prefill launch covers (rows, keys): waves per workgroup, keys per LDS
 // tile and the key split.
 struct PrefillPlan {
-  int nw, ks, kt, nsplit, chunk;
+  int nw, ks, kt, nsplit, chunk, qr;
 };
 constexpr int kMaxPrefillSplits = 64;
 constexpr size_t kMaxPrefillWs = (size_t)512 << 20;  // longer splits where more would be needed
@@ -1576,8 +1576,8 @@ PrefillPlan prefill_plan(int num_cus, bool f32, int B, int Hq, int Hkv, int Lq, 
   p.nw = f32 ? 4 : (rows <= 32 ? 1 : rows <= 64 ? 2 : 4);
   p.kt = f32 ? 64 : 32;
   p.ks = 1;
-  const int qr = (f32 ? 16 : 32) * p.nw;
-  const int64_t tiles = (rows + qr - 1) / qr * B * Hkv;
+  p.qr = (f32 ? 16 : 32) * p.nw;
+  const int64_t tiles = (rows + p.qr - 1) / p.qr * B * Hkv;
   const int64_t longest = (Lk + p.kt - 1) / p.kt;  // steps of the longest tile
   const double mean = std::max(1.0, causal ? (Lk - Lq / 2.0) / p.kt : (double)longest);
   // Chunks that give every CU its share of workgroups: 3 of 4 waves (what fits
@@ -1590,32 +1590,66 @@ PrefillPlan prefill_plan(int num_cus, bool f32, int B, int Hq, int Hkv, int Lq, 
   // Without a split, two wave groups of a workgroup share each tile's keys
   // where that leaves CUs unused (1500 tokens, 24 heads: 51 -> 38 us; 2048
   // tokens, 32 heads: 57 -> 51; 4 x 500 tokens stay: 24 against 26).
-  if (!f32 && p.nw == 4 && longest >= 6 &&
+  if (!f32 && p.nw == 4 && longest >= 7 &&
       (tiles <= num_cus || (tiles <= 2 * (int64_t)num_cus && longest >= 32)))
     p.ks = 2;
   // Of that chunk and longer ones, the one whose cut of the longest tile's
-  // chain (us per step, measured) exceeds the cost of the partials by most: a
-  // merge launch, and their bytes written and read at 2.5 TB/s (100 queries
-  // after 4000 keys: 127 -> 32 us; 500 after 8000: 257 -> 94).
+  // chain (us per step, measured) exceeds the cost of the partials by most:
+  // the workspace and the second launch (a lone call is as long as its host
+  // side, 5 us more with a split: 2 queries over 227 keys 13.8 us without,
+  // 16.0 with; 4 rows' 5 over 378 19.7, 23.3), and the bytes written and read
+  // at 2.5 TB/s (100 queries after 4000 keys: 127 -> 32 us; 500 after 8000:
+  // 257 -> 94).  Where the grid alone fills the CUs the cut has to be a sixth
+  // of the chain, as less of it shows (5600 tokens, 24 heads: 225 us, 250 with
+  // the split that saves 5 of 157 by this count).
   const double step = f32 ? 5.5 : p.nw == 4 ? 0.9 : 1.1;
-  const double unsplit = longest * step / (p.ks == 2 ? 1.6 : 1.0);
+  // (the second group of waves takes 1/7 off: 60 us unsplit for 290 queries
+  // over 2706 keys, 42 split)
+  const double unsplit = longest * (p.nw < 4 ? 0.9 : step) / (p.ks == 2 ? 1.15 : 1.0);
+  const double launch = B > 1 ? 11 : 8;
   double best = 0;
   p.nsplit = 1;
   p.chunk = (int)(longest * p.kt);
   for (; chunk < longest; chunk += chunk / 4 + 1) {
     const int64_t ns = (longest + chunk - 1) / chunk;
     if (prefill_split_bytes(all_rows, (int)ns, D) > ws_bytes) continue;
-    const double net = unsplit - chunk * step - 4 - all_rows * (mean / chunk) * (D * 4 + 8) * 2 / 2.5e6;
-    if (net > best) {
+    const double net =
+        unsplit - chunk * step - launch - all_rows * (mean / chunk) * (D * 4 + 8) * 2 / 2.5e6;
+    if (net > best && net > (tiles > num_cus ? unsplit / 6 : 0)) {
       best = net;
       p.nsplit = (int)ns;
       p.chunk = (int)(chunk * p.kt);
     }
   }
   if (p.nsplit > 1) p.ks = 1;
-  // 64-key tiles (two workgroups per CU) halve the steps of launches that
-  // leave room: 4096 tokens, 32 heads 155 -> 138 us; 4 x 2048 tokens 148 -> 154.
-  if (p.nsplit == 1 && p.ks == 1 && p.nw == 4 && !f32 && tiles <= 4 * (int64_t)num_cus) p.kt = 64;
+  // Without a split, tiles of few rows have four waves load for the one or two
+  // that compute, as the chain of loads is what they wait for, and from 7
+  // steps on another four take half the keys (2 queries over 227 keys: 14.4 ->
+  // 11.5 us; 4 rows' 12 over 512: 27.6 -> 18.9).  The fp32 kernel's tiles take
+  // fewer rows where that leaves no CU a second one: its waves read all of K
+  // and V from LDS, and fewer of them read faster (100 tokens, 8 heads: 15.4
+  // -> 13.8; with a split the second operand reads cost more: 400 tokens 19.4
+  // -> 21.6).
+  if (f32 && p.nsplit == 1)
+    while (p.qr > 16 && (rows + p.qr / 2 - 1) / (p.qr / 2) * B * Hkv <= num_cus) p.qr /= 2;
+  if (p.nsplit == 1 && p.nw < 4 && tiles <= num_cus) {
+    p.nw = 4;
+    p.qr = 128;
+    p.ks = longest >= 7 ? 2 : 1;
+    return p;
+  }
+  // 64-key tiles (two workgroups per CU) halve the steps, 32-key tiles run
+  // three workgroups per CU: the first for launches that leave room (4096
+  // tokens, 32 heads 155 -> 138 us; 4 x 2048 tokens stay, 148 against 154),
+  // and for long chains in a little more, whose third workgroups would only
+  // leave a thin tail (2781 tokens x 2, 24 heads: 122 -> 109; 6000 tokens, 24
+  // heads: 264 -> 234; 7000: 328 -> 311; but 4 x 1150 tokens, 32 heads stay,
+  // 58 against 61, and 5200 tokens, 32 heads, 218 against 231).
+  const double per_cu_tiles = (double)tiles / num_cus;
+  if (p.nsplit == 1 && p.ks == 1 && p.nw == 4 && !f32 &&
+      (per_cu_tiles <= 4 || (per_cu_tiles <= 4.5 && longest >= 40) ||
+       (per_cu_tiles <= 5.5 && longest >= 200)))
+    p.kt = 64;
   return p;
 }
 
@@ -1627,13 +1661,12 @@ void launch_prefill(strata_ctx* ctx, const void* q, const void* k, const void* v
   constexpr bool f32 = sizeof(TQ) == 4;
   const int64_t rows = (int64_t)B * Hq * Lq;
   const PrefillPlan pl = prefill_plan(ctx->num_cus, f32, B, Hq, Hkv, Lq, Lk, D, causal, ex.ws_bytes);
-  PrefillSplit sp{pl.nsplit, pl.chunk, nullptr, nullptr};
+  PrefillSplit sp{pl.nsplit, pl.chunk, pl.qr, nullptr, nullptr};
   if (pl.nsplit > 1) {
     sp.o = static_cast<float*>(ex.ws);
     sp.ms = reinterpret_cast<float2*>(sp.o + rows * pl.nsplit * D);
   }
-  const int qr = (f32 ? 16 : 32) * pl.nw;
-  const int nqt = (int)(((int64_t)Lq * (Hq / Hkv) + qr - 1) / qr);
+  const int nqt = (int)(((int64_t)Lq * (Hq / Hkv) + pl.qr - 1) / pl.qr);
   const dim3 grid(prefill_grid(nqt, B, Hkv), pl.nsplit);
 #define STRATA_PF(KERNEL)                                                                        \
   hipLaunchKernelGGL(KERNEL, grid, dim3(64 * pl.nw * pl.ks), 0, stream, (const TQ*)q, (const TQ*)k,      \

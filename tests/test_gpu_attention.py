@@ -329,6 +329,41 @@ def test_prefill_key_splits(dev, dtype, B, Hq, Hkv, D, Lq, Lk, causal, given):
     assert bool(got[0, :Hq // Hkv, sees].isnan().all()) and bool(got[0, Hq // Hkv:].isfinite().all())
 
 
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,D,Lq,Lk,given", [
+    ("bf16", 1, 8, 2, 128, 4, 230, False), ("bf16", 2, 6, 2, 64, 20, 234, True),
+    ("bf16", 1, 8, 8, 128, 7, 90, False),
+    ("f32", 1, 8, 2, 64, 100, 100, False), ("f32", 2, 6, 2, 64, 7, 70, True),
+    ("f32", 1, 4, 4, 128, 33, 33, False), ("f32", 40, 8, 2, 64, 21, 40, False)])
+def test_prefill_few_rows_without_split(dev, dtype, B, Hq, Hkv, D, Lq, Lk, given):
+    """Short unsplit prefill against float64: bf16 tiles of 32 or 64 rows that
+    four or eight waves load, fp32 tiles of 16 and 32 rows (16 * 40 * 2 tiles
+    fill the CUs: 64).  Given positions include rows that see no key (0) and
+    rows that see them all.  bf16 rounds weights and outputs at 2^-9, fp32 each
+    sum term at 2^-24."""
+    import ctypes as C
+    from lokahi_amd import _abi, ops
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    gen = torch.Generator(device=dev).manual_seed(Lq + Lk)
+    q, k, v = (torch.randn((B, h, l, D), generator=gen, device=dev).to(dt)
+               for h, l in ((Hq, Lq), (Hkv, Lk), (Hkv, Lk)))
+    need = C.c_int64()
+    _abi.check(_abi.load().strata_attn_workspace(ops._ctx(0), ops._code(q), ops._code(k), ops._code(v),
+                                                 B, Hq, Hkv, Lq, Lk, D, 1, C.byref(need)))
+    assert need.value == 0  # the call is not split
+    pos = torch.arange(Lk - Lq, Lk, device=dev, dtype=torch.int32).expand(B, Lq)
+    if given:
+        pos = torch.randint(0, Lk, (B, Lq), generator=gen, device=dev, dtype=torch.int32)
+        pos[0, 3], pos[0, 5], pos[-1, 6] = -1, 0, Lk - 1
+    mask = torch.arange(Lk, device=dev) <= pos[:, None, :, None]
+    sc = torch.matmul(q.double(), k.double().repeat_interleave(Hq // Hkv, 1).transpose(2, 3).contiguous())
+    w = torch.exp((sc - sc.amax(-1, keepdim=True)) / D**0.5) * mask
+    ref = torch.matmul(w, v.double().repeat_interleave(Hq // Hkv, 1)) / w.sum(-1, keepdim=True).clamp_min(1e-12)
+    got = ops.attention(q, k, v, query_positions=pos if given else None)
+    assert float((got.double() - ref).norm() / ref.norm()) < (5e-3 if dtype == "bf16" else 2e-6)
+    if given:
+        assert bool((got[0, :, 3] == 0).all())
+
+
 @pytest.mark.parametrize("Hq,Hkv,D,Lq,Lk", [(24, 8, 128, 200, 200), (6, 2, 64, 193, 211),
                                             (32, 8, 128, 700, 707), (8, 8, 128, 130, 1000),
                                             (32, 8, 128, 1100, 1100), (32, 8, 128, 3000, 3000)])
