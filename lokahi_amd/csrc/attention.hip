@@ -494,10 +494,21 @@ struct PrefillSplit {
   float2* ms;
 };
 
+// Last key this lane's query sees, -1 past the last row.  Given positions may
+// lie past the keys (absolute positions over a trimmed cache): such a query
+// sees them all.
+__device__ __forceinline__ int query_position(const int32_t* qpos, int causal, bool row_ok, int b, int row,
+                                              int Lq, int Lk) {
+  if (!row_ok) return -1;
+  if (!causal) return Lk - 1;
+  return qpos ? min(qpos[(int64_t)b * Lq + row], Lk - 1) : Lk - Lq + row;
+}
+
 // Key limits of a wave's rows pr0 .. pr0 + R - 1 and of the workgroup's rows
 // (up to pr_end): kfull, keys every row of the wave sees (0 with a row past
 // the last: tiles then mask); need, keys any of its rows sees; kmax, keys any
-// row of the workgroup sees.  qp: this lane's position, -1 past the last row.
+// row of the workgroup sees.  qp: this lane's query_position (below Lk, or a
+// tile that holds the last keys only in part would go unmasked).
 // Without given positions they follow from the row numbers; given ones are
 // reduced over the R lanes that hold the wave's rows and over the workgroup
 // (s_kmax, two barriers).
@@ -525,7 +536,7 @@ __device__ __forceinline__ void key_limits(const int32_t* qpos, int causal, int 
   __syncthreads();
   *kfull = f;
   *need = n;
-  *kmax = min(Lk, *s_kmax);
+  *kmax = *s_kmax;
 }
 
 __device__ __forceinline__ f32x4_t mfma_f32(float a, float b, f32x4_t c) {
@@ -567,8 +578,7 @@ __global__ __launch_bounds__(256) void attn_prefill_f32(
   const int pr = qt * qr + 16 * wave + col;  // this lane's packed row
   const int row = pr / G, hq = hkv * G + (pr - row * G);
   const bool row_ok = 16 * wave < qr && row < Lq;
-  const int qp = row_ok ? (causal ? (qpos ? qpos[(int64_t)b * Lq + row] : Lk - Lq + row) : Lk - 1)
-                        : -1;
+  const int qp = query_position(qpos, causal, row_ok, b, row, Lq, Lk);
   const float* kbase = k + (int64_t)b * kv_bs + (int64_t)hkv * kv_hs;
   const float* vbase = v + (int64_t)b * kv_bs + (int64_t)hkv * kv_hs;
   // Tiles: 16-byte chunks, chunk c of the tile -> (key t, element d0); keys
@@ -780,8 +790,7 @@ void attn_prefill_mfma32(
   const int pr = qt * QR + 32 * wave + c32;  // this lane's packed row
   const int row = pr / G, hq = hkv * G + (pr - row * G);
   const bool row_ok = row < Lq;
-  const int qp = row_ok ? (causal ? (qpos ? qpos[(int64_t)b * Lq + row] : Lk - Lq + row) : Lk - 1)
-                        : -1;
+  const int qp = query_position(qpos, causal, row_ok, b, row, Lq, Lk);
   // Buffer descriptors of this head's K and V rows: keys at or past Lk
   // read as zero.
   const v4i32_t rk = rsrc(k + (int64_t)b * kv_bs + (int64_t)hkv * kv_hs, (uint32_t)Lk * ROW);

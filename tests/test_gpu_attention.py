@@ -394,3 +394,43 @@ def test_prefill_without_split(dev, Hq, Hkv, D, Lq, Lk):
     ref = torch.matmul(torch.softmax(sc, -1), v.double().repeat_interleave(Hq // Hkv, 1))
     assert float((got[:, :, rows].double() - ref).norm() / ref.norm()) < 5e-3
     assert bool(got.isfinite().all())
+
+
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,D,Lq,Lk,split", [
+    ("bf16", 1, 32, 8, 128, 8, 100, False),     # 32 packed rows, four waves load
+    ("bf16", 40, 32, 8, 64, 8, 97, False),      # one-wave tiles
+    ("bf16", 40, 32, 8, 128, 16, 97, False),    # two-wave tiles
+    ("bf16", 1, 24, 8, 128, 200, 289, False),   # two wave groups, Lk % 64 == 33
+    ("bf16", 4, 24, 8, 64, 500, 544, False),    # 64-key tiles, Lk % 64 == 32
+    ("bf16", 40, 32, 8, 128, 100, 132, False),  # the plain kernel
+    ("bf16", 1, 32, 8, 128, 100, 2017, True), ("bf16", 2, 6, 2, 64, 17, 1508, True),
+    ("bf16", 1, 8, 2, 128, 8, 1313, True),
+    ("f32", 1, 8, 2, 64, 4, 100, False), ("f32", 1, 8, 2, 128, 60, 65, False),
+    ("f32", 1, 8, 2, 64, 300, 545, True), ("f32", 2, 8, 2, 128, 5, 740, True)])
+def test_prefill_positions_past_the_keys(dev, dtype, B, Hq, Hkv, D, Lq, Lk, split):
+    """Given positions at or past the last key (absolute positions over a
+    trimmed cache): such a row sees every key, and no more than those, whatever
+    part of a tile the last keys fill.  Against float64 over the rule key <=
+    position; bf16 rounds weights and outputs at 2^-9, fp32 each sum term at
+    2^-24."""
+    import ctypes as C
+    from lokahi_amd import _abi, ops
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    gen = torch.Generator(device=dev).manual_seed(Lq + Lk)
+    q, k, v = (torch.randn((B, h, l, D), generator=gen, device=dev).to(dt)
+               for h, l in ((Hq, Lq), (Hkv, Lk), (Hkv, Lk)))
+    need = C.c_int64()
+    _abi.check(_abi.load().strata_attn_workspace(ops._ctx(0), ops._code(q), ops._code(k), ops._code(v),
+                                                 B, Hq, Hkv, Lq, Lk, D, 1, C.byref(need)))
+    assert (need.value > 0) == split
+    past = torch.randint(Lk, 2 * Lk + 200, (B, Lq), generator=gen, device=dev, dtype=torch.int32)
+    some = past.clone()  # a tile with both kinds of rows
+    some[:, ::3] = torch.randint(0, Lk, (B, (Lq + 2) // 3), generator=gen, device=dev, dtype=torch.int32)
+    sc = torch.matmul(q.double(), k.double().repeat_interleave(Hq // Hkv, 1).transpose(2, 3).contiguous())
+    sc = torch.exp((sc - sc.amax(-1, keepdim=True)) / D**0.5)
+    for pos in (past, some, past.clamp_min(2**31 - 1)):
+        w = sc * (torch.arange(Lk, device=dev) <= pos[:, None, :, None])
+        ref = torch.matmul(w, v.double().repeat_interleave(Hq // Hkv, 1)) / w.sum(-1, keepdim=True)
+        got = ops.attention(q, k, v, query_positions=pos)
+        err = float((got.double() - ref).norm() / ref.norm())
+        assert err < (5e-3 if dtype == "bf16" else 2e-6), (int(pos.min()), err)
