@@ -105,7 +105,7 @@ int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const str
                               packed->K == K && packed->count == count
                           ? packed->buf
                           : nullptr;
-  const size_t pb = strata_q4_gemm_mfma_part_bytes(M, K, fast, nfast);
+  size_t pb = strata_q4_gemm_mfma_part_bytes(M, K, fast, nfast);
   // Up to kMlxMaxRows rows the kernel reads the linears' own tensors instead
   // (the same bits): the re-layout takes as long as the GEMM gains (8B gate/up:
   // 128 rows 77 -> 53 us, 512 rows 139 -> 138, 1000 rows 243 against 267).
@@ -114,7 +114,22 @@ int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const str
   void* scr = nullptr;
   if (pk + pb > 0) {
     const int rc = strata_ctx_scratch(ctx, pk + pb, &scr, stream);
-    if (rc) return rc;
+    if (rc && M > kSkinnyMaxRows) return rc;
+    if (rc) {
+      // A short call never depends on scratch (the arena cannot grow under
+      // stream capture): K whole instead of in slices, the 128 x 128 kernel
+      // instead of a re-layout.
+      (void)hipGetLastError();
+      pb = 0;
+      if (pk) {
+        for (int i = 0; i < nfast; ++i) {
+          const int rc1 = strata_q4_gemm_launch(x, M, K, fast[i].w, fast[i].scales, fast[i].biases,
+                                                (int)fast[i].N, fast[i].y, y_dtype, stream);
+          if (rc1) return rc1;
+        }
+        return STRATA_OK;
+      }
+    }
   }
   if (!pk_in && !mlx) {
     const int rc = strata_q4_gemm_pack(fast, nfast, K, scr, stream);

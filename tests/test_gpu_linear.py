@@ -310,3 +310,37 @@ def test_few_rows_keep_fp32_weights(dev, M, K, ns):
         ref = bf16_bits_to_f32(x).astype(np.float64) @ q4.dequantize(w, s, b, 64).astype(np.float64).T
         assert rel_err(to_np_f32(y), ref) < 1e-5
         assert torch.equal(ops.linear(xd, *dp, out_dtype=torch.float32), y)
+
+
+@pytest.mark.parametrize("M,K,ns", [(33, 512, (8192,)), (39, 4096, (14336, 14336)), (34, 1024, (8192, 48)),
+                                    (36, 192, (256,)), (38, 320, (512, 256))])
+def test_short_prefill_needs_no_scratch(dev, M, K, ns):
+    """33-39 rows under capture with a context whose scratch arena cannot grow:
+    the call runs as it does for fewer rows (on K slices or a re-layout it has
+    no scratch for, it goes without), on every replay.  fp32 sums of exact
+    bf16 products against float64: K terms at 2^-24 each."""
+    import ctypes as C
+    from lokahi_amd import _abi, ops
+    gen = torch.Generator(device=dev).manual_seed(M + K)
+    ws = [ops.quantize(torch.randn((n, K), generator=gen, device=dev) * 0.02) for n in ns]
+    x = torch.randn((M, K), generator=gen, device=dev).bfloat16()
+    warm = ops.linear_multi(x, ws, out_dtype=torch.float32)
+    ctx = _abi.Context(0)
+    ys = [torch.empty_like(y) for y in warm]
+    arr = (_abi.Q4Weight * len(ns))(*[_abi.Q4Weight(w.data_ptr(), s.data_ptr(), b.data_ptr(), n, y.data_ptr())
+                                      for (w, s, b), n, y in zip(ws, ns, ys)])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rc = _abi.load().strata_linear_q4_multi(ctx.handle, x.data_ptr(), _abi.BF16, M, K, arr, len(ns), 64, 4,
+                                                _abi.F32, ops._raw_stream(0))
+    _abi.check(rc)
+    for scale in (1.0, -2.0):
+        x.mul_(scale)
+        graph.replay()
+        torch.cuda.synchronize()
+        for (w, s, b), y, yw in zip(ws, ys, warm):
+            ref = x.double() @ ops.dequantize(w, s, b).double().T
+            assert float((y - ref).norm() / ref.norm()) < 1e-5
+            if scale == 1.0:
+                assert float((y - yw).norm() / yw.norm()) < 1e-5
