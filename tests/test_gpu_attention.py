@@ -434,3 +434,16 @@ def test_prefill_positions_past_the_keys(dev, dtype, B, Hq, Hkv, D, Lq, Lk, spli
         got = ops.attention(q, k, v, query_positions=pos)
         err = float((got.double() - ref).norm() / ref.norm())
         assert err < (5e-3 if dtype == "bf16" else 2e-6), (int(pos.min()), err)
+
+
+def test_attention_option_types(dev):
+    """Block sizes and eps of any type that converts to an int and a float."""
+    from lokahi_amd import ops
+    q, k, v = (torch.randn((1, h, 5, 64), device=dev) for h in (4, 2, 2))
+    ref = ops.attention(q, k, v)
+    for qb, kb, eps in ((512.0, np.float64(256), np.float32(1e-12)), (float("inf"), 2**40, torch.tensor(1e-12)),
+                        (np.int64(8), torch.tensor(4), 1)):
+        out = ops.attention(q, k, v, q_block_size=qb, k_block_size=kb, eps=eps)
+        assert torch.equal(out, ref)  # every weight sum is at least 1
+    with pytest.raises(ValueError, match="block sizes"):
+        ops.attention(q, k, v, k_block_size=0.5)
