@@ -30,7 +30,8 @@ _DT = {torch.float32: F32, torch.bfloat16: BF16}
 # raw stream handles, outputs allocated in their final shape and C structs
 # packed by struct.Struct (a ctypes array of Structures takes 3 us for two
 # weights) instead of the objects around them.
-_raw_stream = torch._C._cuda_getCurrentRawStream
+# (A PyTorch without a GPU backend has no such function, and no tensor to call it for.)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 _Q4 = {n: struct.Struct("PPPqP" * n) for n in range(1, 9)}  # strata_q4_weight[n]
 
 

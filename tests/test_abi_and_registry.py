@@ -1,6 +1,8 @@
 """CPU-side checks of the C ABI library and the backend registry."""
 import ctypes as C
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import pytest
@@ -70,3 +72,18 @@ def test_capabilities_declare_the_hot_path():
         assert op in caps.supported_operations
     assert caps.supports_quantized_weights and caps.supports_external_kv_cache
     assert set(caps.supported_dtypes) == {"bfloat16", "float32"}
+
+
+def test_ops_import_without_a_gpu_pytorch():
+    """PyTorch builds without a GPU backend lack the raw-stream function: the
+    modules still import (in a process of their own), and refuse CPU tensors."""
+    code = ("import torch\n"
+            "del torch._C._cuda_getCurrentRawStream\n"
+            "import lokahi_amd.kvcache, lokahi_amd.llama\n"
+            "from lokahi_amd import ops\n"
+            "try:\n"
+            "    ops.silu_mul(torch.ones(8), torch.ones(8))\n"
+            "except ValueError as e:\n"
+            "    print(e)\n")
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, cwd=ROOT)
+    assert done.returncode == 0 and "HIP device" in done.stdout, done.stderr
