@@ -267,6 +267,8 @@ void launch_skinny(const uint16_t* x, int M, int K, const SkinnyBatch& bt, int c
 bool strata_q4_skinny_fits(int M, int K, const strata_q4_weight* ws, int count) {
   if (M < 1 || M > kSkinnyMaxRows || K % 512 != 0 || count < 1 || count > kMaxGemmProblems)
     return false;
+  // byte offsets into x and into a workgroup's up to 64 weight rows are 32-bit
+  if ((uint64_t)M * K * 2 >= (1ull << 32) || (uint64_t)64 * K / 2 >= (1ull << 32)) return false;
   for (int i = 0; i < count; ++i)
     if (ws[i].N % 16 != 0 || !aligned16(ws[i].w) ||
         ((reinterpret_cast<uintptr_t>(ws[i].scales) | reinterpret_cast<uintptr_t>(ws[i].biases)) & 3))
@@ -277,7 +279,8 @@ bool strata_q4_skinny_fits(int M, int K, const strata_q4_weight* ws, int count) 
 int strata_q4_gemm_skinny(const void* x, int M, int K, const strata_q4_weight* ws, int count,
                           int y_dtype, void* stream, bool exact) {
   STRATA_REQUIRE(strata_q4_skinny_fits(M, K, ws, count),
-                 "q4 skinny GEMM: needs 1 <= M <= %d, K %% 512 == 0, N %% 16 == 0", kSkinnyMaxRows);
+                 "q4 skinny GEMM: needs 1 <= M <= %d, K %% 512 == 0, N %% 16 == 0, operands under 4 GiB",
+                 kSkinnyMaxRows);
   STRATA_REQUIRE(aligned16(x), "q4 skinny GEMM: x must be 16-byte aligned");
   SkinnyBatch bt{};
   bt.count = count;

@@ -344,3 +344,22 @@ def test_short_prefill_needs_no_scratch(dev, M, K, ns):
             assert float((y - ref).norm() / ref.norm()) < 1e-5
             if scale == 1.0:
                 assert float((y - yw).norm() / yw.norm()) < 1e-5
+
+
+def test_few_rows_beyond_32_bit_offsets(dev):
+    """x of 4 GiB (64 rows): byte offsets that 32 bits do not hold.  x is zero
+    but for a few columns, so the reference needs only those."""
+    from lokahi_amd import ops
+    M, K, N = 64, 1 << 25, 16
+    gen = torch.Generator(device=dev).manual_seed(5)
+    w = torch.randint(-2**31, 2**31 - 1, (N, K // 8), generator=gen, device=dev, dtype=torch.int32)
+    s, b = (torch.rand((N, K // 64), generator=gen, device=dev).bfloat16() for _ in range(2))
+    cols = torch.tensor([0, 1, 65, K // 4 + 7, K // 2, K - 70, K - 1], device=dev)
+    xc = torch.randn((M, len(cols)), generator=gen, device=dev).bfloat16()
+    x = torch.zeros((M, K), device=dev, dtype=torch.bfloat16)
+    x[:, cols] = xc
+    y = ops.linear(x, w, s, b, out_dtype=torch.float32)
+    codes = (w[:, cols // 8] >> (4 * (cols % 8))) & 15
+    wq = (codes * s[:, cols // 64].float() + b[:, cols // 64].float()).bfloat16()
+    ref = xc.double() @ wq.double().T
+    assert float((y - ref).norm() / ref.norm()) < 1e-5
