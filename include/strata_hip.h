@@ -151,9 +151,14 @@ int strata_attn_gqa(strata_ctx* ctx, const void* q, int q_dtype, const void* k, 
  * query rows whose tiles would leave the GPU idle splits its keys over more
  * workgroups, keeps their fp32 partials there and merges them.  The workspace
  * is in use until the call's work on `stream` is done; calls that may overlap
- * need one each.  strata_attn_workspace sets *bytes to 0 when no split pays. */
+ * need one each.  strata_attn_workspace sets *bytes to 0 when no split pays;
+ * with less than it asks for the keys are split into fewer parts or not at all.
+ * strata_attn_workspace_max: enough for every call of up to max_Lq queries per
+ * row over up to max_Lk keys, causal or not (a caller that keeps one workspace). */
 int strata_attn_workspace(strata_ctx* ctx, int q_dtype, int k_dtype, int v_dtype, int B, int Hq,
                           int Hkv, int Lq, int Lk, int D, int causal, int64_t* bytes);
+int strata_attn_workspace_max(strata_ctx* ctx, int q_dtype, int k_dtype, int v_dtype, int B, int Hq,
+                              int Hkv, int max_Lq, int max_Lk, int D, int64_t* bytes);
 int strata_attn_gqa_ws(strata_ctx* ctx, const void* q, int q_dtype, const void* k, int k_dtype,
                        const void* v, int v_dtype, int64_t kv_batch_stride,
                        int64_t kv_head_stride, const int32_t* qpos, int B, int Hq, int Hkv,

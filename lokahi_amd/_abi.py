@@ -83,6 +83,7 @@ _SIGS = {
                          C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float,
                          C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p], C.c_int),
     "strata_attn_workspace": ([C.c_void_p] + [C.c_int] * 10 + [C.POINTER(C.c_int64)], C.c_int),
+    "strata_attn_workspace_max": ([C.c_void_p] + [C.c_int] * 9 + [C.POINTER(C.c_int64)], C.c_int),
     "strata_attn_gqa_noalloc": ([C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_int,
                                  C.c_void_p, C.c_int, C.c_int64, C.c_int64, C.c_void_p, C.c_int,
                                  C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int,

@@ -257,6 +257,16 @@ int strata_attn_workspace(strata_ctx* ctx, int q_dtype, int k_dtype, int v_dtype
   return STRATA_OK;
 }
 
+int strata_attn_workspace_max(strata_ctx* ctx, int q_dtype, int k_dtype, int v_dtype, int B, int Hq,
+                              int Hkv, int max_Lq, int max_Lk, int D, int64_t* bytes) {
+  STRATA_REQUIRE(ctx != nullptr && bytes != nullptr, "ctx/bytes is NULL");
+  STRATA_REQUIRE(B > 0 && max_Lq >= 0 && max_Lk >= 0 && D > 0, "invalid shape");
+  STRATA_REQUIRE(Hkv > 0 && Hq > 0 && Hq % Hkv == 0,
+                 "query heads must be divisible by key/value heads");
+  *bytes = (int64_t)strata_attn_prefill_ws_max(ctx, q_dtype, k_dtype, v_dtype, B, Hq, max_Lq, max_Lk, D);
+  return STRATA_OK;
+}
+
 int strata_attn_gqa_ws(strata_ctx* ctx, const void* q, int q_dtype, const void* k, int k_dtype,
                        const void* v, int v_dtype, int64_t kv_batch_stride, int64_t kv_head_stride,
                        const int32_t* qpos, int B, int Hq, int Hkv, int Lq, int Lk, int D,

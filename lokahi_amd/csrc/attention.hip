@@ -1777,6 +1777,27 @@ size_t strata_attn_prefill_ws(strata_ctx* ctx, int qd, int kd, int vd, int B, in
   return prefill_split_bytes((int64_t)B * Hq * Lq, p.nsplit, D);
 }
 
+// Bytes that suffice for every call of up to Lq queries per row over up to Lk
+// keys.  The need is not monotonic in either, so this is a bound and no search
+// (24 heads, D = 128, 8192 tokens: 217 MB, the largest need of any length is
+// 104 MB).  A split of chunk steps covers n = ceil(longest / chunk) < longest /
+// chunk + 1 splits of `rows` output rows, and prefill_plan has chunk >= tiles *
+// mean / (3 CUs) and rows <= 128 tiles; longest / mean is under 2.25 where a
+// chunk of 8 steps is less than the whole (half the keys of a causal tile, and
+// the last step's rounding; fewer rows per tile leave more room than the shorter
+// chunks take).  So n rows < rows + 864 CUs, and with rows >= 864 CUs no chunk is
+// short enough to split.
+size_t strata_attn_prefill_ws_max(strata_ctx* ctx, int qd, int kd, int vd, int B, int Hq, int Lq,
+                                  int Lk, int D) {
+  if (Lq <= 1 || (D != 64 && D != 128) || qd != kd || kd != vd) return 0;
+  const bool f32 = qd == STRATA_F32;
+  const int64_t steps = (Lk + (f32 ? 63 : 31)) / (f32 ? 64 : 32), least = f32 ? 1 : 4;
+  const int64_t most = std::min<int64_t>(kMaxPrefillSplits, (steps + least - 1) / least);
+  if (most <= 1) return 0;
+  const int64_t cap = (int64_t)864 * ctx->num_cus, rows = std::min((int64_t)B * Hq * Lq, cap);
+  return std::min(kMaxPrefillWs, (size_t)std::min(rows * most, rows + cap) * (D * 4 + 8));
+}
+
 int strata_attention_dispatch(strata_ctx* ctx, const void* q, int qd, const void* k, int kd,
                               const void* v, int vd, int64_t kv_bs, int64_t kv_hs,
                               const int32_t* qpos, int B, int Hq, int Hkv, int Lq, int Lk, int D,

@@ -399,21 +399,19 @@ int strata_decoder_create(strata_ctx* ctx, const strata_llama_config* cfg,
   if (!rc)
     rc = alloc(reinterpret_cast<void**>(&d->part),
                (size_t)kv->B * c.num_heads * part_stride(d->part_splits, c.head_dim) * 4);
-  // Key-split partials of prefill attention, sized for the prompt lengths up to
-  // max_tokens over a full cache; without them the attention runs unsplit.
-  for (int64_t l = max_tokens / kv->B; !rc && l > 1; l = l * 3 / 4)
-    d->attn_ws_bytes = std::max(d->attn_ws_bytes,
-                                strata_attn_prefill_ws(ctx, STRATA_BF16, STRATA_BF16, STRATA_BF16, kv->B,
-                                                       c.num_heads, c.num_kv_heads, (int)l, kv->Lmax,
-                                                       c.head_dim, 1));
-  d->attn_ws_bytes = std::min(d->attn_ws_bytes, (size_t)256 << 20);
+  if (!rc) rc = pack_prefill_weights(d);
+  if (!rc) rc = build_decode_layouts(d);
+  // Key-split partials of prefill attention, enough for every prompt and
+  // history this decoder takes; allocated after what it cannot do without, and
+  // where there is no memory left for them the keys are not split.
+  if (!rc)
+    d->attn_ws_bytes = strata_attn_prefill_ws_max(ctx, STRATA_BF16, STRATA_BF16, STRATA_BF16, kv->B, c.num_heads,
+                                                  std::min(max_tokens / kv->B, kv->Lmax), kv->Lmax, c.head_dim);
   if (d->attn_ws_bytes && hipMalloc(&d->attn_ws, d->attn_ws_bytes) != hipSuccess) {
     (void)hipGetLastError();
     d->attn_ws = nullptr;
     d->attn_ws_bytes = 0;
   }
-  if (!rc) rc = pack_prefill_weights(d);
-  if (!rc) rc = build_decode_layouts(d);
   if (!rc) rc = strata_rope_table_launch(d->rope_table, kv->Lmax, c.head_dim, c.rope_theta, nullptr);
   if (!rc && hipDeviceSynchronize() != hipSuccess)
     rc = strata_set_error(STRATA_EHIP, "decoder: RoPE table initialisation failed");

@@ -135,6 +135,8 @@ int strata_attention_dispatch(strata_ctx* ctx, const void* q, int qd, const void
                               void* stream);
 size_t strata_attn_prefill_ws(strata_ctx* ctx, int qd, int kd, int vd, int B, int Hq, int Hkv, int Lq,
                               int Lk, int D, int causal);
+size_t strata_attn_prefill_ws_max(strata_ctx* ctx, int qd, int kd, int vd, int B, int Hq, int Lq,
+                                  int Lk, int D);
 int strata_attn_decode_splits(strata_ctx* ctx, int B, int Hkv, int Lcap);
 int strata_rope_launch(void* q, void* k, const int32_t* pos, int B, int Hq, int Hkv, int L, int D,
                        float theta, int dtype, void* stream);

@@ -447,3 +447,36 @@ def test_attention_option_types(dev):
         assert torch.equal(out, ref)  # every weight sum is 1 - 2^-22 or more, above each eps
     with pytest.raises(ValueError, match="block sizes"):
         ops.attention(q, k, v, k_block_size=0.5)
+
+
+@pytest.mark.parametrize("dtype,D", [("bf16", 128), ("bf16", 64), ("f32", 128), ("f32", 64)])
+def test_workspace_bound_covers_every_call(dev, dtype, D):
+    """strata_attn_workspace_max (what the decoder engine keeps) against the
+    need of calls within its lengths: the lengths where the need peaks (24
+    heads: 2771 tokens after 2336, 3000 after 8000), and random ones, causal or
+    not; and it stays within a few times the largest of them."""
+    import ctypes as C
+    import random
+    from lokahi_amd import _abi, ops
+    lib, h, code = _abi.load(), ops._ctx(0), (_abi.BF16 if dtype == "bf16" else _abi.F32)
+    n = C.c_int64()
+
+    def need(B, Hq, Hkv, lq, lk, causal=1):
+        _abi.check(lib.strata_attn_workspace(h, code, code, code, B, Hq, Hkv, lq, lk, D, causal, C.byref(n)))
+        return n.value
+
+    rng = random.Random(D)
+    for B, Hq, Hkv in ((1, 24, 8), (2, 32, 8), (8, 32, 8), (1, 8, 2), (1, 64, 8), (3, 6, 6)):
+        for most in (100, 260, 2048, 16384):
+            _abi.check(lib.strata_attn_workspace_max(h, code, code, code, B, Hq, Hkv, most // B, most, D, C.byref(n)))
+            bound, peak = n.value, 0
+            pairs = [(lq, lk) for lq, lk in ((2771, 5107), (3000, 11000), (1000, 9000), (10, 458))
+                     if lq <= most // B and lk <= most]
+            for _ in range(3000):
+                lq = min(most // B, int(2 * (most / 2 / B) ** rng.random()))
+                pairs.append((lq, rng.randint(lq, most)))
+            for lq, lk in pairs:
+                got = need(B, Hq, Hkv, lq, lk, int(rng.random() < 0.8))
+                assert got <= bound, (B, Hq, Hkv, most, lq, lk, got, bound)
+                peak = max(peak, got)
+            assert most < 2048 or bound < 8 * peak
