@@ -627,9 +627,7 @@ size_t strata_q4_gemm_mfma_part_bytes(int M, int K, const strata_q4_weight* ws, 
 bool strata_q4_gemm_mlx_fits(int K, const strata_q4_weight* ws, int count) {
   if (K % 128 != 0 || (uint64_t)K / 2 * TN >= (1ull << 32)) return false;
   for (int p = 0; p < count; ++p)
-    if (!aligned16(ws[p].w) ||
-        ((reinterpret_cast<uintptr_t>(ws[p].scales) | reinterpret_cast<uintptr_t>(ws[p].biases)) & 3))
-      return false;
+    if (!aligned16(ws[p].w) || !strata_q4_sb_aligned(ws[p])) return false;
   return true;
 }
 

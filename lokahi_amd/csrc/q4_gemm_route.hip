@@ -76,27 +76,27 @@ int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const str
   strata_q4_weight fast[kMaxGemmProblems], few[kMaxGemmProblems];
   int nfast = 0, nfew = 0;
   int64_t Nfast = 0;
+  size_t al = 0;  // bytes of scales and biases that the skinny kernel cannot load where they are
+  auto tile128 = [&](const strata_q4_weight& w) {
+    return strata_q4_gemm_launch(x, M, K, w.w, w.scales, w.biases, (int)w.N, w.y, y_dtype, stream);
+  };
+  auto sb_bytes = [&](const strata_q4_weight& w) { return ((size_t)w.N * (K / 64) * 2 + 255) / 256 * 256; };
   for (int i = 0; i < count; ++i) {
     const bool mid = M >= kMfmaMidRows && x_ok && ws[i].N % 256 == 0 && aligned16(ws[i].w) &&
                      (uint64_t)(Nfast + ws[i].N) * K / 2 < (1ull << 32) && nfast < kMaxGemmProblems;
-    const bool skinny = M <= kSkinnyMaxRows && aligned16(x) && strata_q4_skinny_fits(M, K, &ws[i], 1) &&
+    const bool skinny = M <= kSkinnyMaxRows && aligned16(x) && strata_q4_skinny_shape(M, K, &ws[i], 1) &&
                         nfew < kMaxGemmProblems;
     if (skinny && !(mid && ws[i].N >= kMidWideN)) {
+      if (!strata_q4_sb_aligned(ws[i])) al += 2 * sb_bytes(ws[i]);
       few[nfew++] = ws[i];
     } else if (mid) {
       fast[nfast++] = ws[i];
       Nfast += ws[i].N;
     } else {
-      const int rc = strata_q4_gemm_launch(x, M, K, ws[i].w, ws[i].scales, ws[i].biases,
-                                           (int)ws[i].N, ws[i].y, y_dtype, stream);
+      const int rc = tile128(ws[i]);
       if (rc) return rc;
     }
   }
-  if (nfew > 0) {
-    const int rc = strata_q4_gemm_skinny(x, M, K, few, nfew, y_dtype, stream);
-    if (rc) return rc;
-  }
-  if (nfast == 0) return STRATA_OK;
   // The decoder's load-time re-layout is used when it was built for exactly
   // these linears (all of them on this path, the same total N and K);
   // otherwise this call re-lays the weights out into the scratch arena,
@@ -105,38 +105,68 @@ int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const str
                               packed->K == K && packed->count == count
                           ? packed->buf
                           : nullptr;
-  size_t pb = strata_q4_gemm_mfma_part_bytes(M, K, fast, nfast);
+  size_t pb = nfast ? strata_q4_gemm_mfma_part_bytes(M, K, fast, nfast) : 0;
   // Up to kMlxMaxRows rows the kernel reads the linears' own tensors instead
   // (the same bits): the re-layout takes as long as the GEMM gains (8B gate/up:
   // 128 rows 77 -> 53 us, 512 rows 139 -> 138, 1000 rows 243 against 267).
   const bool mlx = !pk_in && M <= kMlxMaxRows && strata_q4_gemm_mlx_fits(K, fast, nfast);
-  const size_t pk = pk_in || mlx ? 0 : (strata_q4_gemm_mfma_scratch(Nfast, K) + 255) / 256 * 256;
+  size_t pk = pk_in || mlx || !nfast ? 0 : (strata_q4_gemm_mfma_scratch(Nfast, K) + 255) / 256 * 256;
   void* scr = nullptr;
-  if (pk + pb > 0) {
-    const int rc = strata_ctx_scratch(ctx, pk + pb, &scr, stream);
+  bool have = true;
+  if (al + pk + pb > 0) {
+    const int rc = strata_ctx_scratch(ctx, al + pk + pb, &scr, stream);
     if (rc && M > kSkinnyMaxRows) return rc;
-    if (rc) {
-      // A short call never depends on scratch (the arena cannot grow under
-      // stream capture): K whole instead of in slices, the 128 x 128 kernel
-      // instead of a re-layout.
-      (void)hipGetLastError();
-      pb = 0;
-      if (pk) {
-        for (int i = 0; i < nfast; ++i) {
-          const int rc1 = strata_q4_gemm_launch(x, M, K, fast[i].w, fast[i].scales, fast[i].biases,
-                                                (int)fast[i].N, fast[i].y, y_dtype, stream);
-          if (rc1) return rc1;
+    // A short call never depends on scratch (the arena cannot grow under
+    // stream capture): K whole instead of in slices, the 128 x 128 kernel
+    // instead of a copy.
+    have = rc == STRATA_OK;
+    if (!have) (void)hipGetLastError();
+  }
+  if (nfew > 0) {
+    // Scales and biases at odd 2-byte addresses are copied for the skinny
+    // kernel's 4-byte loads (3072 x 8192, 24 rows: 18 us with the copies, 181
+    // on the 128 x 128 kernel, 14 aligned).
+    char* at = static_cast<char*>(scr);
+    strata_q4_weight run[kMaxGemmProblems];
+    int nrun = 0;
+    for (int i = 0; i < nfew; ++i) {
+      strata_q4_weight w = few[i];
+      if (!strata_q4_sb_aligned(w)) {
+        if (!have) {
+          const int rc = tile128(w);
+          if (rc) return rc;
+          continue;
         }
-        return STRATA_OK;
+        const size_t bytes = (size_t)w.N * (K / 64) * 2;
+        for (const uint16_t** t : {&w.scales, &w.biases}) {
+          STRATA_HIP_CHECK(hipMemcpyAsync(at, *t, bytes, hipMemcpyDeviceToDevice, as_stream(stream)));
+          *t = reinterpret_cast<const uint16_t*>(at);
+          at += sb_bytes(w);
+        }
       }
+      run[nrun++] = w;
+    }
+    if (nrun > 0) {
+      const int rc = strata_q4_gemm_skinny(x, M, K, run, nrun, y_dtype, stream);
+      if (rc) return rc;
     }
   }
-  if (!pk_in && !mlx) {
-    const int rc = strata_q4_gemm_pack(fast, nfast, K, scr, stream);
-    if (rc) return rc;
-    pk_in = scr;
+  if (nfast == 0) return STRATA_OK;
+  if (!have && pk) {
+    for (int i = 0; i < nfast; ++i) {
+      const int rc = tile128(fast[i]);
+      if (rc) return rc;
+    }
+    return STRATA_OK;
   }
-  float* part = pb ? reinterpret_cast<float*>(static_cast<char*>(scr) + pk) : nullptr;
+  if (!have) pb = 0;
+  char* own = static_cast<char*>(scr) + al;
+  if (pk) {
+    const int rc = strata_q4_gemm_pack(fast, nfast, K, own, stream);
+    if (rc) return rc;
+    pk_in = own;
+  }
+  float* part = pb ? reinterpret_cast<float*>(own + pk) : nullptr;
   return strata_q4_gemm_mfma_run(x, M, K, pk_in, fast, nfast, y_dtype, stream, part, pb);
 }
 

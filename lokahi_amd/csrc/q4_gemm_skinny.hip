@@ -264,15 +264,20 @@ void launch_skinny(const uint16_t* x, int M, int K, const SkinnyBatch& bt, int c
 
 }  // namespace
 
-bool strata_q4_skinny_fits(int M, int K, const strata_q4_weight* ws, int count) {
+bool strata_q4_skinny_shape(int M, int K, const strata_q4_weight* ws, int count) {
   if (M < 1 || M > kSkinnyMaxRows || K % 512 != 0 || count < 1 || count > kMaxGemmProblems)
     return false;
   // byte offsets into x and into a workgroup's up to 64 weight rows are 32-bit
   if ((uint64_t)M * K * 2 >= (1ull << 32) || (uint64_t)64 * K / 2 >= (1ull << 32)) return false;
   for (int i = 0; i < count; ++i)
-    if (ws[i].N % 16 != 0 || !aligned16(ws[i].w) ||
-        ((reinterpret_cast<uintptr_t>(ws[i].scales) | reinterpret_cast<uintptr_t>(ws[i].biases)) & 3))
-      return false;
+    if (ws[i].N % 16 != 0 || !aligned16(ws[i].w)) return false;
+  return true;
+}
+
+bool strata_q4_skinny_fits(int M, int K, const strata_q4_weight* ws, int count) {
+  if (!strata_q4_skinny_shape(M, K, ws, count)) return false;
+  for (int i = 0; i < count; ++i)
+    if (!strata_q4_sb_aligned(ws[i])) return false;
   return true;
 }
 

@@ -118,8 +118,13 @@ struct GemmPacked {
 int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const strata_q4_weight* ws,
                          int count, int y_dtype, void* stream, const GemmPacked* packed = nullptr);
 // Linears sharing x for a few rows (M <= kSkinnyMaxRows, K % 512 == 0, every
-// N % 16 == 0, 16-byte aligned weights and x, 4-byte aligned scales and biases): one launch, each weight read once.
+// N % 16 == 0, 16-byte aligned weights and x, 4-byte aligned scales and
+// biases): one launch, each weight read once.
 constexpr int kSkinnyMaxRows = 64;
+bool strata_q4_skinny_shape(int M, int K, const strata_q4_weight* ws, int count);  // but for scales and biases
+inline bool strata_q4_sb_aligned(const strata_q4_weight& w) {
+  return ((reinterpret_cast<uintptr_t>(w.scales) | reinterpret_cast<uintptr_t>(w.biases)) & 3) == 0;
+}
 bool strata_q4_skinny_fits(int M, int K, const strata_q4_weight* ws, int count);
 // exact (M <= 16): weights not rounded to bf16, as in the GEMV.
 int strata_q4_gemm_skinny(const void* x, int M, int K, const strata_q4_weight* ws, int count,

@@ -363,3 +363,46 @@ def test_few_rows_beyond_32_bit_offsets(dev):
     wq = (codes * s[:, cols // 64].float() + b[:, cols // 64].float()).bfloat16()
     ref = xc.double() @ wq.double().T
     assert float((y - ref).norm() / ref.norm()) < 1e-5
+
+
+@pytest.mark.parametrize("M,K,ns", [(9, 512, (48,)), (24, 8192, (3072,)), (32, 1024, (16384, 64)),
+                                    (64, 1536, (80, 1024)), (40, 512, (8192, 256))])
+def test_scales_at_odd_addresses(dev, M, K, ns):
+    """Scales and biases that start 2 bytes past a 4-byte boundary (views into a
+    larger buffer) take the same kernels as aligned ones: the same bits, also on
+    every replay of a captured call; with a scratch arena that cannot grow, fp32
+    sums in another order (K terms at 2^-24 each)."""
+    import ctypes as C
+    from lokahi_amd import _abi, ops
+    gen = torch.Generator(device=dev).manual_seed(M + K)
+    ws = [ops.quantize(torch.randn((n, K), generator=gen, device=dev) * 0.02) for n in ns]
+    x = torch.randn((M, K), generator=gen, device=dev).bfloat16()
+
+    def odd(t):
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=dev)
+        buf[1:] = t.flatten()
+        return buf[1:].view(t.shape)
+
+    wo = [(w, odd(s), odd(b)) for w, s, b in ws]
+    assert all(t.data_ptr() % 4 == 2 for _, s, b in wo for t in (s, b))
+    ref = ops.linear_multi(x, ws, out_dtype=torch.float32)
+    for y, r in zip(ops.linear_multi(x, wo, out_dtype=torch.float32), ref):
+        assert torch.equal(y, r)
+    ys = [torch.empty_like(y) for y in ref]
+    arr = (_abi.Q4Weight * len(ns))(*[_abi.Q4Weight(w.data_ptr(), s.data_ptr(), b.data_ptr(), n, y.data_ptr())
+                                      for (w, s, b), n, y in zip(wo, ns, ys)])
+    fresh = _abi.Context(0)
+    for handle, bound in ((ops._ctx(0), 0.0), (fresh.handle, 1e-5)):
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            rc = _abi.load().strata_linear_q4_multi(handle, x.data_ptr(), _abi.BF16, M, K, arr, len(ns), 64, 4,
+                                                    _abi.F32, ops._raw_stream(0))
+        _abi.check(rc)
+        for _ in range(3):
+            for y in ys:
+                y.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            for y, r in zip(ys, ref):
+                assert float((y - r).norm() / r.norm()) <= bound
