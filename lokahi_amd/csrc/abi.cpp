@@ -142,15 +142,19 @@ int strata_linear_q4_multi(strata_ctx* ctx, const void* x, int x_dtype, int64_t 
   if (M == 0) return STRATA_OK;
   if (M > 8 && x_dtype == STRATA_BF16)
     return strata_q4_gemm_multi(ctx, x, (int)M, (int)K, weights, count, y_dtype, stream);
-  // From 3 rows the row-block GEMV reads its weights twice (rows in passes of
-  // 2 or 4) and spends 4 dots per code; the skinny kernel without weight
-  // rounding takes them once: 8B gate/up 5 rows 49 -> 28 us, down 3 rows 33 ->
-  // 17 and 8 rows 63 -> 17, q/k/v 8 rows 16.6 -> 10.7 (2 rows 7.4 against
-  // 10.3).  4 rows of K = 4096 stage as two x items per thread: q/k/v 9.9
-  // against 10.7 us, kept.
-  if (M >= 3 && !(M == 4 && K == 4096) && x_dtype == STRATA_BF16 &&
-      strata_q4_skinny_fits((int)M, (int)K, weights, count))
-    return strata_q4_gemm_skinny(x, (int)M, (int)K, weights, count, y_dtype, stream, true);
+  if (x_dtype == STRATA_BF16 && strata_q4_few_rows_on_mfma((int)M, (int)K)) {
+    // each linear by its own shape, so that it gives the same bits in a fused
+    // call as alone
+    strata_q4_weight few[8], rest[8];
+    int nfew = 0, nrest = 0;
+    for (int i = 0; i < count; ++i) {
+      if (strata_q4_skinny_fits((int)M, (int)K, &weights[i], 1)) few[nfew++] = weights[i];
+      else rest[nrest++] = weights[i];
+    }
+    if (nfew) rc = strata_q4_gemm_skinny(x, (int)M, (int)K, few, nfew, y_dtype, stream, true);
+    if (!rc && nrest) rc = strata_q4_gemv(ctx, x, x_dtype, (int)M, (int)K, rest, nrest, y_dtype, stream);
+    return rc;
+  }
   return strata_q4_gemv(ctx, x, x_dtype, (int)M, (int)K, weights, count, y_dtype, stream);
 }
 

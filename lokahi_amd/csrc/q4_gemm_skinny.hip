@@ -281,6 +281,26 @@ bool strata_q4_skinny_fits(int M, int K, const strata_q4_weight* ws, int count) 
   return true;
 }
 
+// The GEMV spends 4 dots per code and row and takes rows in blocks of 4 (2 for 3
+// rows, or where 4 rows of x exceed its LDS), in steps of 4096 k (64 lanes, two
+// 16-byte loads of codes each): its time follows the row blocks and, up to K =
+// 8192, the whole steps that K takes.  This kernel's depends on K and the columns
+// only.  So up to 4 rows (one row block, or two of 2) stay with the GEMV where K
+// fills its steps.  Microseconds, GEMV | this kernel, weights from HBM:
+//   rows  columns x K:  4096 x 4096  6144 x 4096  28672 x 4096  28672 x 3584  8192 x 8192  28672 x 8192
+//   3                   7.3 |  6.7  10.4 |  9.6   29.5 | 30.7   28.5 | 26.1  22.6 | 18.9   53.6 | 57.5
+//   4                   7.3 |  6.8   9.0 |  9.8   27.6 | 30.4   26.9 | 26.1  22.4 | 19.1   54.3 | 58.2
+//   8                  12.2 |  6.8  15.3 |  9.9   46.7 | 31.0   46.3 | 26.6  39.2 | 20.1  103.1 | 59.2
+// and 4096 x 14336: 4 rows 32.5 | 18.4, 8 rows 60.7 | 18.7.  Both are as long as a
+// chain over K for narrow linears, this one the longer (8 rows, 1024 columns: K =
+// 3072 5.8 | 5.3, 8192 7.6 | 9.6; 4 rows, 14336 8.9 | 14.4); the columns are left
+// out of the rule, as a linear gives the same bits in a fused call as alone and
+// q/k/v are best in one launch.
+bool strata_q4_few_rows_on_mfma(int M, int K) {
+  const bool full = K % 4096 == 0 && K <= 8192;
+  return M >= 3 && M <= 8 && !(M <= 4 && full);
+}
+
 int strata_q4_gemm_skinny(const void* x, int M, int K, const strata_q4_weight* ws, int count,
                           int y_dtype, void* stream, bool exact) {
   STRATA_REQUIRE(strata_q4_skinny_fits(M, K, ws, count),

@@ -126,6 +126,8 @@ inline bool strata_q4_sb_aligned(const strata_q4_weight& w) {
   return ((reinterpret_cast<uintptr_t>(w.scales) | reinterpret_cast<uintptr_t>(w.biases)) & 3) == 0;
 }
 bool strata_q4_skinny_fits(int M, int K, const strata_q4_weight* ws, int count);
+// Whether linears of M <= 8 rows run there, with exact set, and not on the GEMV.
+bool strata_q4_few_rows_on_mfma(int M, int K);
 // exact (M <= 16): weights not rounded to bf16, as in the GEMV.
 int strata_q4_gemm_skinny(const void* x, int M, int K, const strata_q4_weight* ws, int count,
                           int y_dtype, void* stream, bool exact = false);

@@ -406,3 +406,24 @@ def test_scales_at_odd_addresses(dev, M, K, ns):
             torch.cuda.synchronize()
             for y, r in zip(ys, ref):
                 assert float((y - r).norm() / r.norm()) <= bound
+
+
+@pytest.mark.parametrize("M,K,ns", [(4, 4096, (4096, 1024)), (3, 8192, (1024, 48)), (5, 8192, (1024, 48)),
+                                    (4, 4608, (256,)), (3, 12288, (64,)), (6, 1024, (320, 100, 64)),
+                                    (8, 512, (36, 16)), (4, 3584, (16384, 320))])
+def test_few_rows_either_kernel(dev, M, K, ns):
+    """3-8 rows on both sides of the choice between the GEMV (K that fills its
+    steps, up to 4 rows) and the MFMA kernel, and linears of one call on either
+    (N % 16 != 0: the GEMV): the weights' fp32 values against float64, and each
+    linear's bits as alone."""
+    from lokahi_amd import ops
+    gen = torch.Generator(device=dev).manual_seed(M * K)
+    x = torch.randn((M, K), generator=gen, device=dev).bfloat16()
+    ws = [ops.quantize(torch.randn((n, K), generator=gen, device=dev) * 0.02) for n in ns]
+    ys = ops.linear_multi(x, ws, out_dtype=torch.float32)
+    for (w, s, b), n, y in zip(ws, ns, ys):
+        codes = torch.stack([(w.view(torch.int32) >> (4 * i)) & 15 for i in range(8)], -1).view(n, K // 64, 64)
+        wd = (codes * s.double()[..., None] + b.double()[..., None]).view(n, K)
+        ref = x.double() @ wd.T
+        assert float((y - ref).norm() / ref.norm()) < 1e-5
+        assert torch.equal(ops.linear(x, w, s, b, out_dtype=torch.float32), y)
