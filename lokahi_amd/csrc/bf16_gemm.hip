@@ -237,21 +237,34 @@ int pick_tm(int M, int N, int cus) {
   return best;
 }
 
+// The GEMV reads all of W once per 4 rows (2 rows when M < 4), the GEMM once per
+// tile of up to 160 rows but walks K in ~0.7 us steps while its tiles leave CUs
+// idle.  So it wins from a number of passes x N that grows with K as a pass of the
+// GEMV gets cheaper per byte, up to K = 4096, where 64 lanes with 8 loads each
+// are full.  Microseconds, GEMV | this kernel, weights from HBM:
+//   rows, N:   8, 8192       16, 8192     32, 4096     3, 12288     64, 2048     8, 24576
+//   K = 1024   14.2 | 13.1   25.5 | 13.6  24.5 | 14.5  13.9 | 13.2  22.7 | 13.9   34.3 | 14.8
+//   K = 2048   18.4 | 23.4   32.6 | 24.0  32.4 | 25.6  18.0 | 23.5  29.2 | 24.5   44.8 | 26.6
+//   K = 4096   22.6 | 43.5   40.7 | 45.3  37.9 | 47.5  31.4 | 44.4  41.4 | 46.0   62.4 | 50.5
+//   K = 8192   50.3 | 84.5   94.0 | 86.8  94.4 | 89.4  63.3 | 78.9  95.1 | 86.6  136.4 | 94.1
+// (K = 6144, 8 rows of 8192: 40 | 82).  One 4-row pass loses to the GEMM on large
+// W only, and only where K leaves more than an eighth of the lanes' last step
+// empty: 128256 x 3072 146 | 138, x 3584 157 | 160, x 4096 168 | 182, x 6144 274 |
+// 269, x 8192 348 | 353; 32000 x 3072 41 | 46.
+bool gemm_wins(int M, int K, int N) {
+  if (M < 3) return false;
+  if (M == 4) return N >= 65536 && (int64_t)K * 8 < (int64_t)(K + 4095) / 4096 * 4096 * 7;
+  const int64_t passes = M > 4 ? (M + 3) / 4 : 2;
+  return passes * N >= (K <= 4096 ? 16384 + 6 * K : K < 8192 ? 40960 : 32768);
+}
+
 }  // namespace
 
 int strata_bf16_linear(strata_ctx* ctx, const void* x, int64_t ldx, int M, int K,
                        const uint16_t* w, int N, void* y, int y_dtype, void* stream) {
-  // The GEMV reads all of W once per 4 rows (2 rows when M < 4), the GEMM
-  // once per tile of up to 160 rows but walks K in ~0.45 us steps: it wins
-  // from passes * N ~ 24 Ki (4096 x 4096: 16 rows 21 against 29 us, 32 rows
-  // 36 against 33; 32000 x 2048: 8 rows 58 against 36).  One 4-row pass is
-  // as fast as the GEMM where its x rows are one load per thread (128256 x
-  // 4096: 165 against 171 us; 128256 x 3072: 142 against 131) and on fewer
-  // rows of W (32000 x 2048: 32 against 36).
   const bool fits = K % BK == 0 && ldx % 8 == 0 && (uint64_t)ldx * 160 * 2 + (uint64_t)K * 2 < (1ull << 32) &&
                     (uint64_t)K * TN * 2 < (1ull << 32);
-  const int64_t passes = M >= 4 ? (M + 3) / 4 : (M + 1) / 2;
-  bool gemm = fits && passes * N >= 24576 && (passes > 1 || (M == 4 && K != 4096 && N >= 65536));
+  bool gemm = fits && (gemm_wins(M, K, N) || !strata_bf16_gemv_fits(ctx, M, K));
   if (ldx != K && M > 1) gemm = fits;  // the GEMV takes contiguous rows
   if (gemm) {
     const uint16_t* xx = static_cast<const uint16_t*>(x);

@@ -19,11 +19,17 @@ int strata_q4_gemv(strata_ctx* ctx, const void* x, int x_dtype, int M, int K,
                           y_dtype);
 }
 
+static int bf16_gemv_rows(int M) { return M >= 4 ? 4 : (M >= 2 ? 2 : 1); }  // x rows per pass
+
+bool strata_bf16_gemv_fits(strata_ctx* ctx, int M, int K) {
+  return (int64_t)bf16_gemv_rows(M) * K * 2 <= ctx->max_lds_per_block;
+}
+
 int strata_bf16_gemv(strata_ctx* ctx, const void* x, int M, int K, const uint16_t* w, int N,
                      void* y, int y_dtype, void* stream) {
-  const int MT = M >= 4 ? 4 : (M >= 2 ? 2 : 1);
+  const int MT = bf16_gemv_rows(M);
   const size_t lds = (size_t)MT * K * 2;
-  STRATA_REQUIRE((int64_t)lds <= ctx->max_lds_per_block, "bf16 GEMV: K=%d too large", K);
+  STRATA_REQUIRE(strata_bf16_gemv_fits(ctx, M, K), "bf16 GEMV: K=%d too large", K);
   // 8 uint4 (64 weights) per lane per chunk, one row per wave, 8 waves per WG.
   constexpr int NW = 8, R = 1, U = 8;
   dim3 grid((N + NW * R - 1) / (NW * R), (M + MT - 1) / MT);

@@ -61,6 +61,7 @@ int strata_q4_gemv(strata_ctx* ctx, const void* x, int x_dtype, int M, int K,
                    const strata_q4_weight* ws, int count, int y_dtype, void* stream);
 int strata_bf16_gemv(strata_ctx* ctx, const void* x, int M, int K, const uint16_t* w, int N,
                      void* y, int y_dtype, void* stream);
+bool strata_bf16_gemv_fits(strata_ctx* ctx, int M, int K);  // its x rows fit in LDS
 // y[m] = x[m] @ w^T, x rows ldx elements apart.
 int strata_bf16_linear(strata_ctx* ctx, const void* x, int64_t ldx, int M, int K,
                        const uint16_t* w, int N, void* y, int y_dtype, void* stream);

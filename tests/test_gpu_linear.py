@@ -427,3 +427,22 @@ def test_few_rows_either_kernel(dev, M, K, ns):
         ref = x.double() @ wd.T
         assert float((y - ref).norm() / ref.norm()) < 1e-5
         assert torch.equal(ops.linear(x, w, s, b, out_dtype=torch.float32), y)
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 2559, 4096), (64, 2561, 4096), (12, 8192, 4096), (14, 10240, 4096),
+                                   (4, 65536, 1024), (4, 65535, 1024), (4, 65536, 4096), (3, 12288, 2048),
+                                   (16, 8192, 8192), (15, 8191, 8192), (8, 20480, 5120), (8, 20478, 5120),
+                                   (2, 100, 16384), (5, 100, 8256)])
+def test_bf16_dense_linear_either_kernel(dev, M, N, K):
+    """Both sides of the dense linear's choice between the GEMV and the MFMA
+    kernel (passes x columns by K, 4 rows, and K whose rows the GEMV's LDS does
+    not hold).  fp32 sums of exact bf16 products against float64: K terms at
+    2^-24 each."""
+    from lokahi_amd import ops
+    gen = torch.Generator(device=dev).manual_seed(M + N)
+    W = (torch.randn((N, K), generator=gen, device=dev) * 0.02).bfloat16()
+    x = torch.randn((M, K), generator=gen, device=dev).bfloat16()
+    ref = torch.cat([x.double() @ w.double().T for w in W.split(16384)], 1)
+    y = ops.linear(x, W, None, None, out_dtype=torch.float32)
+    assert float((y - ref).norm() / ref.norm()) < 1e-5
+    assert torch.equal(ops.linear(x, W, None, None), y.bfloat16())
