@@ -255,8 +255,9 @@ void set_lengths(strata_decoder* d, int len) {
 // Load-time re-layout of the prefill weights (the MLX layout stays the
 // interchange and decode format): for each layer the four GEMM launches of a
 // prefill, in the layout of q4_gemm_relayout_kernel, when prefills can reach
-// the 256-column MFMA kernel and every linear qualifies.  Costs one more copy of the
-// q4 linears; on an allocation failure the prefill re-lays out per call.
+// the 256-column MFMA kernel and every linear qualifies (up to 64 tokens only the
+// launches that leave the skinny kernel).  Costs one more copy of those linears;
+// on an allocation failure the prefill re-lays out per call.
 // STRATA_DECODER_NO_PREFILL_PACK (read per decoder creation) skips it:
 // prefills then re-lay out per call and the copy's memory is not held.
 int pack_prefill_weights(strata_decoder* d) {
@@ -280,6 +281,10 @@ int pack_prefill_weights(strata_decoder* d) {
           return STRATA_OK;  // this model's prefill re-lays out per call
         }
         N += w.N;
+      }
+      if (!strata_q4_gemm_packs(d->max_tokens, Ks[gi], groups[gi], counts[gi])) {
+        packed.push_back(GemmPacked{});
+        continue;
       }
       void* p = nullptr;
       if (hipMalloc(&p, strata_q4_gemm_mfma_scratch(N, Ks[gi])) != hipSuccess) {

@@ -60,6 +60,14 @@ int strata_q4_dequant_launch(const uint32_t* w, const uint16_t* s, const uint16_
   return STRATA_OK;
 }
 
+bool strata_q4_gemm_packs(int max_rows, int K, const strata_q4_weight* ws, int count) {
+  if (max_rows > kSkinnyMaxRows) return true;
+  if (max_rows < kMfmaMidRows) return false;
+  for (int i = 0; i < count; ++i)
+    if (ws[i].N < kMidWideN && strata_q4_skinny_shape(max_rows, K, &ws[i], 1)) return false;
+  return true;
+}
+
 int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const strata_q4_weight* ws,
                          int count, int y_dtype, void* stream, const GemmPacked* packed) {
   // Each linear goes its own way, so that it gives the same bits in a

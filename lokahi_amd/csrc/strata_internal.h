@@ -118,6 +118,8 @@ struct GemmPacked {
 };
 int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const strata_q4_weight* ws,
                          int count, int y_dtype, void* stream, const GemmPacked* packed = nullptr);
+// Whether some call of these linears with up to max_rows rows reads a re-layout.
+bool strata_q4_gemm_packs(int max_rows, int K, const strata_q4_weight* ws, int count);
 // Linears sharing x for a few rows (M <= kSkinnyMaxRows, K % 512 == 0, every
 // N % 16 == 0, 16-byte aligned weights and x, 4-byte aligned scales and
 // biases): one launch, each weight read once.

@@ -234,3 +234,33 @@ def test_engine_eight_row_decode_one_layout_launch(dev):
     op_logits = to_np_f32(model(seq[:, 40:41], past_key_values=c2, use_cache=True,
                                 logits="last")[:, -1])
     assert rel_err(eng_logits, op_logits) < 2e-2
+
+
+def test_engine_packs_only_what_its_prefills_read(dev):
+    """The load-time prefill layouts of an engine for up to 40 tokens: gate and
+    up (8192 columns, the MFMA kernel from 33 rows) are laid out, the narrow
+    linears (the skinny kernel up to 64 rows) are not, and the tokens are those
+    of the op-by-op path."""
+    from lokahi_amd.llama import DecoderEngine, HipLlamaForCausalLM, LlamaConfig, random_weights
+    cfg = LlamaConfig(vocab_size=512, hidden_size=2048, intermediate_size=8192, num_hidden_layers=8,
+                      num_attention_heads=32, num_key_value_heads=8)
+    model = HipLlamaForCausalLM(cfg, random_weights(cfg, 71))
+    q4 = lambda n, k: n * k // 2 + n * k // 64 * 4
+    wide, all_ = (8 * s for s in (q4(16384, 2048), q4(16384, 2048) + q4(3072, 2048) + q4(2048, 2048) + q4(2048, 8192)))
+
+    def held(tokens):
+        cache = model.new_cache(1, 64)
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        eng = DecoderEngine(model, cache, max_batch=1, max_tokens=tokens)
+        torch.cuda.synchronize()
+        return before - torch.cuda.mem_get_info()[0], eng, cache
+
+    none, _, _ = held(32)
+    few, eng, cache = held(40)
+    more, _, _ = held(65)
+    slack = 32 * 2**21  # 2 MiB pages, one allocation per layout
+    assert few - none < wide + slack and wide < more - none and all_ - slack < more - none
+    assert few - none > wide - slack
+    ids = torch.randint(0, 512, (1, 40), device=dev)
+    assert rel_err(to_np_f32(eng.forward(ids)), to_np_f32(model(ids, logits="last")[:, -1])) < 2e-2
