@@ -289,10 +289,10 @@ def test_prefill_key_splits(dev, dtype, B, Hq, Hkv, D, Lq, Lk, causal, given):
     """Prefill whose keys are split over workgroups (with the workspace ops
     passes) against float64, and against the call without a workspace.  Given
     positions include rows that see no key (0, as keys masked for every row
-    give), rows that end in the first split and repeats.  The weights of a
-    split are exact powers of two apart from one fp32 rounding each, so the
-    split result stays within the unsplit one's own distance from float64
-    (bf16: weights and outputs rounded at 2^-9; fp32: 2^-24 per sum term)."""
+    give), rows that end in the first split and repeats.  The merge weighs each
+    split's sums by one fp32 exp2 (2^-23 each), so the split result stays within
+    the unsplit one's own distance from float64 (bf16: weights and outputs
+    rounded at 2^-9; fp32: 2^-24 per sum term)."""
     import ctypes as C
     from lokahi_amd import _abi, ops
     dt = torch.bfloat16 if dtype == "bf16" else torch.float32
@@ -368,10 +368,11 @@ def test_prefill_few_rows_without_split(dev, dtype, B, Hq, Hkv, D, Lq, Lk, given
                                             (32, 8, 128, 700, 707), (8, 8, 128, 130, 1000),
                                             (32, 8, 128, 1100, 1100), (32, 8, 128, 3000, 3000)])
 def test_prefill_without_split(dev, Hq, Hkv, D, Lq, Lk):
-    """Unsplit bf16 prefill (no workspace): key tiles shared by two wave groups
-    of a workgroup (an odd and an even number of tiles, a last tile for one
-    group only), 64-key tiles, and the plain kernel, against float64 rows and
-    each row's independence of the others in its tile."""
+    """Unsplit bf16 prefill (no workspace), the shapes of a small batch: key tiles
+    shared by two wave groups of a workgroup (an odd and an even number of
+    tiles, a last tile for one group only) and, for the last shape, 64-key
+    tiles, against float64 rows; and each row's bits whatever the other rows
+    of its tile hold."""
     import ctypes as C
     from lokahi_amd import _abi, ops
     gen = torch.Generator(device=dev).manual_seed(Lq + D)
@@ -394,6 +395,84 @@ def test_prefill_without_split(dev, Hq, Hkv, D, Lq, Lk):
     ref = torch.matmul(torch.softmax(sc, -1), v.double().repeat_interleave(Hq // Hkv, 1))
     assert float((got[:, :, rows].double() - ref).norm() / ref.norm()) < 5e-3
     assert bool(got.isfinite().all())
+    keep = torch.arange(Lq, device=dev) % 3 != 1
+    other = torch.where(keep[:, None], q, 3 * torch.randn(q.shape, generator=gen, device=dev).bfloat16())
+    again = call(other)
+    assert torch.equal(again[:, :, keep], got[:, :, keep])
+    assert not torch.equal(again[:, :, ~keep], got[:, :, ~keep])
+
+
+@pytest.mark.parametrize("kernel,D", [("one wave", 128), ("one wave", 64), ("two waves", 64), ("two waves", 128),
+                                      ("plain", 128), ("plain", 64), ("64 keys", 64), ("64 keys", 128)])
+@pytest.mark.parametrize("mask", ["causal", "given", "none"])
+def test_prefill_unsplit_kernels_of_a_full_gpu(dev, kernel, D, mask):
+    """The unsplit bf16 kernels for more tiles than CUs, the batch sized from the
+    CU count: tiles of one and of two waves (up to 32 and 64 packed rows), the
+    plain four-wave kernel (over 5.5 tiles per CU) and 64-key tiles (between 2
+    and 4), causal, with given positions (rows that see no key, or all) and
+    without a mask.  The first, a middle and the last batch row against float64
+    (bf16 weights and outputs: 2^-9 each); rows keep their bits whatever the
+    other rows of their tile hold."""
+    import ctypes as C
+    from lokahi_amd import _abi, ops
+    cus, Hq, Hkv = torch.cuda.get_device_properties(0).multi_processor_count, 12, 4
+    Lq, Lk, tiles, per_cu = {"one wave": (10, 101, 1, 1), "two waves": (21, 201, 1, 1),
+                             "plain": (100, 164, 3, 6), "64 keys": (100, 164, 3, 3)}[kernel]
+    B = per_cu * cus // (tiles * Hkv) + 1
+    gen = torch.Generator(device=dev).manual_seed(D + Lq)
+    q, k, v = (torch.randn((B, h, l, D), generator=gen, device=dev).bfloat16()
+               for h, l in ((Hq, Lq), (Hkv, Lk), (Hkv, Lk)))
+    pos = torch.arange(Lk - Lq, Lk, device=dev, dtype=torch.int32).repeat(B, 1)
+    if mask == "given":
+        pos = torch.randint(0, Lk, (B, Lq), generator=gen, device=dev, dtype=torch.int32)
+        pos[:, 3], pos[:, 6] = -1, Lk - 1
+
+    def call(q):
+        out = torch.empty_like(q)
+        _abi.check(_abi.load().strata_attn_gqa(
+            ops._ctx(0), q.data_ptr(), ops._code(q), k.data_ptr(), ops._code(k), v.data_ptr(),
+            ops._code(v), Hkv * Lk * D, Lk * D, pos.data_ptr() if mask == "given" else None, B, Hq, Hkv, Lq,
+            Lk, D, int(mask != "none"), 32768, 1024, C.c_float(1e-12), out.data_ptr(), ops._stream(0)))
+        return out
+
+    got = call(q)
+    rows = torch.tensor([0, B // 2, B - 1], device=dev)
+    sc = torch.matmul(q[rows].double(),
+                      k[rows].double().repeat_interleave(Hq // Hkv, 1).transpose(2, 3).contiguous()) / D**0.5
+    w = torch.exp(sc - sc.amax(-1, keepdim=True))
+    if mask != "none":
+        w = w * (torch.arange(Lk, device=dev) <= pos[rows][:, None, :, None])
+    ref = torch.matmul(w, v[rows].double().repeat_interleave(Hq // Hkv, 1)) / w.sum(-1, keepdim=True).clamp_min(1e-12)
+    assert float((got[rows].double() - ref).norm() / ref.norm()) < 5e-3
+    assert bool(got.isfinite().all())
+    keep = torch.arange(Lq, device=dev) % 3 != 1
+    again = call(torch.where(keep[:, None], q, 3 * torch.randn(q.shape, generator=gen, device=dev).bfloat16()))
+    assert torch.equal(again[:, :, keep], got[:, :, keep])
+
+
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,D,Lq,Lk", [("bf16", 1, 32, 8, 128, 100, 4100), ("bf16", 3, 6, 2, 64, 30, 1500),
+                                                    ("f32", 1, 8, 2, 64, 200, 712), ("f32", 2, 6, 2, 128, 37, 437)])
+def test_prefill_key_splits_over_cache_views(dev, dtype, B, Hq, Hkv, D, Lq, Lk):
+    """Split prefill over K and V that are views into a longer cache, whose slots
+    past the keys hold NaN: the bits of the call on contiguous copies."""
+    import ctypes as C
+    from lokahi_amd import _abi, ops
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    gen = torch.Generator(device=dev).manual_seed(Lq + Lk)
+    lmax = Lk + 177
+    q = torch.randn((B, Hq, Lq, D), generator=gen, device=dev).to(dt)
+    kc, vc = (torch.full((B, Hkv, lmax, D), float("nan"), device=dev, dtype=dt) for _ in range(2))
+    k, v = kc[:, :, :Lk], vc[:, :, :Lk]
+    for t in (k, v):
+        t.copy_(torch.randn((B, Hkv, Lk, D), generator=gen, device=dev))
+    need = C.c_int64()
+    _abi.check(_abi.load().strata_attn_workspace(ops._ctx(0), ops._code(q), ops._code(k), ops._code(v),
+                                                 B, Hq, Hkv, Lq, Lk, D, 1, C.byref(need)))
+    assert need.value > 0  # the call is split
+    pos = torch.arange(Lk - Lq, Lk, device=dev, dtype=torch.int32)
+    got = ops.attention(q, k, v, query_positions=pos, kv_strides=(Hkv * lmax * D, lmax * D))
+    ref = ops.attention(q, k.contiguous(), v.contiguous(), query_positions=pos)
+    assert torch.equal(got, ref) and bool(got.isfinite().all())
 
 
 @pytest.mark.parametrize("dtype,B,Hq,Hkv,D,Lq,Lk,split", [

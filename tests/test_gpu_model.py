@@ -264,3 +264,38 @@ def test_engine_packs_only_what_its_prefills_read(dev):
     assert few - none > wide - slack
     ids = torch.randint(0, 512, (1, 40), device=dev)
     assert rel_err(to_np_f32(eng.forward(ids)), to_np_f32(model(ids, logits="last")[:, -1])) < 2e-2
+
+
+@pytest.mark.parametrize("B,past,new", [(1, 8000, 3000), (2, 8000, 1000), (4, 2000, 150), (1, 4000, 100)])
+def test_engine_prefill_over_a_history_splits_keys(dev, B, past, new):
+    """Prefill over a long cached history in the engine, whose attention splits
+    its keys in the engine's own workspace and merges them token-major: the
+    second layer's new keys and values (every row of the first layer's
+    attention is behind them) and the logits against the op-by-op path
+    (head-major attention, compared with float64 in test_gpu_attention.py) to
+    the bf16 flow's tolerance."""
+    import ctypes as C
+    from lokahi_amd import _abi, ops
+    from lokahi_amd.llama import DecoderEngine, HipLlamaForCausalLM, LlamaConfig, random_weights
+    cfg = LlamaConfig(vocab_size=512, hidden_size=3072, intermediate_size=1024, num_hidden_layers=2,
+                      num_attention_heads=24, num_key_value_heads=8)
+    model = HipLlamaForCausalLM(cfg, random_weights(cfg, 73, std=0.03))
+    need = C.c_int64()
+    _abi.check(_abi.load().strata_attn_workspace(ops._ctx(0), _abi.BF16, _abi.BF16, _abi.BF16, B, 24, 8, new,
+                                                 past + new, 128, 1, C.byref(need)))
+    assert need.value > 0  # the call is split
+    gen = torch.Generator(device=dev).manual_seed(past + new)
+    caches = [model.new_cache(B, past + new + 8) for _ in range(2)]
+    for layer in range(2):  # a history that both paths share
+        k, v = (torch.randn((B, 8, past, 128), generator=gen, device=dev).bfloat16() for _ in range(2))
+        for c in caches:
+            c.update(k, v, layer)
+    ids = torch.randint(0, 512, (B, new), generator=gen, device=dev)
+    eng = DecoderEngine(model, caches[0], max_batch=B, max_tokens=B * new)
+    a = to_np_f32(eng.forward(ids))
+    b = to_np_f32(model(ids, past_key_values=caches[1], use_cache=True, logits="last")[:, -1])
+    assert rel_err(a, b) < 2e-2
+    for name in ("k_storage", "v_storage"):
+        x, y = (getattr(c, name)[1][:, :, past:past + new].float() for c in caches)
+        err = (x - y).norm(dim=(1, 3)) / y.norm(dim=(1, 3))  # per row and token
+        assert float(err.max()) < 2e-2
