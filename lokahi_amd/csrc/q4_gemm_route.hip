@@ -124,7 +124,7 @@ int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const str
   if (al + pk + pb > 0) {
     const int rc = strata_ctx_scratch(ctx, al + pk + pb, &scr, stream);
     if (rc && M > kSkinnyMaxRows) return rc;
-    // A short call never depends on scratch (the arena cannot grow under
+    // A short call is not refused for scratch (the arena cannot grow under
     // stream capture): K whole instead of in slices, the 128 x 128 kernel
     // instead of a copy.
     have = rc == STRATA_OK;

@@ -98,11 +98,13 @@ int strata_q4_gemm_mfma_run(const void* x, int M, int K, const void* packed,
 size_t strata_q4_gemm_mfma_part_bytes(int M, int K, const strata_q4_weight* ws, int count);
 // From this many rows a linear of at least kMidWideN columns (a multiple of
 // 256) goes to the 256-column MFMA kernel; narrower ones from one row past
-// the skinny kernel's 64.  Skinny against MFMA kernel: 8B gate/up at 32 rows 36
-// against 42 us, at 39 rows 60 against 42; 3B gate/up 17.6 against 25 and 30
-// against 25.5; at 64 rows q/k/v 20.4 against 22.3 (8B) and 17.1 against 20.3
-// (3B), down 30.9 against 30.7 and 17.5 against 24.7.
-constexpr int kMfmaMidRows = 33;
+// the skinny kernel's 64.  Below 40 rows a call shares nothing with calls on
+// other streams: the MFMA kernel's K slices meet in the context's scratch arena,
+// and without them it is slow (8B gate/up at 39 rows, weights from HBM: skinny 46
+// us, MFMA 43, K whole 57; 3B gate/up 20, 26, 46; 8192 x 8192 36, 33, 104).
+// Skinny against MFMA kernel at 64 rows: q/k/v 20.4 against 22.3 us (8B) and 17.1
+// against 20.3 (3B), down 30.9 against 30.7 and 17.5 against 24.7.
+constexpr int kMfmaMidRows = 40;
 constexpr int kMidWideN = 8192;
 // Rows up to which a call without a load-time re-layout reads the MLX tensors.
 constexpr int kMlxMaxRows = 512;

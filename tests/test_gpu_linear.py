@@ -346,6 +346,42 @@ def test_short_prefill_needs_no_scratch(dev, M, K, ns):
                 assert float((y - yw).norm() / yw.norm()) < 1e-5
 
 
+@pytest.mark.parametrize("M,K,ns", [(9, 512, (16384, 48)), (33, 4096, (14336, 14336)), (39, 8192, (8192,)),
+                                    (34, 1024, (8192, 8192, 256)), (36, 192, (8192,)), (39, 640, (256, 512))])
+def test_short_prefill_shares_no_memory(dev, M, K, ns):
+    """Up to 39 rows a call keeps nothing in memory that calls on other streams
+    use: the same bits with a context that has no scratch and cannot get any (a
+    captured call), and from two streams at once."""
+    import ctypes as C
+    from lokahi_amd import _abi, ops
+    gen = torch.Generator(device=dev).manual_seed(M + K)
+    ws = [ops.quantize(torch.randn((n, K), generator=gen, device=dev) * 0.02) for n in ns]
+    xs = torch.randn((2, M, K), generator=gen, device=dev).bfloat16()
+    refs = [ops.linear_multi(x, ws, out_dtype=torch.float32) for x in xs]
+    ctx = _abi.Context(0)
+    ys = [torch.empty_like(y) for y in refs[0]]
+    arr = (_abi.Q4Weight * len(ns))(*[_abi.Q4Weight(w.data_ptr(), s.data_ptr(), b.data_ptr(), n, y.data_ptr())
+                                      for (w, s, b), n, y in zip(ws, ns, ys)])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rc = _abi.load().strata_linear_q4_multi(ctx.handle, xs.data_ptr(), _abi.BF16, M, K, arr, len(ns), 64, 4,
+                                                _abi.F32, ops._raw_stream(0))
+    _abi.check(rc)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, r) for y, r in zip(ys, refs[0]))
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = [[], []]
+    for _ in range(20):
+        for i, stream in enumerate(streams):
+            with torch.cuda.stream(stream):
+                outs[i].append(ops.linear_multi(xs[i], ws, out_dtype=torch.float32))
+    torch.cuda.synchronize()
+    for got, ref in zip(outs, refs):
+        assert all(torch.equal(y, r) for g in got for y, r in zip(g, ref))
+
+
 def test_few_rows_beyond_32_bit_offsets(dev):
     """x of 4 GiB (64 rows): byte offsets that 32 bits do not hold.  x is zero
     but for a few columns, so the reference needs only those."""

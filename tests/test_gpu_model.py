@@ -238,7 +238,7 @@ def test_engine_eight_row_decode_one_layout_launch(dev):
 
 def test_engine_packs_only_what_its_prefills_read(dev):
     """The load-time prefill layouts of an engine for up to 40 tokens: gate and
-    up (8192 columns, the MFMA kernel from 33 rows) are laid out, the narrow
+    up (8192 columns, the MFMA kernel from 40 rows) are laid out, the narrow
     linears (the skinny kernel up to 64 rows) are not, and the tokens are those
     of the op-by-op path."""
     from lokahi_amd.llama import DecoderEngine, HipLlamaForCausalLM, LlamaConfig, random_weights
