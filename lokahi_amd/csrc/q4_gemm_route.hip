@@ -64,7 +64,7 @@ bool strata_q4_gemm_packs(int max_rows, int K, const strata_q4_weight* ws, int c
   if (max_rows > kSkinnyMaxRows) return true;
   if (max_rows < kMfmaMidRows) return false;
   for (int i = 0; i < count; ++i)
-    if (ws[i].N < kMidWideN && strata_q4_skinny_shape(max_rows, K, &ws[i], 1)) return false;
+    if (ws[i].N < kMidWideN && strata_q4_skinny_fits(max_rows, K, &ws[i], 1)) return false;
   return true;
 }
 
@@ -84,18 +84,15 @@ int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const str
   strata_q4_weight fast[kMaxGemmProblems], few[kMaxGemmProblems];
   int nfast = 0, nfew = 0;
   int64_t Nfast = 0;
-  size_t al = 0;  // bytes of scales and biases that the skinny kernel cannot load where they are
   auto tile128 = [&](const strata_q4_weight& w) {
     return strata_q4_gemm_launch(x, M, K, w.w, w.scales, w.biases, (int)w.N, w.y, y_dtype, stream);
   };
-  auto sb_bytes = [&](const strata_q4_weight& w) { return ((size_t)w.N * (K / 64) * 2 + 255) / 256 * 256; };
   for (int i = 0; i < count; ++i) {
     const bool mid = M >= kMfmaMidRows && x_ok && ws[i].N % 256 == 0 && aligned16(ws[i].w) &&
                      (uint64_t)(Nfast + ws[i].N) * K / 2 < (1ull << 32) && nfast < kMaxGemmProblems;
-    const bool skinny = M <= kSkinnyMaxRows && aligned16(x) && strata_q4_skinny_shape(M, K, &ws[i], 1) &&
+    const bool skinny = M <= kSkinnyMaxRows && aligned16(x) && strata_q4_skinny_fits(M, K, &ws[i], 1) &&
                         nfew < kMaxGemmProblems;
     if (skinny && !(mid && ws[i].N >= kMidWideN)) {
-      if (!strata_q4_sb_aligned(ws[i])) al += 2 * sb_bytes(ws[i]);
       few[nfew++] = ws[i];
     } else if (mid) {
       fast[nfast++] = ws[i];
@@ -105,6 +102,11 @@ int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const str
       if (rc) return rc;
     }
   }
+  if (nfew > 0) {
+    const int rc = strata_q4_gemm_skinny(x, M, K, few, nfew, y_dtype, stream);
+    if (rc) return rc;
+  }
+  if (nfast == 0) return STRATA_OK;
   // The decoder's load-time re-layout is used when it was built for exactly
   // these linears (all of them on this path, the same total N and K);
   // otherwise this call re-lays the weights out into the scratch arena,
@@ -113,53 +115,23 @@ int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const str
                               packed->K == K && packed->count == count
                           ? packed->buf
                           : nullptr;
-  size_t pb = nfast ? strata_q4_gemm_mfma_part_bytes(M, K, fast, nfast) : 0;
+  size_t pb = strata_q4_gemm_mfma_part_bytes(M, K, fast, nfast);
   // Up to kMlxMaxRows rows the kernel reads the linears' own tensors instead
   // (the same bits): the re-layout takes as long as the GEMM gains (8B gate/up:
   // 128 rows 77 -> 53 us, 512 rows 139 -> 138, 1000 rows 243 against 267).
   const bool mlx = !pk_in && M <= kMlxMaxRows && strata_q4_gemm_mlx_fits(K, fast, nfast);
-  size_t pk = pk_in || mlx || !nfast ? 0 : (strata_q4_gemm_mfma_scratch(Nfast, K) + 255) / 256 * 256;
+  const size_t pk = pk_in || mlx ? 0 : (strata_q4_gemm_mfma_scratch(Nfast, K) + 255) / 256 * 256;
   void* scr = nullptr;
   bool have = true;
-  if (al + pk + pb > 0) {
-    const int rc = strata_ctx_scratch(ctx, al + pk + pb, &scr, stream);
+  if (pk + pb > 0) {
+    const int rc = strata_ctx_scratch(ctx, pk + pb, &scr, stream);
     if (rc && M > kSkinnyMaxRows) return rc;
     // A short call is not refused for scratch (the arena cannot grow under
     // stream capture): K whole instead of in slices, the 128 x 128 kernel
-    // instead of a copy.
+    // instead of a re-layout.
     have = rc == STRATA_OK;
     if (!have) (void)hipGetLastError();
   }
-  if (nfew > 0) {
-    // Scales and biases at odd 2-byte addresses are copied for the skinny
-    // kernel's 4-byte loads (3072 x 8192, 24 rows: 18 us with the copies, 181
-    // on the 128 x 128 kernel, 14 aligned).
-    char* at = static_cast<char*>(scr);
-    strata_q4_weight run[kMaxGemmProblems];
-    int nrun = 0;
-    for (int i = 0; i < nfew; ++i) {
-      strata_q4_weight w = few[i];
-      if (!strata_q4_sb_aligned(w)) {
-        if (!have) {
-          const int rc = tile128(w);
-          if (rc) return rc;
-          continue;
-        }
-        const size_t bytes = (size_t)w.N * (K / 64) * 2;
-        for (const uint16_t** t : {&w.scales, &w.biases}) {
-          STRATA_HIP_CHECK(hipMemcpyAsync(at, *t, bytes, hipMemcpyDeviceToDevice, as_stream(stream)));
-          *t = reinterpret_cast<const uint16_t*>(at);
-          at += sb_bytes(w);
-        }
-      }
-      run[nrun++] = w;
-    }
-    if (nrun > 0) {
-      const int rc = strata_q4_gemm_skinny(x, M, K, run, nrun, y_dtype, stream);
-      if (rc) return rc;
-    }
-  }
-  if (nfast == 0) return STRATA_OK;
   if (!have && pk) {
     for (int i = 0; i < nfast; ++i) {
       const int rc = tile128(fast[i]);
@@ -168,13 +140,12 @@ int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const str
     return STRATA_OK;
   }
   if (!have) pb = 0;
-  char* own = static_cast<char*>(scr) + al;
   if (pk) {
-    const int rc = strata_q4_gemm_pack(fast, nfast, K, own, stream);
+    const int rc = strata_q4_gemm_pack(fast, nfast, K, scr, stream);
     if (rc) return rc;
-    pk_in = own;
+    pk_in = scr;
   }
-  float* part = pb ? reinterpret_cast<float*>(own + pk) : nullptr;
+  float* part = pb ? reinterpret_cast<float*>(static_cast<char*>(scr) + pk) : nullptr;
   return strata_q4_gemm_mfma_run(x, M, K, pk_in, fast, nfast, y_dtype, stream, part, pb);
 }
 

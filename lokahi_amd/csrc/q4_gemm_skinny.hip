@@ -116,14 +116,17 @@ __global__ __launch_bounds__(256) void q4_gemm_skinny_kernel(const uint16_t* __r
   for (int i = 0; i < 4; ++i) xv[i] = kq * xb + ((c ^ (4 * i + kq)) << 4);
   // a weight load fills 16 rows: slot q of row r holds piece q ^ (r / 4 % 4)
   const uint32_t wv = (lane >> 2) * wb + (((lane & 3) ^ ((lane >> 4) & 3)) << 4);
-  const uint32_t sv = c * sb;  // the pair of groups of the chunk
+  // the chunk's first group for kq < 2, its second for the others; 2-byte loads,
+  // as scales and biases may start at any 2-byte address (as fast as the pairs in
+  // 4-byte loads: 28672 x 4096, 24 rows 40 us, 5 rows 31)
+  const uint32_t sv = c * sb + (kq >> 1) * 2;
   auto issue = [&](int ch, int st) {
     const uint32_t k = kbeg + (ch << 7), base = lds0 + st * S::kBytes;
 #pragma unroll
     for (int cc = 0; cc < NC; ++cc) {
       dma16(base + S::kX + cc * 1024, wv, rw, 16 * cc * wb + k / 2);
-      dma4(base + S::kX + S::kW + cc * 512, sv, rs, 16 * cc * sb + k / 32);
-      dma4(base + S::kX + S::kW + cc * 512 + 256, sv, rb, 16 * cc * sb + k / 32);
+      dma2(base + S::kX + S::kW + cc * 512, sv, rs, 16 * cc * sb + k / 32);
+      dma2(base + S::kX + S::kW + cc * 512 + 256, sv, rb, 16 * cc * sb + k / 32);
     }
 #pragma unroll
     for (int i = 0; i < MB * 4; ++i) dma16(base + i * 1024, xv[i & 3], rx, 4 * i * xb + k * 2);
@@ -148,11 +151,14 @@ __global__ __launch_bounds__(256) void q4_gemm_skinny_kernel(const uint16_t* __r
       static_assert(MB == 1, "one block of rows");
       const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
       uint4 xp[4];  // k 32 s + 8 kq .. +7 in the order 0 4 1 5 2 6 3 7
-      uint32_t wd[NC][4], sr[NC], br[NC];
+      uint32_t wd[NC][4], sr[NC][2], br[NC][2];
 #pragma unroll
       for (int cc = 0; cc < NC; ++cc) {
-        sr[cc] = *reinterpret_cast<const uint32_t*>(sg + S::kX + S::kW + cc * 512 + lane * 4);
-        br[cc] = *reinterpret_cast<const uint32_t*>(sg + S::kX + S::kW + cc * 512 + 256 + lane * 4);
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          sr[cc][g] = *reinterpret_cast<const uint32_t*>(sg + S::kX + S::kW + cc * 512 + (32 * g + c) * 4);
+          br[cc][g] = *reinterpret_cast<const uint32_t*>(sg + S::kX + S::kW + cc * 512 + 256 + (32 * g + c) * 4);
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           wd[cc][j] = *reinterpret_cast<const uint32_t*>(sg + S::kX + cc * 1024 + c * 64 +
@@ -175,8 +181,7 @@ __global__ __launch_bounds__(256) void q4_gemm_skinny_kernel(const uint16_t* __r
               mfma16x32(xp[j], make_uint4((w & 0x000f000fu) | 0x43004300u, ((w >> 4) & 0x000f000fu) | 0x43004300u,
                                           ((w >> 8) & 0x000f000fu) | 0x43004300u,
                                           ((w >> 12) & 0x000f000fu) | 0x43004300u), zero);
-          const float s = __uint_as_float(j >= 2 ? sr[cc] & 0xffff0000u : sr[cc] << 16);
-          const float b = __uint_as_float(j >= 2 ? br[cc] & 0xffff0000u : br[cc] << 16);
+          const float s = __uint_as_float(sr[cc][j >> 1] << 16), b = __uint_as_float(br[cc][j >> 1] << 16);
           const float cb = fmaf(-128.f, s, b);
 #pragma unroll
           for (int r = 0; r < 4; ++r) acc[0][cc][r] = fmaf(cb, xs[r], fmaf(s, d[r], acc[0][cc][r]));
@@ -198,9 +203,7 @@ __global__ __launch_bounds__(256) void q4_gemm_skinny_kernel(const uint16_t* __r
         xr[mb][j] = *reinterpret_cast<const uint4*>(sg + (16 * mb + c) * 256 + (((4 * kq + j) ^ c) << 4));
 #pragma unroll
     for (int cc = 0; cc < NC; ++cc) {
-      // the lane's group is the pair's first (kq < 2) or second
-      const float s = __uint_as_float(kq < 2 ? sr[cc] << 16 : sr[cc] & 0xffff0000u);
-      const float b = __uint_as_float(kq < 2 ? br[cc] << 16 : br[cc] & 0xffff0000u);
+      const float s = __uint_as_float(sr[cc] << 16), b = __uint_as_float(br[cc] << 16);
       const uint32_t ww[4] = {wr[cc].x, wr[cc].y, wr[cc].z, wr[cc].w};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -264,20 +267,13 @@ void launch_skinny(const uint16_t* x, int M, int K, const SkinnyBatch& bt, int c
 
 }  // namespace
 
-bool strata_q4_skinny_shape(int M, int K, const strata_q4_weight* ws, int count) {
+bool strata_q4_skinny_fits(int M, int K, const strata_q4_weight* ws, int count) {
   if (M < 1 || M > kSkinnyMaxRows || K % 512 != 0 || count < 1 || count > kMaxGemmProblems)
     return false;
   // byte offsets into x and into a workgroup's up to 64 weight rows are 32-bit
   if ((uint64_t)M * K * 2 >= (1ull << 32) || (uint64_t)64 * K / 2 >= (1ull << 32)) return false;
   for (int i = 0; i < count; ++i)
     if (ws[i].N % 16 != 0 || !aligned16(ws[i].w)) return false;
-  return true;
-}
-
-bool strata_q4_skinny_fits(int M, int K, const strata_q4_weight* ws, int count) {
-  if (!strata_q4_skinny_shape(M, K, ws, count)) return false;
-  for (int i = 0; i < count; ++i)
-    if (!strata_q4_sb_aligned(ws[i])) return false;
   return true;
 }
 

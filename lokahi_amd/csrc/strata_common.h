@@ -43,6 +43,11 @@ __device__ __forceinline__ void dma4(uint32_t lds, uint32_t voff, v4i32_t r, uin
   asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds"
                :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory", "m0");
 }
+// 2 bytes per lane, to the low half of the lane's 4-byte slot.
+__device__ __forceinline__ void dma2(uint32_t lds, uint32_t voff, v4i32_t r, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_ushort %1, %2, %3 offen lds"
+               :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory", "m0");
+}
 
 // ---------------------------------------------------------------- bf16 <-> f32
 // bf16 values travel as uint16_t bit patterns (upper half of an IEEE f32).

@@ -123,10 +123,8 @@ int strata_q4_gemm_multi(strata_ctx* ctx, const void* x, int M, int K, const str
 // Whether some call of these linears with up to max_rows rows reads a re-layout.
 bool strata_q4_gemm_packs(int max_rows, int K, const strata_q4_weight* ws, int count);
 // Linears sharing x for a few rows (M <= kSkinnyMaxRows, K % 512 == 0, every
-// N % 16 == 0, 16-byte aligned weights and x, 4-byte aligned scales and
-// biases): one launch, each weight read once.
+// N % 16 == 0, 16-byte aligned weights and x): one launch, each weight read once.
 constexpr int kSkinnyMaxRows = 64;
-bool strata_q4_skinny_shape(int M, int K, const strata_q4_weight* ws, int count);  // but for scales and biases
 inline bool strata_q4_sb_aligned(const strata_q4_weight& w) {
   return ((reinterpret_cast<uintptr_t>(w.scales) | reinterpret_cast<uintptr_t>(w.biases)) & 3) == 0;
 }

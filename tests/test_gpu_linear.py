@@ -346,16 +346,25 @@ def test_short_prefill_needs_no_scratch(dev, M, K, ns):
                 assert float((y - yw).norm() / yw.norm()) < 1e-5
 
 
-@pytest.mark.parametrize("M,K,ns", [(9, 512, (16384, 48)), (33, 4096, (14336, 14336)), (39, 8192, (8192,)),
+@pytest.mark.parametrize("M,K,ns", [(5, 1536, (320, 48)), (9, 512, (16384, 48)), (33, 4096, (14336, 14336)), (39, 8192, (8192,)),
                                     (34, 1024, (8192, 8192, 256)), (36, 192, (8192,)), (39, 640, (256, 512))])
-def test_short_prefill_shares_no_memory(dev, M, K, ns):
+@pytest.mark.parametrize("offset", [0, 1])
+def test_short_prefill_shares_no_memory(dev, M, K, ns, offset):
     """Up to 39 rows a call keeps nothing in memory that calls on other streams
     use: the same bits with a context that has no scratch and cannot get any (a
-    captured call), and from two streams at once."""
+    captured call), and from two streams at once; also with scales and biases
+    that start 2 bytes past a 4-byte boundary."""
     import ctypes as C
     from lokahi_amd import _abi, ops
     gen = torch.Generator(device=dev).manual_seed(M + K)
     ws = [ops.quantize(torch.randn((n, K), generator=gen, device=dev) * 0.02) for n in ns]
+
+    def moved(t):
+        buf = torch.empty(t.numel() + offset, dtype=t.dtype, device=dev)
+        buf[offset:] = t.flatten()
+        return buf[offset:].view(t.shape)
+
+    ws = [(w, moved(s), moved(b)) for w, s, b in ws]
     xs = torch.randn((2, M, K), generator=gen, device=dev).bfloat16()
     refs = [ops.linear_multi(x, ws, out_dtype=torch.float32) for x in xs]
     ctx = _abi.Context(0)
