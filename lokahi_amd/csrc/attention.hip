@@ -746,7 +746,7 @@ __device__ __forceinline__ f32x16_t mfma32_bf16(const bf16x8_t& a, const bf16x8_
 // SIMD; the P^T operand is the S^T accumulator itself (no shuffles).
 // K and V tiles (KT keys) are streamed by direct global -> LDS loads into a
 // ring of two stages, row-major with XOR-swizzled 16-byte chunks: the loads
-// of tile t + NST - 1 are issued at the top of tile t, and no register holds
+// of tile t + 1 are issued at the top of tile t, and no register holds
 // them.  V^T operands come from row-major V through the LDS transpose read
 // (ds_read_b64_tr_b16: in each 16-lane group, lane l' receives element
 // (l' & 3) of the 4-element rows addressed by lanes 4k + (l' >> 2), k < 4).
@@ -770,7 +770,6 @@ void attn_prefill_mfma32(
   constexpr int STAGE = 2 * TILE;     // K tile, then V tile
   constexpr int NST = 2;              // stages of a ring
   constexpr int RING = NST * STAGE;
-  constexpr int AHEAD = NST - 1;      // tiles in flight ahead of the one computed
   constexpr int QR = 32 * NW;         // query rows per workgroup
   constexpr int NI = KT * NCHK / (64 * NW);  // 16-byte loads per thread per tile and operand
   static_assert(NI >= 1 && KT * NCHK % (64 * NW) == 0, "tile loads must divide over the workgroup");
@@ -886,26 +885,17 @@ void attn_prefill_mfma32(
     v_off[db] = TILE + v_key * ROW + 16 * ((col / 8) ^ fv(v_key)) + 2 * (col % 8);
   }
 
-  // Wait until at most n tiles' loads (2 NI each) of this thread are in flight.
-  auto wait_tiles = [&](int n) {
-    if (n <= 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    else if (n == 1) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * NI) : "memory");
-    else if (n == 2) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(4 * NI) : "memory");
-    else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(6 * NI) : "memory");
-  };
-  static_assert(AHEAD <= 3, "wait_tiles covers up to three tiles in flight");
   // this wave's tiles: ks_id, ks_id + KS, ... of the nt_all
   const int nt_all = (kend - kbeg + KT - 1) / KT;
   const int nt = (nt_all - ks_id + KS - 1) / KS, steps = (nt_all + KS - 1) / KS;
-  // prologue: tiles 0 .. AHEAD - 1 in flight, tile 0 complete
-  wait_tiles(0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // tile 0 is complete
   __syncthreads();
   // one tile on stage ST (a compile-time constant, so every LDS address is a
   // lane offset plus an immediate)
   auto tile = [&](int t, auto STC) {
     constexpr int ST = decltype(STC)::value;
     const int kb0 = kbeg + (t * KS + ks_id) * KT;
-    if (t + AHEAD < nt) issue(kb0 + AHEAD * KS * KT, (ST + AHEAD) % NST);  // the stage tile t - 1 used
+    if (t + 1 < nt) issue(kb0 + KS * KT, ST ^ 1);  // the stage tile t - 1 used
     const uint8_t* ks = lds + ST * STAGE;
     // Waves whose rows see no key of the tile skip its math (one scalar
     // branch); rows of a live wave that see none are masked to p = 0.
@@ -1003,7 +993,7 @@ void attn_prefill_mfma32(
     }
     // tile t + 1 complete in this thread (later tiles' loads may remain in
     // flight), then in every thread
-    wait_tiles(min(nt - 1, t + AHEAD) - (t + 1));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // tile t + 1 is complete
     __syncthreads();
   };
   for (int t = 0; t < steps; t += NST) {
