@@ -71,8 +71,8 @@ int strata_selftest(strata_ctx* ctx, char* json, size_t cap);
  * Rejects bits != 4, group_size != 64, K % group_size != 0 with STRATA_EINVAL
  * (mode is always "affine"). M <= 8 keeps the weights' fp32 values; larger M
  * (bf16 x only) runs the fused-dequant bf16 MFMA GEMMs (weights rounded to
- * bf16), which use the context's scratch arena for the call: issue large-M
- * calls of one ctx on one stream (or order the streams). */
+ * bf16).  From 40 rows these use the context's scratch arena for the call:
+ * issue such calls of one ctx on one stream (or order the streams). */
 int strata_linear_q4(strata_ctx* ctx, const void* x, int x_dtype, int64_t M, int64_t K,
                      const uint32_t* w, const uint16_t* scales, const uint16_t* biases,
                      int64_t N, int group_size, int bits, void* y, int y_dtype,
