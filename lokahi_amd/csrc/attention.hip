@@ -466,17 +466,24 @@ void launch_decode_merge(const float* part, int nsplit, int D, int rows, float e
 // tiles first (measured 1.5x on the bf16 two-block kernel at 8k causal), so
 // with 8 KV heads an XCD works on one head of one b at a time, whose K/V tiles
 // stay in its L2 (groups of four consecutive tiles: 0-2% slower, 8k causal 561
-// against 555 us; a serpentine order over 32 CUs: 0-5% slower).  Returns false
-// for the padding of the grid.
+// against 555 us; a serpentine order over 32 CUs: 0-5% slower).  by_head (fp32,
+// tiles of about one length, B * Hkv a multiple of 8): an XCD takes all tiles of
+// one head of one b before the next, as with many b the heads at work at once
+// exceed its L2 (32 x 128 queries after 1000 keys, 32 heads: 1163 -> 1022 us; 32 x
+// 500 unmasked 1964 -> 1880; the bf16 kernels lose by it, 8 x 300 after 6000 282
+// -> 346).  Returns false for the padding of the grid.
 constexpr int kXcds = 8;
 __host__ __device__ inline int prefill_grid(int nqt, int B, int Hkv) {
   return (nqt * B * Hkv + kXcds - 1) / kXcds * kXcds;
 }
-__device__ inline bool prefill_item(int wg, int nqt, int B, int Hkv, int* qt, int* b, int* hkv) {
+__device__ inline bool prefill_item(int wg, bool by_head, int nqt, int B, int Hkv, int* qt, int* b,
+                                    int* hkv) {
   const int per = B * Hkv;
   if (wg >= nqt * per) return false;
-  *qt = nqt - 1 - wg / per;
-  const int rest = wg % per;
+  const int slot = wg / kXcds, head = slot / nqt;
+  const int t = by_head ? slot - head * nqt : wg / per;
+  *qt = nqt - 1 - t;
+  const int rest = by_head ? head * kXcds + wg % kXcds : wg - t * per;
   *b = rest / Hkv;
   *hkv = rest % Hkv;
   return true;
@@ -490,6 +497,7 @@ __device__ inline bool prefill_item(int wg, int nqt, int B, int Hkv, int* qt, in
 struct PrefillSplit {
   int nsplit, chunk;
   int rows;  // packed query rows per tile (fp32 kernel: 16, 32 or 64)
+  int by_head;  // order of the tiles (fp32 kernel, prefill_item)
   float* o;
   float2* ms;
 };
@@ -572,7 +580,7 @@ __global__ __launch_bounds__(256) void attn_prefill_f32(
   const int G = Hq / Hkv;
   int qt, b, hkv;
   const int qr = sp.rows;
-  if (!prefill_item(blockIdx.x, (Lq * G + qr - 1) / qr, B, Hkv, &qt, &b, &hkv)) return;  // padding
+  if (!prefill_item(blockIdx.x, sp.by_head, (Lq * G + qr - 1) / qr, B, Hkv, &qt, &b, &hkv)) return;  // padding
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, grp = lane >> 4;
   const int pr = qt * qr + 16 * wave + col;  // this lane's packed row
@@ -779,7 +787,7 @@ void attn_prefill_mfma32(
 
   const int G = Hq / Hkv;
   int qt, b, hkv;
-  if (!prefill_item(blockIdx.x, (Lq * G + QR - 1) / QR, B, Hkv, &qt, &b, &hkv))
+  if (!prefill_item(blockIdx.x, false, (Lq * G + QR - 1) / QR, B, Hkv, &qt, &b, &hkv))
     return;  // grid padding
   const int lane = threadIdx.x & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1561,7 +1569,7 @@ int launch_decode(strata_ctx* ctx, const void* q, const void* k, const void* v, 
 // How a prefill launch covers (rows, keys): waves per workgroup, keys per LDS
 // tile and the key split.
 struct PrefillPlan {
-  int nw, ks, kt, nsplit, chunk, qr;
+  int nw, ks, kt, nsplit, chunk, qr, by_head;
 };
 constexpr int kMaxPrefillSplits = 64;
 constexpr size_t kMaxPrefillWs = (size_t)512 << 20;  // longer splits where more would be needed
@@ -1586,11 +1594,19 @@ PrefillPlan prefill_plan(int num_cus, bool f32, int B, int Hq, int Hkv, int Lq, 
   const int64_t least = f32 ? 1 : p.nw == 1 ? 4 : 8;
   int64_t chunk = std::max(least, (int64_t)std::ceil(tiles * mean / (per_cu * (double)num_cus)));
   chunk = std::max(chunk, (longest + kMaxPrefillSplits - 1) / kMaxPrefillSplits);
+  // Whether the tiles are of about one length (no mask, or a history of at least
+  // half the keys) or a causal triangle, whose long tiles go first and whose
+  // short ones fill the CUs that they leave.
+  const bool even = !causal || 2 * (int64_t)(Lk - Lq) >= Lk;
+  p.by_head = f32 && even && (int64_t)B * Hkv % kXcds == 0;
   // Without a split, two wave groups of a workgroup share each tile's keys
-  // where that leaves CUs unused (1500 tokens, 24 heads: 51 -> 38 us; 2048
-  // tokens, 32 heads: 57 -> 51; 4 x 500 tokens stay: 24 against 26).
+  // where every tile has a place at once: one such workgroup fits per CU, two at
+  // D = 64, and in a triangle the second tile of a CU is a short one (us with one
+  // group | with two: 700 tokens, 24 heads 30 | 22; 1500 tokens, causal 57 | 39,
+  // no mask 55 | 65, D = 64 44 | 36; 2048 tokens, 32 heads, causal 58 | 53, no
+  // mask 75 | 86).
   if (!f32 && p.nw == 4 && longest >= 7 &&
-      (tiles <= num_cus || (tiles <= 2 * (int64_t)num_cus && longest >= 32)))
+      (tiles <= num_cus || (!(even && D == 128) && tiles <= 2 * (int64_t)num_cus && longest >= 32)))
     p.ks = 2;
   // Of that chunk and longer ones, the one whose cut of the longest tile's
   // chain (us per step, measured) exceeds the cost of the partials by most:
@@ -1637,17 +1653,32 @@ PrefillPlan prefill_plan(int num_cus, bool f32, int B, int Hq, int Hkv, int Lq, 
     p.ks = longest >= 7 ? 2 : 1;
     return p;
   }
-  // 64-key tiles (two workgroups per CU) halve the steps, 32-key tiles run
-  // three workgroups per CU: the first for launches that leave room (4096
-  // tokens, 32 heads 155 -> 138 us; 4 x 2048 tokens stay, 148 against 154),
-  // and for long chains in a little more, whose third workgroups would only
-  // leave a thin tail (2781 tokens x 2, 24 heads: 122 -> 109; 6000 tokens, 24
-  // heads: 264 -> 234; 7000: 328 -> 311; but 4 x 1150 tokens, 32 heads stay,
-  // 58 against 61, and 5200 tokens, 32 heads, 218 against 231).
-  const double per_cu_tiles = (double)tiles / num_cus;
-  if (p.nsplit == 1 && p.ks == 1 && p.nw == 4 && !f32 &&
-      (per_cu_tiles <= 4 || (per_cu_tiles <= 4.5 && longest >= 40) ||
-       (per_cu_tiles <= 5.5 && longest >= 200)))
+  if (f32 || p.nsplit > 1 || p.ks > 1 || p.nw < 4) return p;
+  // Keys for at most three steps: such a call is one tile's latency, so one wave
+  // per workgroup while two of these fit per CU (33 tokens, 32 heads: 10.1 -> 8.7
+  // us; 64 tokens, 24 heads: 9.9 -> 8.6; 32 x 33 tokens stay: 12.2 | 13.4).
+  if (longest <= 3 && (rows + 31) / 32 * B * Hkv <= 2 * (int64_t)num_cus) {
+    p.nw = 1;
+    p.qr = 32;
+    return p;
+  }
+  // 64-key tiles halve the steps.  At D = 64 as many workgroups of them fit per
+  // CU (us, 32 | 64 keys: 3 tiles per CU of 94 steps 100 | 93, 8 of 16 56 | 52).
+  // At D = 128 two fit and three of 32 keys.  Tiles of one length end together,
+  // so the rounds of the busiest CU decide: its 2 or 4 tiles are whole rounds of
+  // two (no mask: 512 tiles of 16 steps 29.6 | 28.9, 768 40 | 46, 1024 58 | 53,
+  // 1128 of 47 steps 130 | 149, 1536 of 64 211 | 209; 32 x 100 queries after 4000
+  // keys, 24 heads, 768 tiles 225 | 339), chains of 8 steps at 4 excepted (37.9 |
+  // 38.4).  In a triangle they win until a CU's queue is long against its last
+  // tile, later the longer the chain (2 tiles per CU of 8 steps 20.4 | 18.8, 3 23 |
+  // 29; 3 of 32 49 | 44, 4 49 | 51; 4 of 64 84 | 81, 4.5 91 | 97; 4.4 of 188 269 |
+  // 238, 5.9 289 | 302).  Up to 6 steps half a tile of padding, or of keys past
+  // the diagonal, costs as much (150 tokens, 24 heads 12.0 | 12.4; neither: 32 x 64
+  // tokens, 24 heads 13.2 | 12.5).
+  const int64_t rounds = (tiles + num_cus - 1) / num_cus;
+  if (longest < 7 && !(longest % 2 == 0 && (even || longest == 2))) return p;
+  if (D == 64 || (even ? rounds <= 2 || (rounds == 4 && longest >= 16)
+                       : (double)tiles / num_cus <= 2 + 0.8 * std::log2(longest / 8.0)))
     p.kt = 64;
   return p;
 }
@@ -1660,7 +1691,7 @@ void launch_prefill(strata_ctx* ctx, const void* q, const void* k, const void* v
   constexpr bool f32 = sizeof(TQ) == 4;
   const int64_t rows = (int64_t)B * Hq * Lq;
   const PrefillPlan pl = prefill_plan(ctx->num_cus, f32, B, Hq, Hkv, Lq, Lk, D, causal, ex.ws_bytes);
-  PrefillSplit sp{pl.nsplit, pl.chunk, pl.qr, nullptr, nullptr};
+  PrefillSplit sp{pl.nsplit, pl.chunk, pl.qr, pl.by_head, nullptr, nullptr};
   if (pl.nsplit > 1) {
     sp.o = static_cast<float*>(ex.ws);
     sp.ms = reinterpret_cast<float2*>(sp.o + rows * pl.nsplit * D);

@@ -403,21 +403,24 @@ def test_prefill_without_split(dev, Hq, Hkv, D, Lq, Lk):
 
 
 @pytest.mark.parametrize("kernel,D", [("one wave", 128), ("one wave", 64), ("two waves", 64), ("two waves", 128),
-                                      ("plain", 128), ("plain", 64), ("64 keys", 64), ("64 keys", 128)])
+                                      ("short", 64), ("short", 128), ("plain", 128), ("plain", 64),
+                                      ("64 keys", 64), ("64 keys", 128), ("three rounds", 128)])
 @pytest.mark.parametrize("mask", ["causal", "given", "none"])
 def test_prefill_unsplit_kernels_of_a_full_gpu(dev, kernel, D, mask):
     """The unsplit bf16 kernels for more tiles than CUs, the batch sized from the
-    CU count: tiles of one and of two waves (up to 32 and 64 packed rows), the
-    plain four-wave kernel (over 5.5 tiles per CU) and 64-key tiles (between 2
-    and 4), causal, with given positions (rows that see no key, or all) and
-    without a mask.  The first, a middle and the last batch row against float64
+    CU count: tiles of one and of two waves (up to 32 and 64 packed rows), of one
+    wave for three key steps, the plain four-wave kernel (few steps, or tiles of
+    one length in three rounds) and 64-key tiles (in two), causal, with given
+    positions (rows that see no key, or all) and without a mask.  The first, a
+    middle and the last batch row against float64
     (bf16 weights and outputs: 2^-9 each); rows keep their bits whatever the
     other rows of their tile hold."""
     import ctypes as C
     from lokahi_amd import _abi, ops
     cus, Hq, Hkv = torch.cuda.get_device_properties(0).multi_processor_count, 12, 4
     Lq, Lk, tiles, per_cu = {"one wave": (10, 101, 1, 1), "two waves": (21, 201, 1, 1),
-                             "plain": (100, 164, 3, 6), "64 keys": (100, 164, 3, 3)}[kernel]
+                             "short": (30, 70, 3, 1), "plain": (100, 164, 3, 6), "64 keys": (100, 260, 3, 1),
+                             "three rounds": (100, 260, 3, 2)}[kernel]
     B = per_cu * cus // (tiles * Hkv) + 1
     gen = torch.Generator(device=dev).manual_seed(D + Lq)
     q, k, v = (torch.randn((B, h, l, D), generator=gen, device=dev).bfloat16()
@@ -448,6 +451,32 @@ def test_prefill_unsplit_kernels_of_a_full_gpu(dev, kernel, D, mask):
     keep = torch.arange(Lq, device=dev) % 3 != 1
     again = call(torch.where(keep[:, None], q, 3 * torch.randn(q.shape, generator=gen, device=dev).bfloat16()))
     assert torch.equal(again[:, :, keep], got[:, :, keep])
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,Lq,Lk,causal", [(2, 8, 4, 64, 130, 130, False), (1, 16, 8, 128, 37, 200, True),
+                                                     (8, 2, 1, 64, 33, 1000, True), (3, 24, 8, 128, 20, 300, False),
+                                                     (3, 6, 3, 64, 70, 150, False)])
+def test_prefill_f32_tiles_of_one_length(dev, B, Hq, Hkv, D, Lq, Lk, causal):
+    """fp32 prefill without a mask or after a history, whose tiles run head by
+    head where B x KV heads is a multiple of 8 (all shapes but the last), with
+    and without a split of the keys, against float64 (2^-24 per sum term)."""
+    import ctypes as C
+    from lokahi_amd import _abi, ops
+    gen = torch.Generator(device=dev).manual_seed(Lq + Lk)
+    q, k, v = (torch.randn((B, h, l, D), generator=gen, device=dev) for h, l in ((Hq, Lq), (Hkv, Lk), (Hkv, Lk)))
+    sc = torch.matmul(q.double(), k.double().repeat_interleave(Hq // Hkv, 1).transpose(2, 3).contiguous()) / D**0.5
+    if causal:
+        seen = torch.arange(Lk, device=dev) <= torch.arange(Lk - Lq, Lk, device=dev)[:, None]
+        sc = sc.masked_fill(~seen, float("-inf"))
+    ref = torch.matmul(torch.softmax(sc, -1), v.double().repeat_interleave(Hq // Hkv, 1))
+    got = ops.attention(q, k, v, causal=causal)
+    one = torch.empty_like(q)
+    _abi.check(_abi.load().strata_attn_gqa(
+        ops._ctx(0), q.data_ptr(), ops._code(q), k.data_ptr(), ops._code(k), v.data_ptr(), ops._code(v),
+        Hkv * Lk * D, Lk * D, None, B, Hq, Hkv, Lq, Lk, D, int(causal), 32768, 1024, C.c_float(1e-12),
+        one.data_ptr(), ops._stream(0)))
+    for y in (got, one):
+        assert float((y - ref).norm() / ref.norm()) < 1e-5
 
 
 @pytest.mark.parametrize("dtype,B,Hq,Hkv,D,Lq,Lk", [("bf16", 1, 32, 8, 128, 100, 4100), ("bf16", 3, 6, 2, 64, 30, 1500),
