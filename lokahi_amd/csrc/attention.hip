@@ -1609,19 +1609,21 @@ PrefillPlan prefill_plan(int num_cus, bool f32, int B, int Hq, int Hkv, int Lq, 
       (tiles <= num_cus || (!(even && D == 128) && tiles <= 2 * (int64_t)num_cus && longest >= 32)))
     p.ks = 2;
   // Of that chunk and longer ones, the one whose cut of the longest tile's
-  // chain (us per step, measured) exceeds the cost of the partials by most:
-  // the workspace and the second launch (a lone call is as long as its host
-  // side, 5 us more with a split: 2 queries over 227 keys 13.8 us without,
-  // 16.0 with; 4 rows' 5 over 378 19.7, 23.3), and the bytes written and read
-  // at 2.5 TB/s (100 queries after 4000 keys: 127 -> 32 us; 500 after 8000:
-  // 257 -> 94).  Where the grid alone fills the CUs the cut has to be a sixth
-  // of the chain, as less of it shows (5600 tokens, 24 heads: 225 us, 250 with
-  // the split that saves 5 of 157 by this count).
+  // chain (us per step, measured) exceeds the cost of the partials by most: 8 us
+  // for the workspace and the second launch, most of it the host side of a call
+  // from Python (us without | with a split: 2 queries over 227 keys 13.8 | 16; 8
+  // rows' 5 over 600, 24 heads 17.0 | 14.1; fp32, 4 rows' 16 over 150, 8 heads
+  // 18.6 | 13.5; D = 64, 5 over 450 11.3 | 14.2), and the bytes written and read at
+  // 2.5 TB/s (100 queries after 4000 keys: 127 | 32 us; 500 after 8000: 257 | 94;
+  // 8 rows' 200 over 4000, 24 heads 138 | 118).  Where the grid alone fills the CUs
+  // the cut has to be a sixth of the chain, as less of it shows (5600 tokens, 24
+  // heads: 225 us, 250 with the split that saves 5 of 157 by this count).
   const double step = f32 ? 5.5 : p.nw == 4 ? 0.9 : 1.1;
   // (the second group of waves takes 1/7 off: 60 us unsplit for 290 queries
-  // over 2706 keys, 42 split)
-  const double unsplit = longest * (p.nw < 4 ? 0.9 : step) / (p.ks == 2 ? 1.15 : 1.0);
-  const double launch = B > 1 ? 11 : 8;
+  // over 2706 keys, 42 split; D = 64 a tenth)
+  const double unsplit =
+      longest * (p.nw < 4 ? 0.9 : step) * (!f32 && D == 64 ? 0.9 : 1.0) / (p.ks == 2 ? 1.15 : 1.0);
+  const double launch = 8;
   double best = 0;
   p.nsplit = 1;
   p.chunk = (int)(longest * p.kt);
