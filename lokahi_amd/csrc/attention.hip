@@ -480,10 +480,16 @@ __device__ inline bool prefill_item(int wg, bool by_head, int nqt, int B, int Hk
                                     int* hkv) {
   const int per = B * Hkv;
   if (wg >= nqt * per) return false;
-  const int slot = wg / kXcds, head = slot / nqt;
-  const int t = by_head ? slot - head * nqt : wg / per;
+  int t, rest;
+  if (by_head) {
+    const int slot = wg / kXcds, head = slot / nqt;
+    t = slot - head * nqt;
+    rest = head * kXcds + wg % kXcds;
+  } else {
+    t = wg / per;
+    rest = wg - t * per;
+  }
   *qt = nqt - 1 - t;
-  const int rest = by_head ? head * kXcds + wg % kXcds : wg - t * per;
   *b = rest / Hkv;
   *hkv = rest % Hkv;
   return true;
