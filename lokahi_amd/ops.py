@@ -65,11 +65,6 @@ def _lib():
     return _abi._lib or _abi.load()
 
 
-def _int32(n) -> int:
-    """n (any type that converts) as an int, at most 2^31 - 1."""
-    return n if type(n) is int and n < 2**31 else int(min(n, 2**31 - 1))
-
-
 def _rows(x: torch.Tensor, K: int):
     """(contiguous x, rows of K elements)."""
     x = x.contiguous()
@@ -320,10 +315,12 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if out is None:
         out = q.new_empty((B, Hq, Lq, D))
     ws = _attention_workspace(dev, q, k, v, causal) if Lq > 1 else None
+    if not (type(q_block_size) is type(k_block_size) is int and q_block_size < 2**31 > k_block_size):
+        q_block_size, k_block_size = (int(min(n, 2**31 - 1)) for n in (q_block_size, k_block_size))
     rc = _lib().strata_attn_gqa_ws(
         _ctx(dev), q.data_ptr(), _code(q), k.data_ptr(), _code(k), v.data_ptr(), _code(v), bs, hs,
         None if qpos is None else qpos.data_ptr(), B, Hq, Hkv, Lq, Lk, D, 1 if causal else 0,
-        _int32(q_block_size), _int32(k_block_size), float(eps), out.data_ptr(),
+        q_block_size, k_block_size, float(eps), out.data_ptr(),
         None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _raw_stream(dev))
     if rc:
         check(rc)
