@@ -1680,11 +1680,11 @@ PrefillPlan prefill_plan(int num_cus, bool f32, int B, int Hq, int Hkv, int Lq, 
   // 38.4).  In a triangle they win until a CU's queue is long against its last
   // tile, later the longer the chain (2 tiles per CU of 8 steps 20.4 | 18.8, 3 23 |
   // 29; 3 of 32 49 | 44, 4 49 | 51; 4 of 64 84 | 81, 4.5 91 | 97; 4.4 of 188 269 |
-  // 238, 5.9 289 | 302).  Up to 6 steps half a tile of padding, or of keys past
-  // the diagonal, costs as much (150 tokens, 24 heads 12.0 | 12.4; neither: 32 x 64
-  // tokens, 24 heads 13.2 | 12.5).
+  // 238, 5.9 289 | 302).  Up to 6 steps an odd one, half a tile of padding, costs as
+  // much (24 heads, K and V from HBM: 150 tokens 10.8 | 11.1, but 120 10.3 | 9.9,
+  // 165 12.5 | 11.9, 190 12.2 | 10.9).
   const int64_t rounds = (tiles + num_cus - 1) / num_cus;
-  if (longest < 7 && !(longest % 2 == 0 && (even || longest == 2))) return p;
+  if (longest < 7 && longest % 2 == 1) return p;
   if (D == 64 || (even ? rounds <= 2 || (rounds == 4 && longest >= 16)
                        : (double)tiles / num_cus <= 2 + 0.8 * std::log2(longest / 8.0)))
     p.kt = 64;
